@@ -163,16 +163,15 @@ static void carve(lvbgs_ctx* c, Arena& ar) {
     v.rec = ar.take<uint32_t>(npx);
     v.mres = ar.take<uint32_t>(npx);
     v.wl0 = ar.take<uint32_t>(npx);
-    v.wl1 = ar.take<uint32_t>(npx);
     // continuation stripes sized so no stripe can overflow; cached contexts for up to an eighth
     // of the pixels, spread over the stripes; entries beyond rebuild theirs
     const size_t ctx_cap = std::min(npx, std::max(npx / 8, (size_t)1024));
     v.cont_region = cont_stripe_slots(c->W, c->H);
     v.cont_ctx_region = (uint32_t)((ctx_cap + kContStripes - 1) / kContStripes);
     v.cont = ar.take<uint32_t>((size_t)kContStripes * v.cont_region);
+    v.wl1 = ar.take<uint32_t>((size_t)kContStripes * v.cont_region);  // at least npx
     v.cont_ctx = ar.take<uint32_t>((size_t)kContStripes * v.cont_ctx_region * kCtxWords);
     v.cont2 = ar.take<uint32_t>(npx);
-    v.stamp = ar.take<unsigned long long>(npx);
     v.dsLT = ar.take<float>(nds);
     v.dsST = ar.take<float>(nds);
     v.sc = ar.take<Scalars>(1);

@@ -175,7 +175,7 @@ struct alignas(128) Scalars {
     uint32_t nz_count_unused;
     uint32_t err_flags;          // sticky error bits (see kErr*)
     unsigned long long cd_sum_unused;
-    uint32_t wl_count[kWlRing];  // fix-point worklist counts (ring)
+    uint32_t wl_count[kWlRing];  // worklist counts of fix-point iterations >= 2 (ring)
     int32_t refresh_pending;     // refresh request consumed by the refresh kernel
     float refresh_frac;
     int32_t refresh_force_fg;
@@ -192,12 +192,14 @@ struct alignas(128) Scalars {
     unsigned long long coop_part[64]; // samples examined by the cooperative match phase
     uint32_t iters;              // per-frame: fix-point iterations that had work
     uint32_t max_iter_seen;      // largest fix-point iteration index that had work (sticky)
-    uint32_t epoch;              // steps since allocation (worklist de-duplication tags)
+    uint32_t epoch;              // steps since allocation (kept in checkpoints)
     uint32_t wl_work[8];         // per-frame: worklist size of fix-point iterations 1..7
     uint32_t cont2_count;        // per-frame: pixels handed to the cooperative match phase
     uint8_t lut[256];            // LBSP threshold LUT (m_anLBSPThreshold_8bitLUT)
     // per-frame: pixels handed to the match continuation, stripe k at cont_cnt[k * kContStride]
     alignas(128) uint32_t cont_cnt[kContStripes * kContStride];
+    // per-frame: entries of the first fix-point worklist, striped the same way
+    alignas(128) uint32_t wl_first[kContStripes * kContStride];
 };
 constexpr uint32_t kErrFixpointCap = 1u;
 

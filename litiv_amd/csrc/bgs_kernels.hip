@@ -630,13 +630,54 @@ LV_D ScanState unpack_state(uint32_t mr) {
     return ScanState{mr & 255u, mr >> 24, (mr >> 8) & 63u, (mr >> 14) & 1023u};
 }
 
-// worklist push with de-duplication; stamp = (epoch, iteration)
-LV_D void wl_push(const View& v, uint32_t t, uint32_t k, uint64_t epoch, uint32_t* wl_dst) {
-    const unsigned long long tag = (unsigned long long)((epoch << 20) | (uint64_t)(k & 0xFFFFFu));
-    if (atomicExch(&v.stamp[t], tag) != tag) {
-        const uint32_t slot = atomicAdd(&v.sc->wl_count[k % kWlRing], 1u);
-        wl_dst[slot] = t;
+// Appends one value per calling lane that wants to (push) to a list: one atomic per wavefront on the
+// list's counter. Must be called by the lanes of a wavefront together.
+LV_D void wave_append(bool push, uint32_t value, uint32_t* counter, uint32_t* list) {
+    const unsigned long long bal = __ballot(push);
+    if (!bal) return;
+    const int lane = (int)(threadIdx.x & 63u), leader = __ffsll((long long)bal) - 1;
+    uint32_t base = 0;
+    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(bal));
+    base = (uint32_t)__shfl((int)base, leader, 64);
+    if (push) G(list)[base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = value;
+}
+
+// Worklist of fix-point iteration 1, filled by the match phases: split into kContStripes stripes like
+// the continuation list (the pixels of tile b push to stripe b % kContStripes, at most one entry
+// each, so a stripe holds at most cont_region entries). With one counter for all pushes its atomics
+// were what the continuation spent its time on, 12 to 16 ns each: match_seq 575 -> 154 us on a 3840x2160
+// frame with 36 K pushes, 211 -> 81 us at 1920x1080. A target may be listed twice (two changed writers):
+// both items match it against the same decisions, or the one that saw the older ones is followed by
+// another in the next iteration, which its changed writer pushes.
+LV_D void push_first(const View& v, bool push, uint32_t t, uint32_t stripe) {
+    wave_append(push, t, &v.sc->wl_first[stripe * kContStride], v.wl1 + (size_t)stripe * v.cont_region);
+}
+
+// worklist of iteration k >= 2: one counter (few entries)
+LV_D void push_next(const View& v, bool push, uint32_t t, uint32_t k, uint32_t* wl_dst) {
+    wave_append(push, t, &v.sc->wl_count[k % kWlRing], wl_dst);
+}
+
+// exclusive prefix of the kContStripes counters at cnt (kContStride words apart) into pre, by the
+// first wavefront of the block; the caller synchronizes before reading pre
+LV_D void stripe_prefix(const uint32_t* cnt, uint32_t* pre) {
+    static_assert(kContStripes <= 64 && (kContStripes & (kContStripes - 1)) == 0, "one wavefront scans the stripe counts");
+    if (threadIdx.x >= 64u) return;
+    const int lane = (int)threadIdx.x;
+    uint32_t c = lane < kContStripes ? G(cnt)[lane * kContStride] : 0u;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_up((int)c, (unsigned)o, 64);
+        if (lane >= o) c += t;
     }
+    if (lane < kContStripes) pre[lane + 1] = c;
+    if (lane == 0) pre[0] = 0u;
+}
+// item i of a striped list: the last stripe whose prefix is at most i
+LV_D uint32_t stripe_of(const uint32_t* pre, uint32_t i) {
+    uint32_t k = 0;
+    for (uint32_t half = kContStripes / 2; half > 0; half >>= 1)
+        if (pre[k + half] <= i) k += half;
+    return k;
 }
 
 // forward target of p's own diffusion (if any): target after p in raster order with open gate
@@ -669,7 +710,10 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
         for (int i = 0; i < 8; ++i) v.sc->wl_work[i] = 0;
         v.sc->iters = 0;
     }
-    if (bid == 0 && threadIdx.x < kContStripes) v.sc->cont_cnt[threadIdx.x * kContStride] = 0;
+    if (bid == 0 && threadIdx.x < kContStripes) {
+        v.sc->cont_cnt[threadIdx.x * kContStride] = 0;
+        v.sc->wl_first[threadIdx.x * kContStride] = 0;
+    }
     if (bid == 0 && threadIdx.x < kStripes) {
         v.sc->ex_part[threadIdx.x] = 0;
         v.sc->wr_part[threadIdx.x] = 0;
@@ -932,7 +976,7 @@ struct PredTile;
 template <int C, int ALGO, int KF>
 LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, const FrameTile<C>& tile,
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,
-                      uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px);
+                      uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px, bool& push, uint32_t& target);
 
 // records and previous raw decisions of the raster-earlier part of a tile's 5x5 neighbourhood:
 // rows y0-2 .. y0+TH-1, columns x0-2 .. x0+TW+1
@@ -1049,17 +1093,20 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
     const int lx = src % TW, ly = src / TW, x = x0 + lx, y = y0 + ly;
     const uint32_t p = (uint32_t)(y * v.W + x);
     uint32_t examined = 0;
-    bool cont = false;
+    bool cont = false, push = false;
+    uint32_t target = 0;
     const PxIn<C> in = s_in[src];
     PxCtx<C> px;
     if (x < v.W && y < v.H && in.roi)
-        cont = !match_pixel<C, ALGO, KF>(v, frame, lut, tile, pred, in, lx, ly, x, y, p, seq_limit, examined, px);
+        cont = !match_pixel<C, ALGO, KF>(v, frame, lut, tile, pred, in, lx, ly, x, y, p, seq_limit, examined, px, push,
+                                         target);
     // unfinished pixels go to the continuation with their context: one atomic per wavefront, on
     // this tile's stripe of the list (at most cont_region entries reach one stripe)
+    const uint32_t k = bid % (uint32_t)kContStripes;
+    push_first(v, push, target, k);
     const unsigned long long bal = __ballot(cont);
     if (bal) {
         const int lane = (int)(threadIdx.x & 63u), leader = __ffsll((long long)bal) - 1;
-        const uint32_t k = bid % (uint32_t)kContStripes;
         uint32_t base = 0;
         if (lane == leader) base = atomicAdd(&v.sc->cont_cnt[k * kContStride], (uint32_t)__popcll(bal));
         base = (uint32_t)__shfl((int)base, leader, 64);
@@ -1078,7 +1125,7 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
 template <int C, int ALGO, int KF>
 LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, const FrameTile<C>& tile,
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,
-                      uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px) {
+                      uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px, bool& push, uint32_t& target) {
     // guess: raster-earlier writers decide as in the previous frame
     const uint32_t applied = applied_writers_tile(pred, lx, ly);
     uint64_t sbm;
@@ -1097,9 +1144,7 @@ LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, c
     if (st.good < (uint32_t)v.REQ && st.s < N) return false;
     const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
     G(v.dec)[p] = fg;
-    const uint8_t guess = G(v.last_raw)[p] ? 1 : 0;
-    uint32_t t;
-    if (fg != guess && forward_target(v, G(v.rec)[p], x, y, t)) wl_push(v, t, 1u, v.sc->epoch, v.wl1);
+    push = fg != pred.guess[ly + 2][lx + 2] && forward_target(v, pred.rec[ly + 2][lx + 2], x, y, target);
     return true;
 }
 
@@ -1119,16 +1164,30 @@ LV_D uint32_t applied_writers_global(const View& v, int x, int y) {
     return applied;
 }
 
-// decision of a finished scan: match result, raw decision, and the forward target of a pixel whose
-// decision differs from the speculative guess goes to the first fix-point worklist
+// decision of a finished scan: match result, raw decision; true when the decision differs from the
+// speculative guess and the pixel has a forward target (for the first fix-point worklist)
 template <int C>
-LV_D void finish_pixel(const View& v, uint32_t p, int x, int y, const ScanState& st, uint64_t epoch) {
+LV_D bool finish_pixel(const View& v, uint32_t p, int x, int y, const ScanState& st, uint32_t& t) {
     G(v.mres)[p] = pack_state(st);
     const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
     G(v.dec)[p] = fg;
     const uint8_t guess = G(v.last_raw)[p] ? 1 : 0;
-    uint32_t t;
-    if (fg != guess && forward_target(v, G(v.rec)[p], x, y, t)) wl_push(v, t, 1u, epoch, v.wl1);
+    return fg != guess && forward_target(v, G(v.rec)[p], x, y, t);
+}
+
+// the stripe of the pixel's tile
+LV_D uint32_t tile_stripe(const View& v, int x, int y) {
+    return (uint32_t)((y / TH) * ((v.W + TW - 1) / TW) + x / TW) % (uint32_t)kContStripes;
+}
+// push_first for lanes of different stripes: one append per stripe present in the wavefront
+LV_D void push_first_mixed(const View& v, bool push, uint32_t t, uint32_t stripe) {
+    unsigned long long bal = __ballot(push);
+    while (bal) {
+        const uint32_t s0 = (uint32_t)__shfl((int)stripe, __ffsll((long long)bal) - 1, 64);
+        const bool mine = push && stripe == s0;
+        push_first(v, mine, t, s0);
+        bal &= ~__ballot(mine);
+    }
 }
 
 // Phase B: the scans phase A cut at its sample limit, continued with one lane per pixel over the
@@ -1138,31 +1197,17 @@ LV_D void finish_pixel(const View& v, uint32_t p, int x, int y, const ScanState&
 // slots goes on to phase C.
 template <int C, int ALGO, int KF>
 LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
-    static_assert(kContStripes <= 64 && (kContStripes & (kContStripes - 1)) == 0, "one wavefront scans the stripe counts");
     const uint8_t* frame = v.frame;
     __shared__ uint8_t lut[256];
     __shared__ uint32_t s_pre[kContStripes + 1];  // exclusive prefix of the stripe counts
-    if (threadIdx.x < 64u) {
-        const int lane = (int)threadIdx.x;
-        uint32_t c = lane < kContStripes ? v.sc->cont_cnt[lane * kContStride] : 0u;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = (uint32_t)__shfl_up((int)c, (unsigned)o, 64);
-            if (lane >= o) c += t;
-        }
-        if (lane < kContStripes) s_pre[lane + 1] = c;
-        if (lane == 0) s_pre[0] = 0u;
-    }
+    stripe_prefix(v.sc->cont_cnt, s_pre);
     load_lut(lut, v.sc);
     __syncthreads();
     const uint32_t n = s_pre[kContStripes];
     if (bid * TPB >= n) return;  // uniform: no item reaches this block
-    const uint64_t epoch = v.sc->epoch;
     uint32_t examined = 0;
     for (uint32_t i = bid * TPB + threadIdx.x; i < n; i += nblk * TPB) {
-        // item i = entry j of stripe k: the last stripe whose prefix is at most i
-        uint32_t k = 0;
-        for (uint32_t half = kContStripes / 2; half > 0; half >>= 1)
-            if (s_pre[k + half] <= i) k += half;
+        const uint32_t k = stripe_of(s_pre, i);  // item i = entry j of stripe k
         const uint32_t j = i - s_pre[k];
         const uint32_t p = G(v.cont)[(size_t)k * v.cont_region + j];
         const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
@@ -1173,15 +1218,18 @@ LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
         uint64_t sbm;
         int nrep;
         auto rec_of = [&](int i) { return G(v.rec)[(size_t)(y + kPredDY[i]) * v.W + (x + kPredDX[i])]; };
+        bool push = false;
+        uint32_t t = 0;
         if (!build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of)) {
             v.cont2[atomicAdd(&v.sc->cont2_count, 1u)] = p;
-            continue;
+        } else {
+            ScanState st = unpack_state(G(v.mres)[p]);
+            const uint32_t s0 = st.s;
+            scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
+            examined += st.s - s0;
+            push = finish_pixel<C>(v, p, x, y, st, t);
         }
-        ScanState st = unpack_state(G(v.mres)[p]);
-        const uint32_t s0 = st.s;
-        scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
-        examined += st.s - s0;
-        finish_pixel<C>(v, p, x, y, st, epoch);
+        push_first_mixed(v, push, t, k);
     }
     block_add<TPB>(examined, v.sc->coop_part);
 }
@@ -1201,7 +1249,6 @@ LV_D void match_cont_body(const View& v, uint32_t bid, uint32_t nblk) {
     const uint32_t sub = threadIdx.x & (kGroup - 1);
     const uint32_t g0 = (bid * TPB + threadIdx.x) / kGroup;
     const uint32_t rounds = (n + ngroups - 1) / ngroups;  // uniform trip count: every lane takes part
-    const uint64_t epoch = v.sc->epoch;
     uint64_t examined = 0;
     for (uint32_t r = 0; r < rounds; ++r) {
         const uint32_t i = g0 + r * ngroups;
@@ -1224,20 +1271,39 @@ LV_D void match_cont_body(const View& v, uint32_t bid, uint32_t nblk) {
         __syncthreads();
         const uint32_t s_before = st.s;
         scan_coop<C, ALGO, 5 * C>(v, frame, lut, px, x, y, applied, sbm, st, active);
+        bool push = false;
+        uint32_t t = 0;
         if (active && sub == 0) {
             examined += st.s - s_before;
-            finish_pixel<C>(v, p, x, y, st, epoch);
+            push = finish_pixel<C>(v, p, x, y, st, t);
         }
+        push_first_mixed(v, push, t, tile_stripe(v, x, y));
     }
     block_add<TPB>(examined, v.sc->coop_part);
 }
 
+// worklist of fix-point iteration k: entry i, and its entry count for every thread of the block (pre:
+// the block's LDS, kContStripes + 1 words, holding the stripes' prefix of iteration 1; the block
+// synchronizes in here)
+LV_D uint32_t wl_item(const View& v, uint32_t k, const uint32_t* pre, uint32_t i) {
+    if (k != 1u) return ((k & 1u) ? v.wl1 : v.wl0)[i];
+    const uint32_t s = stripe_of(pre, i);
+    return v.wl1[(size_t)s * v.cont_region + (i - pre[s])];
+}
+LV_D uint32_t wl_total(const View& v, uint32_t k, uint32_t* pre) {
+    if (k != 1u)
+        return __hip_atomic_load(&v.sc->wl_count[k % kWlRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    stripe_prefix(v.sc->wl_first, pre);
+    __syncthreads();
+    return pre[kContStripes];
+}
+
 // fix-point re-match of worklisted pixels (all lanes call; kGroup lanes per item)
 template <int C, int ALGO>
-LV_D void rematch_round(const View& v, const uint8_t* frame, const uint8_t* lut, uint8_t* patch, const uint32_t* wl,
-                        uint32_t n, uint32_t i, uint32_t k, uint64_t epoch, uint32_t* wl_next) {
+LV_D void rematch_round(const View& v, const uint8_t* frame, const uint8_t* lut, uint8_t* patch, const uint32_t* pre,
+                        uint32_t n, uint32_t i, uint32_t k, uint32_t* wl_next) {
     const bool active = i < n;
-    const uint32_t p = active ? wl[i] : 0u;
+    const uint32_t p = active ? wl_item(v, k, pre, i) : 0u;
     const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
     PxCtx<C> px;
     uint32_t applied = 0;
@@ -1253,16 +1319,18 @@ LV_D void rematch_round(const View& v, const uint8_t* frame, const uint8_t* lut,
     __syncthreads();
     ScanState st = scan_init<C>();
     scan_coop<C, ALGO, 5 * C>(v, frame, lut, px, x, y, applied, sbm, st, active);
+    bool push = false;
+    uint32_t t = 0;
     if (active && (threadIdx.x & (kGroup - 1)) == 0) {
         G(v.mres)[p] = pack_state(st);
         const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
         const uint8_t old = G(v.dec)[p];
         if (fg != old) {
             __hip_atomic_store(&v.dec[p], fg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t t;
-            if (forward_target(v, G(v.rec)[p], x, y, t)) wl_push(v, t, k + 1u, epoch, wl_next);
+            push = forward_target(v, G(v.rec)[p], x, y, t);
         }
     }
+    push_next(v, push, t, k + 1u, wl_next);
 }
 
 // fix-point iteration k (k >= 1): worklist k -> worklist k+1
@@ -1271,11 +1339,12 @@ LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k) 
     const uint8_t* frame = v.frame;
     __shared__ uint8_t lut[256];
     __shared__ uint8_t patches[TPB / kGroup][25 * C];
+    __shared__ uint32_t s_pre[kContStripes + 1];
     // slot k+2 was last read by iteration k-2 (finished); it must be empty before iteration k+1
     // pushes into it, whether or not this iteration has work.
     if (bid == 0 && threadIdx.x == 0)
         __hip_atomic_store(&v.sc->wl_count[(k + 2) % kWlRing], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t n = __hip_atomic_load(&v.sc->wl_count[k % kWlRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t n = wl_total(v, k, s_pre);
     if (n == 0) return;
     if (bid == 0 && threadIdx.x == 0) {
         atomicAdd(&v.sc->iters, 1u);
@@ -1285,14 +1354,12 @@ LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k) 
     if (bid * (TPB / kGroup) >= n) return;  // uniform: no item reaches this block
     load_lut(lut, v.sc);
     __syncthreads();
-    const uint32_t* wl = (k & 1u) ? v.wl1 : v.wl0;
     uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
-    const uint64_t epoch = v.sc->epoch;
     const uint32_t ngroups = nblk * (TPB / kGroup);
     const uint32_t g0 = (bid * TPB + threadIdx.x) / kGroup;
     const uint32_t rounds = (n + ngroups - 1) / ngroups;
     for (uint32_t r = 0; r < rounds; ++r)
-        rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], wl, n, g0 + r * ngroups, k, epoch, wl_next);
+        rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], s_pre, n, g0 + r * ngroups, k, wl_next);
 }
 
 // remaining fix-point iterations in one workgroup (normally no work is left)
@@ -1301,13 +1368,14 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
     const uint8_t* frame = v.frame;
     __shared__ uint8_t lut[256];
     __shared__ uint8_t patches[256 / kGroup][25 * C];
+    __shared__ uint32_t s_pre[kContStripes + 1];
     __shared__ uint32_t s_n;
     load_lut(lut, v.sc);
-    const uint64_t epoch = v.sc->epoch;
     for (uint32_t k = k0;; ++k) {
         __syncthreads();
+        const uint32_t total = wl_total(v, k, s_pre);
         if (threadIdx.x == 0) {
-            s_n = __hip_atomic_load(&v.sc->wl_count[k % kWlRing], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_n = total;
             if (s_n != 0) {
                 if (k - k0 >= cap) {
                     atomicOr(&v.sc->err_flags, kErrFixpointCap);
@@ -1324,12 +1392,11 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
         __syncthreads();
         const uint32_t n = s_n;
         if (n == 0) break;
-        const uint32_t* wl = (k & 1u) ? v.wl1 : v.wl0;
         uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
         const uint32_t ngroups = blockDim.x / kGroup, g0 = threadIdx.x / kGroup;
         const uint32_t rounds = (n + ngroups - 1) / ngroups;
         for (uint32_t r = 0; r < rounds; ++r)
-            rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], wl, n, g0 + r * ngroups, k, epoch, wl_next);
+            rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], s_pre, n, g0 + r * ngroups, k, wl_next);
         __threadfence();
     }
 }
