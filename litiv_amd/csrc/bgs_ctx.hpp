@@ -34,6 +34,7 @@ struct lvbgs_ctx {
     // checkpoint load: the sample planes repacked into the device record layout on the host, held
     // between the geometry set-up and the upload of the scalars
     std::vector<uint32_t> restore_stage;
+    uint32_t* h_err = nullptr;   // pinned: the steps' error bits, written by the device when one is set
     // timing
     int timed_stage = 0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pairs;

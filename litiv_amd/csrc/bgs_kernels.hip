@@ -1379,6 +1379,7 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
             if (s_n != 0) {
                 if (k - k0 >= cap) {
                     atomicOr(&v.sc->err_flags, kErrFixpointCap);
+                    __hip_atomic_store(v.h_err, kErrFixpointCap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     s_n = 0;
                 } else {
                     __hip_atomic_store(&v.sc->wl_count[(k + 2) % kWlRing], 0u, __ATOMIC_RELAXED,

@@ -57,6 +57,8 @@ struct View {
     uint32_t* cont2;         // pixels left by the continuation to the cooperative phase
     float *dsLT, *dsST;      // (W/8)*(H/8)*C
     Scalars* sc;
+    uint32_t* h_err;         // host-visible copy of Scalars::err_flags (pinned), so a synchronizing
+                             // host reads it without a copy (25 us each, 2 ms for a batch of 64)
 };
 
 }  // namespace lvbgs

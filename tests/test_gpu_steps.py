@@ -30,3 +30,35 @@ def flashing(w, h, c, n, seed=0):
 def test_first_worklist_stripes(algo, c, w, h, schedule):
     # more tiles than stripes and fewer; read by a full-grid iteration, by few blocks, by the tail alone
     run_sequence(algo, flashing(w, h, c, 10), schedule=schedule, lr=None if algo == SUBSENSE else 2.0)
+
+
+@pytest.mark.parametrize("pad_in,pad_out", [(0, 0), (7, 0), (0, 5), (3, 9)])
+def test_host_rows_packed_and_padded(pad_in, pad_out):
+    # packed rows take one linear copy, padded rows the 2-D copy, in and out independently
+    import ctypes as C
+
+    from litiv_amd import BackgroundSubtractorSuBSENSE
+    from litiv_amd.bgs import lib
+    w, h = 83, 45
+    frames = flashing(w, h, 3, 4)
+    a, b = BackgroundSubtractorSuBSENSE(), BackgroundSubtractorSuBSENSE()
+    a.initialize(frames[0])
+    b.initialize(frames[0])
+    for f in frames:
+        src = np.zeros((h, 3 * w + pad_in), np.uint8)
+        src[:, :3 * w] = f.reshape(h, 3 * w)
+        out = np.full((h, w + pad_out), 7, np.uint8)
+        assert lib().lvbgs_apply(b._h, src.ctypes.data, src.strides[0], out.ctypes.data, out.strides[0], C.c_double(0.0)) == 0
+        assert np.array_equal(out[:, :w], a.apply(f)) and (out[:, w:] == 7).all()
+    bg = np.full((h, 3 * w + pad_out), 7, np.uint8)
+    assert lib().lvbgs_get_background_image(b._h, bg.ctypes.data, bg.strides[0]) == 0
+    assert np.array_equal(bg[:, :3 * w].reshape(h, w, 3), a.getBackgroundImage()) and (bg[:, 3 * w:] == 7).all()
+
+
+@pytest.mark.parametrize("w,h", [(4, 9), (5, 5), (9, 4), (8, 6)])
+def test_validate_roi_border(w, h):
+    from litiv_amd import BackgroundSubtractorSuBSENSE
+    roi = BackgroundSubtractorSuBSENSE.validateROI(np.full((h, w), 255, np.uint8))
+    want = np.zeros((h, w), np.uint8)
+    want[2:max(2, h - 2), 2:max(2, w - 2)] = 255
+    assert np.array_equal(roi, want)
