@@ -189,7 +189,6 @@ static void carve(lvbgs_ctx* c, Arena& ar) {
     v.cont = ar.take<uint32_t>((size_t)kContStripes * v.cont_region);
     v.wl1 = ar.take<uint32_t>((size_t)kContStripes * v.cont_region);  // at least npx
     v.cont_ctx = ar.take<uint32_t>((size_t)kContStripes * v.cont_ctx_region * kCtxWords);
-    v.cont2 = ar.take<uint32_t>(npx);
     v.dsLT = ar.take<float>(nds);
     v.dsST = ar.take<float>(nds);
     v.sc = ar.take<Scalars>(1);
@@ -454,13 +453,11 @@ static int check_lr(lvbgs_ctx* c, double lr) {
     return LVBGS_OK;
 }
 
-// Automatic sequential-phase limit of the single-stream path, from measurements on MI355X:
-// SuBSENSE RGB frames of 1280x720 and larger cut their scans at 8 samples and continue the cut
-// pixels densely (1080p 11% and 4K 16% faster per frame than one full pass); smaller frames,
-// one-channel SuBSENSE and LOBSTER scan every sample in one pass.
-static uint32_t auto_seq_limit(const lvbgs_ctx* c) {
-    return (c->algo == LVBGS_SUBSENSE && c->C == 3 && c->npx >= 900000u) ? 8u : 255u;
-}
+// Samples scanned per pixel before phase B takes over in the single-stream path: one batch of four
+// loads. Measured per frame on MI355X at 4 / 8 / 12 / 255 samples: 320x240 RGB 127 / 129 / 131 / 157 us,
+// 1280x720 286 / 288 / 291 / 357, 3840x2160 grey 998 / 1002 / 1006 / 1025, LOBSTER 640x512 grey 79 / 80 /
+// 82 / 88, 3840x2160 RGB 779 / 780 / 787 / 817.
+constexpr uint32_t kSeqLimit = 4;
 
 static int step(lvbgs_ctx* c, const uint8_t* d_img, uint8_t* d_mask, double lr) {
     StepOptions o = c->opt;
@@ -483,7 +480,8 @@ static int step(lvbgs_ctx* c, const uint8_t* d_img, uint8_t* d_mask, double lr) 
     v.frame = d_img;
     v.out_mask = d_mask;
     v.lr = lr;
-    v.seq_limit = o.seq_limit > 0 ? (uint32_t)o.seq_limit : auto_seq_limit(c);
+    v.seq_limit = o.seq_limit > 0 ? (uint32_t)o.seq_limit : kSeqLimit;
+    v.group_limit = kGroupLimit;
     frame_step(v, o, c->stream);
     ++c->apply_count;
     return LVBGS_OK;
@@ -1206,6 +1204,7 @@ extern "C" int lvbgs_batch_apply_device(lvbgs_batch* b, const void* const* d_img
         v.out_mask = d_masks ? (uint8_t*)d_masks[s] : nullptr;
         v.lr = lrs ? lrs[s] : 0.0;
         v.seq_limit = (uint32_t)stream_options(b, s).seq_limit;
+        v.group_limit = kGroupLimit / (uint32_t)ns;
         b->h_views[i][k] = v;
         ++b->ctx[s]->apply_count;
     }

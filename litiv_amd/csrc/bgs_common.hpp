@@ -194,7 +194,6 @@ struct alignas(128) Scalars {
     uint32_t max_iter_seen;      // largest fix-point iteration index that had work (sticky)
     uint32_t epoch;              // steps since allocation (kept in checkpoints)
     uint32_t wl_work[8];         // per-frame: worklist size of fix-point iterations 1..7
-    uint32_t cont2_count;        // per-frame: pixels handed to the cooperative match phase
     uint8_t lut[256];            // LBSP threshold LUT (m_anLBSPThreshold_8bitLUT)
     // per-frame: pixels handed to the match continuation, stripe k at cont_cnt[k * kContStride]
     alignas(128) uint32_t cont_cnt[kContStripes * kContStride];

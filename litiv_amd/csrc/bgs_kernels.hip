@@ -382,28 +382,14 @@ constexpr int kPredDY[12] = {-2, -2, -2, -2, -2, -1, -1, -1, -1, -1, 0, 0};
 // static forward gate of a record whose target lies after the writer in raster order
 LV_D bool fwd_gate(uint32_t r) { return rec_gate_a(r) || (rec_gate_b(r) && rec_ghost_fwd(r)); }
 
-// Candidate writers of p: bit i set when predecessor i targets p with an open forward gate.
-LV_D uint32_t candidate_writers(const View& v, int x, int y) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
-        const uint32_t r = G(v.rec)[q];
-        const uint32_t code = (uint32_t)((2 - kPredDY[i]) * 5 + (2 - kPredDX[i]));
-        if (rec_tgt(r) == code && fwd_gate(r)) m |= 1u << i;
-    }
-    return m;
-}
-
 // Ordered scan s = 0..N-1 until REQ matches (SUB:366-395, LOB:480-495). Samples overwritten by
-// applied writers (mask `applied`, slot bitmap `sbm`) are taken from the writer; the last writer
-// in raster order wins. Two evaluation orders give the same result as the sequential loop:
+// applied writers are taken from the writer; the last writer in raster order wins. Two evaluation orders
+// give the same result as the sequential loop:
 //   scan_seq  : one lane per pixel, samples in order, KF loads in flight, up to `limit`, with
 //               at most kRepl overwritten slots substituted from the thread's LDS entries;
-//   scan_coop : kGroup lanes per pixel evaluate kGroup consecutive samples at once; a ballot finds
-//               the REQ-th match in sample order, distances are reduced only up to it.
-constexpr int kGroup = 8;
-constexpr uint32_t kBig = 0xFFFFu;
+//   scan_group: the kGroup lanes of a group evaluate kGroup consecutive samples of one pixel at once; the
+//               matches are then taken in sample order up to the REQ-th.
+constexpr int kGroup = 16;
 
 struct ScanState {
     uint32_t good, s, md, ms;
@@ -412,33 +398,6 @@ struct ScanState {
 template <int C>
 LV_D ScanState scan_init() {
     return ScanState{0u, 0u, C * 16u, C * 255u};
-}
-
-LV_D uint64_t applied_slots(const View& v, int x, int y, uint32_t applied) {
-    uint64_t sbm = 0;  // slots (mod 64) touched by applied writers
-    for (uint32_t m = applied; m; m &= m - 1) {
-        const int i = __builtin_ctz(m);
-        const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
-        sbm |= 1ull << (rec_slot_diff(G(v.rec)[q]) & 63u);
-    }
-    return sbm;
-}
-
-// decodes a fetched sample, replacing it by the last applied writer's value when one wrote slot s
-template <int C>
-LV_D void sample_value(const View& v, const uint8_t* frame, int x, int y, uint32_t s, uint32_t applied, uint64_t sbm,
-                       uint64_t ra, uint32_t rb, uint32_t col[C], uint32_t desc[C]) {
-    decode_raw<C>(ra, rb, col, desc);
-    if ((sbm >> (s & 63u)) & 1u) {
-        for (int i = 11; i >= 0; --i) {
-            if (!((applied >> i) & 1u)) continue;
-            const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
-            if (rec_slot_diff(G(v.rec)[q]) == s) {
-                current_value<C>(v, frame, q, col, desc);
-                break;
-            }
-        }
-    }
 }
 
 // Overwritten slots of a pixel with their replacement values (the last applied writer's current
@@ -562,68 +521,6 @@ LV_D void scan_seq(const View& v, const uint8_t* lut, const PxCtx<C>& px, int x,
     }
 }
 
-// Called by every lane of the wavefront; lanes 8g..8g+7 share one pixel and one state (active and
-// px/x/y/applied/sbm/st identical within the group). Returns with st final.
-template <int C, int ALGO, int RS>
-LV_D void scan_coop(const View& v, const uint8_t* frame, const uint8_t* lut, const PxCtx<C>& px, int x, int y,
-                    uint32_t applied, uint64_t sbm, ScanState& st, bool active) {
-    const uint32_t N = (uint32_t)v.N, REQ = (uint32_t)v.REQ;
-    const int lane = (int)(threadIdx.x & 63u), sub = lane & (kGroup - 1), gbase = lane & ~(kGroup - 1);
-    const uint32_t p = active ? (uint32_t)(y * v.W + x) : 0u;
-    bool done = !active || st.good >= REQ || st.s >= N;
-    while (__ballot(!done) != 0ull) {
-        const uint32_t s = st.s + (uint32_t)sub;
-        bool m = false;
-        uint32_t td = kBig, ts = kBig;
-        if (!done && s < N) {
-            uint64_t ra;
-            uint32_t rb;
-            fetch_raw<C>(v, s, p, ra, rb);
-            uint32_t col[C], desc[C];
-            sample_value<C>(v, frame, x, y, s, applied, sbm, ra, rb, col, desc);
-            m = test_sample<C, ALGO, RS>(px, lut, col, desc, td, ts);
-        }
-        const uint32_t bits = (uint32_t)(__ballot(m) >> gbase) & 0xFFu;
-        uint32_t lim = kGroup;  // lanes whose sample precedes the stopping point
-        bool stop = false;
-        if (!done) {
-            const uint32_t need = REQ - st.good;
-            if ((uint32_t)__popc(bits) >= need) {
-                uint32_t c = 0, pos = 0;
-                for (uint32_t k = 0; k < (uint32_t)kGroup; ++k)
-                    if ((bits >> k) & 1u) {
-                        if (++c == need) {
-                            pos = k;
-                            break;
-                        }
-                    }
-                lim = pos + 1u;
-                stop = true;
-            }
-        }
-        uint32_t tdv = (m && (uint32_t)sub < lim) ? td : kBig, tsv = (m && (uint32_t)sub < lim) ? ts : kBig;
-#pragma unroll
-        for (int o = 1; o < kGroup; o <<= 1) {
-            const uint32_t a = (uint32_t)__shfl_xor((int)tdv, o, 64), b = (uint32_t)__shfl_xor((int)tsv, o, 64);
-            tdv = a < tdv ? a : tdv;
-            tsv = b < tsv ? b : tsv;
-        }
-        if (!done) {
-            st.md = tdv < st.md ? tdv : st.md;
-            st.ms = tsv < st.ms ? tsv : st.ms;
-            if (stop) {
-                st.good = REQ;
-                st.s += lim;
-                done = true;
-            } else {
-                st.good += (uint32_t)__popc(bits);
-                st.s = st.s + kGroup < N ? st.s + kGroup : N;
-                done = st.s >= N;
-            }
-        }
-    }
-}
-
 LV_D uint32_t pack_state(const ScanState& st) { return mres_pack(st.good, st.md, st.ms, st.s); }
 
 LV_D ScanState unpack_state(uint32_t mr) {
@@ -706,7 +603,6 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     if (bid == 0 && threadIdx.x == 0) {
         // per-frame counters consumed by later kernels of this step
         for (int i = 0; i < kWlRing; ++i) v.sc->wl_count[i] = 0;
-        v.sc->cont2_count = 0;
         for (int i = 0; i < 8; ++i) v.sc->wl_work[i] = 0;
         v.sc->iters = 0;
     }
@@ -800,31 +696,6 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
         }
     }
     if constexpr (ALGO == kSuBSENSE) block_add<TPB>(nz ? 1ull : 0ull, v.sc->nz_part);
-}
-
-// builds the match context of ROI pixel (x,y); taps from the LDS tile or from global memory
-template <int C, int ALGO, int RS>
-LV_D void build_ctx(const View& v, const uint8_t* frame, const uint8_t* win, int x, int y, PxCtx<C>& px) {
-    const uint32_t p = (uint32_t)(y * v.W + x);
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        px.cur[c] = G(frame)[(size_t)p * C + c];
-        px.intra[c] = G(v.desc_cur)[(size_t)p * C + c];
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            uint32_t acc = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int n = 4 * w + k;
-                acc |= (uint32_t)win[(kLbspDY[n] + 2) * RS + (kLbspDX[n] + 2) * C + c] << (8 * k);
-            }
-            px.taps[c][w] = acc;
-        }
-    if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, G(v.R)[p], G(v.unstable)[p], px);
-    else lobster_thresholds<C>(v, px);
 }
 
 // a tile pixel's per-frame match inputs, loaded together with the tile and staged in LDS (the
@@ -960,13 +831,130 @@ LV_D void build_ctx_global(const View& v, const uint8_t* frame, int x, int y, Px
     else lobster_thresholds<C>(v, px);
 }
 
-// 5x5 patch of one pixel staged in LDS by the kGroup lanes that share it (row stride 5*C)
-template <int C>
-LV_D void stage_patch(const uint8_t* frame, int W, int x, int y, uint8_t* patch, int sub) {
-    for (int j = sub; j < 25 * C; j += kGroup) {
-        const int r = j / (5 * C), rem = j % (5 * C);
-        patch[j] = G(frame)[((size_t)(y - 2 + r) * W + (x - 2)) * C + rem];
+// ----------------------------------------------------------------------------------------------
+// group match: the kGroup lanes of a group work on one pixel. A scan that one lane runs as a chain of
+// dependent loads (50 samples: 13 rounds of four) takes four rounds here, and the twelve records and
+// decisions of the raster-earlier neighbours are read by twelve lanes at once.
+// ----------------------------------------------------------------------------------------------
+struct GroupLds {
+    uint32_t taps[TPB / kGroup][12];
+};
+
+LV_D int pred_dx(uint32_t i) { return (int)(i % 5u) - 2; }
+LV_D int pred_dy(uint32_t i) { return (int)(i / 5u) - 2; }
+
+// Writers of p applied by the match: bit i of the result is set when predecessor i targets p with an
+// open forward gate and its decision is background (CURRENT: the decisions of the fix point, else those of
+// the previous frame). slot = the sample slot lane i's predecessor writes. Every lane of the wavefront calls.
+template <bool CURRENT>
+LV_D uint32_t group_writers(const View& v, int x, int y, bool active, uint32_t& slot) {
+    const int lane = (int)(threadIdx.x & 63u), gbase = lane & ~(kGroup - 1);
+    const uint32_t sub = (uint32_t)(lane & (kGroup - 1));
+    bool on = false;
+    slot = 0;
+    if (active && sub < 12u) {
+        const int dx = pred_dx(sub), dy = pred_dy(sub);
+        const uint32_t q = (uint32_t)((y + dy) * v.W + (x + dx));
+        const uint32_t r = G(v.rec)[q];
+        const uint8_t d = CURRENT ? __hip_atomic_load(&v.dec[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                  : G(v.last_raw)[q];
+        on = rec_tgt(r) == (uint32_t)((2 - dy) * 5 + (2 - dx)) && fwd_gate(r) && d == 0;
+        slot = rec_slot_diff(r);
     }
+    return (uint32_t)(__ballot(on) >> gbase) & 0xFFFu;
+}
+
+// Scans on from st.s to REQ matches or N samples. Every lane of the wavefront calls; the lanes of a group
+// share px, x, y, applied and st.
+template <int C, int ALGO>
+LV_D void scan_group(const View& v, const uint8_t* frame, const uint8_t* lut, const PxCtx<C>& px, int x, int y,
+                     uint32_t applied, uint32_t slot, ScanState& st, bool active) {
+    const uint32_t N = (uint32_t)v.N, REQ = (uint32_t)v.REQ;
+    const int lane = (int)(threadIdx.x & 63u), gbase = lane & ~(kGroup - 1);
+    const uint32_t p = active ? (uint32_t)(y * v.W + x) : 0u;
+    bool done = !active || st.good >= REQ || st.s >= N;
+    while (__ballot(!done) != 0ull) {
+        const uint32_t s = st.s + (uint32_t)(lane - gbase);
+        const bool mine = !done && s < N;
+        // the last applied writer of this sample, if any
+        int w = -1;
+        for (uint32_t m = done ? 0u : applied; __ballot(m != 0u) != 0ull; m &= m - 1u) {
+            const int i = m ? __builtin_ctz(m) : 0;
+            const uint32_t si = (uint32_t)__shfl((int)slot, gbase + i, 64);
+            if (m != 0u && si == s) w = i;
+        }
+        bool match = false;
+        uint32_t td = 0, ts = 0;
+        if (mine) {
+            uint64_t ra;
+            uint32_t rb;
+            if (w >= 0) raw_current<C>(v, frame, (uint32_t)((y + pred_dy((uint32_t)w)) * v.W + x + pred_dx((uint32_t)w)), ra, rb);
+            else fetch_raw<C>(v, s, p, ra, rb);
+            uint32_t col[C], desc[C];
+            decode_raw<C>(ra, rb, col, desc);
+            match = test_sample<C, ALGO, 0>(px, lut, col, desc, td, ts);
+        }
+        // matches in sample order (few: at most REQ are taken)
+        uint32_t bits = done ? 0u : (uint32_t)(__ballot(match) >> gbase) & ((1u << kGroup) - 1u);
+        const uint32_t dist = td << 16 | ts;
+        while (__ballot(bits != 0u) != 0ull) {
+            const int i = bits ? __builtin_ctz(bits) : 0;
+            const uint32_t d = (uint32_t)__shfl((int)dist, gbase + i, 64);
+            if (bits) {
+                bits &= bits - 1u;
+                const uint32_t a = d >> 16, b = d & 0xFFFFu;
+                st.md = a < st.md ? a : st.md;
+                st.ms = b < st.ms ? b : st.ms;
+                if (++st.good == REQ) {
+                    st.s += (uint32_t)i + 1u;
+                    bits = 0;
+                    done = true;
+                }
+            }
+        }
+        if (!done) {
+            st.s = st.s + kGroup < N ? st.s + kGroup : N;
+            done = st.s >= N;
+        }
+    }
+}
+
+// the match context of the group's pixel from global memory: lane 4c+w packs tap word w of channel c
+template <int C, int ALGO>
+LV_D void group_ctx(const View& v, const uint8_t* frame, int x, int y, bool active, GroupLds& L, PxCtx<C>& px) {
+    const uint32_t sub = threadIdx.x & (kGroup - 1), g = threadIdx.x / kGroup, p = (uint32_t)(y * v.W + x);
+    if (active && sub < 4u * C) {
+        const uint32_t w = sub & 3u, c = sub >> 2;
+        // (dx + 2) | (dy + 2) << 4 of taps 4w .. 4w+3, one byte each
+        constexpr auto code = [](int n) { return (uint32_t)((kLbspDX[n] + 2) | ((kLbspDY[n] + 2) << 4)); };
+        constexpr auto codes = [code](int a) {
+            return code(a) | code(a + 1) << 8 | code(a + 2) << 16 | code(a + 3) << 24;
+        };
+        constexpr uint32_t k0 = codes(0), k1 = codes(4), k2 = codes(8), k3 = codes(12);
+        const uint32_t ks = w == 0u ? k0 : w == 1u ? k1 : w == 2u ? k2 : k3;
+        uint32_t acc = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int dx = (int)((ks >> (8 * k)) & 15u) - 2, dy = (int)((ks >> (8 * k + 4)) & 15u) - 2;
+            acc |= (uint32_t)G(frame)[((size_t)(y + dy) * v.W + (x + dx)) * C + c] << (8 * k);
+        }
+        L.taps[g][sub] = acc;
+    }
+    if (active) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            px.cur[c] = G(frame)[(size_t)p * C + c];
+            px.intra[c] = G(v.desc_cur)[(size_t)p * C + c];
+        }
+        if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, G(v.R)[p], G(v.unstable)[p], px);
+        else lobster_thresholds<C>(v, px);
+    }
+    wave_sync();
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) px.taps[c][w] = L.taps[g][4 * c + w];
+    wave_sync();  // read before the group's next pixel overwrites them
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -1132,34 +1120,43 @@ LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, c
     int nrep;
     ScanState st = scan_init<C>();
     const uint32_t N = (uint32_t)v.N;
-    // more than kRepl overwritten slots (very rare): the whole scan goes to the cooperative phase.
+    // more than kRepl overwritten slots (very rare): the pixel keeps its guess for now and goes to the first
+    // fix-point worklist itself, where a group matches it against any number of writers.
     // The replacements are gathered before the context is built, so the two are not live together.
     auto rec_of = [&](int i) { return pred.rec[ly + 2 + kPredDY[i]][lx + 2 + kPredDX[i]]; };
-    const uint32_t limit =
-        build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of) ? (seq_limit < N ? seq_limit : N) : 0u;
+    const uint8_t guess = pred.guess[ly + 2][lx + 2];
+    const bool fits = build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
+    const uint32_t limit = !fits ? 0u : seq_limit < N ? seq_limit : N;
     build_ctx_staged<C, ALGO, FrameTile<C>::LW * C>(v, &tile.px[(ly * FrameTile<C>::LW + lx) * C], in, px);
     scan_seq<C, ALGO, FrameTile<C>::LW * C, KF>(v, lut, px, x, y, sbm, nrep, st, limit);
     examined = st.s;
     G(v.mres)[p] = pack_state(st);
-    if (st.good < (uint32_t)v.REQ && st.s < N) return false;
-    const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
+    if (fits && st.good < (uint32_t)v.REQ && st.s < N) return false;
+    const uint8_t fg = !fits ? guess : st.good < (uint32_t)v.REQ ? 1 : 0;
     G(v.dec)[p] = fg;
-    push = fg != pred.guess[ly + 2][lx + 2] && forward_target(v, pred.rec[ly + 2][lx + 2], x, y, target);
+    push = fg != guess && forward_target(v, pred.rec[ly + 2][lx + 2], x, y, target);
+    if (!fits) {
+        push = true;
+        target = p;
+    }
     return true;
 }
 
-// candidate writers of p whose decision is background: guessed from the previous raw mask, or the
-// current decisions during the fix point
-template <bool CURRENT>
+// candidate writers of p that were background in the previous frame, by one lane
 LV_D uint32_t applied_writers_global(const View& v, int x, int y) {
-    const uint32_t cand = candidate_writers(v, x, y);
-    uint32_t applied = 0;
-    for (uint32_t m = cand; m; m &= m - 1) {
-        const int i = __builtin_ctz(m);
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
         const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
-        const uint8_t d = CURRENT ? __hip_atomic_load(&v.dec[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                  : (G(v.last_raw)[q] ? 1 : 0);
-        if (d == 0) applied |= 1u << i;
+        const uint32_t r = G(v.rec)[q];
+        const uint32_t code = (uint32_t)((2 - kPredDY[i]) * 5 + (2 - kPredDX[i]));
+        if (rec_tgt(r) == code && fwd_gate(r)) m |= 1u << i;
+    }
+    uint32_t applied = 0;
+    for (; m; m &= m - 1) {
+        const int i = __builtin_ctz(m);
+        const uint32_t q = (uint32_t)((y + pred_dy((uint32_t)i)) * v.W + (x + pred_dx((uint32_t)i)));
+        if (G(v.last_raw)[q] == 0) applied |= 1u << i;
     }
     return applied;
 }
@@ -1175,10 +1172,6 @@ LV_D bool finish_pixel(const View& v, uint32_t p, int x, int y, const ScanState&
     return fg != guess && forward_target(v, G(v.rec)[p], x, y, t);
 }
 
-// the stripe of the pixel's tile
-LV_D uint32_t tile_stripe(const View& v, int x, int y) {
-    return (uint32_t)((y / TH) * ((v.W + TW - 1) / TW) + x / TW) % (uint32_t)kContStripes;
-}
 // push_first for lanes of different stripes: one append per stripe present in the wavefront
 LV_D void push_first_mixed(const View& v, bool push, uint32_t t, uint32_t stripe) {
     unsigned long long bal = __ballot(push);
@@ -1190,21 +1183,18 @@ LV_D void push_first_mixed(const View& v, bool push, uint32_t t, uint32_t stripe
     }
 }
 
-// Phase B: the scans phase A cut at its sample limit, continued with one lane per pixel over the
-// dense list of unfinished pixels (its stripes walked in order), so long scans (mostly foreground
-// pixels, which examine every sample) fill whole wavefronts. The context is the one phase A cached
-// (rebuilt from global memory past a stripe's cache); a pixel with more than kRepl overwritten
-// slots goes on to phase C.
+// Phase B continues the scans phase A cut, over the dense list of unfinished pixels (its stripes walked in
+// order), with the context phase A cached (rebuilt from global memory past a stripe's cache).
+// Two forms, chosen by the length of the list: a group per pixel up to View::group_limit entries,
+// which is what the chip holds at once (256 CUs x 24 wavefronts x 4 groups = 24 K, taken as 32 K): there a lane
+// per pixel leaves most of it idle behind chains of 13 dependent loads. Past it a lane per pixel does the
+// same work with fewer instructions. Measured per frame, lanes / groups: 320x240 RGB 160 / 127 us
+// (1 K entries), 640x480 194 / 153 (20 K), 960x720 254 / 260 (50 K), 1920x1080 408 / 423 (170 K),
+// 3840x2160 1208 / 1282 (450 K).
 template <int C, int ALGO, int KF>
-LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
+LV_D void match_seq_lanes(const View& v, const uint8_t* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
+                          uint32_t nblk) {
     const uint8_t* frame = v.frame;
-    __shared__ uint8_t lut[256];
-    __shared__ uint32_t s_pre[kContStripes + 1];  // exclusive prefix of the stripe counts
-    stripe_prefix(v.sc->cont_cnt, s_pre);
-    load_lut(lut, v.sc);
-    __syncthreads();
-    const uint32_t n = s_pre[kContStripes];
-    if (bid * TPB >= n) return;  // uniform: no item reaches this block
     uint32_t examined = 0;
     for (uint32_t i = bid * TPB + threadIdx.x; i < n; i += nblk * TPB) {
         const uint32_t k = stripe_of(s_pre, i);  // item i = entry j of stripe k
@@ -1214,18 +1204,54 @@ LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
         PxCtx<C> px;
         if (j < v.cont_ctx_region) load_ctx<C>(v.cont_ctx + ((size_t)k * v.cont_ctx_region + j) * kCtxWords, px);
         else build_ctx_global<C, ALGO>(v, frame, x, y, px);
-        const uint32_t applied = applied_writers_global<false>(v, x, y);
+        const uint32_t applied = applied_writers_global(v, x, y);
         uint64_t sbm;
         int nrep;
         auto rec_of = [&](int i) { return G(v.rec)[(size_t)(y + kPredDY[i]) * v.W + (x + kPredDX[i])]; };
+        // at most kRepl slots: phase A keeps the others (same writers, same guesses)
+        (void)build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
+        ScanState st = unpack_state(G(v.mres)[p]);
+        const uint32_t s0 = st.s;
+        scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
+        examined += st.s - s0;
+        uint32_t t = 0;
+        const bool push = finish_pixel<C>(v, p, x, y, st, t);
+        push_first_mixed(v, push, t, k);
+    }
+    block_add<TPB>(examined, v.sc->coop_part);
+}
+
+template <int C, int ALGO>
+LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
+                           uint32_t nblk) {
+    const uint8_t* frame = v.frame;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t step = nblk * (TPB / kGroup);
+    uint32_t examined = 0;
+    for (uint32_t i0 = (bid * TPB + (threadIdx.x & ~63u)) / kGroup; i0 < n; i0 += step) {  // uniform per wavefront
+        const uint32_t i = i0 + lane / kGroup;
+        const bool active = i < n;
+        uint32_t k = 0, p = 0;
+        PxCtx<C> px{};
+        ScanState st = scan_init<C>();
+        int x = 0, y = 0;
+        if (active) {
+            k = stripe_of(s_pre, i);
+            const uint32_t j = i - s_pre[k];
+            p = G(v.cont)[(size_t)k * v.cont_region + j];
+            x = (int)(p % (uint32_t)v.W);
+            y = (int)(p / (uint32_t)v.W);
+            if (j < v.cont_ctx_region) load_ctx<C>(v.cont_ctx + ((size_t)k * v.cont_ctx_region + j) * kCtxWords, px);
+            else build_ctx_global<C, ALGO>(v, frame, x, y, px);
+            st = unpack_state(G(v.mres)[p]);
+        }
+        uint32_t slot;
+        const uint32_t applied = group_writers<false>(v, x, y, active, slot);
+        const uint32_t s0 = st.s;
+        scan_group<C, ALGO>(v, frame, lut, px, x, y, applied, slot, st, active);
         bool push = false;
         uint32_t t = 0;
-        if (!build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of)) {
-            v.cont2[atomicAdd(&v.sc->cont2_count, 1u)] = p;
-        } else {
-            ScanState st = unpack_state(G(v.mres)[p]);
-            const uint32_t s0 = st.s;
-            scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
+        if (active && lane % kGroup == 0) {
             examined += st.s - s0;
             push = finish_pixel<C>(v, p, x, y, st, t);
         }
@@ -1234,52 +1260,18 @@ LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
     block_add<TPB>(examined, v.sc->coop_part);
 }
 
-// Phase C: pixels left by phase B (more than kRepl overwritten slots), kGroup lanes per pixel
-template <int C, int ALGO>
-LV_D void match_cont_body(const View& v, uint32_t bid, uint32_t nblk) {
-    const uint8_t* frame = v.frame;
+template <int C, int ALGO, int KF>
+LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
     __shared__ uint8_t lut[256];
-    __shared__ uint8_t patches[TPB / kGroup][25 * C];
-    const uint32_t n = v.sc->cont2_count;
-    if (bid * (TPB / kGroup) >= n) return;  // uniform: no item reaches this block
+    __shared__ uint32_t s_pre[kContStripes + 1];  // exclusive prefix of the stripe counts
+    stripe_prefix(v.sc->cont_cnt, s_pre);
     load_lut(lut, v.sc);
     __syncthreads();
-    uint8_t* patch = patches[threadIdx.x / kGroup];
-    const uint32_t ngroups = nblk * (TPB / kGroup);
-    const uint32_t sub = threadIdx.x & (kGroup - 1);
-    const uint32_t g0 = (bid * TPB + threadIdx.x) / kGroup;
-    const uint32_t rounds = (n + ngroups - 1) / ngroups;  // uniform trip count: every lane takes part
-    uint64_t examined = 0;
-    for (uint32_t r = 0; r < rounds; ++r) {
-        const uint32_t i = g0 + r * ngroups;
-        const bool active = i < n;
-        const uint32_t p = active ? G(v.cont2)[i] : 0u;
-        const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
-        PxCtx<C> px;
-        uint32_t applied = 0;
-        uint64_t sbm = 0;
-        ScanState st = scan_init<C>();
-        __syncthreads();  // previous round's readers of the patch are done
-        if (active) {
-            stage_patch<C>(frame, v.W, x, y, patch, (int)sub);
-            wave_sync();  // the group's patch bytes, written by its eight lanes
-            build_ctx<C, ALGO, 5 * C>(v, frame, patch, x, y, px);
-            applied = applied_writers_global<false>(v, x, y);
-            sbm = applied_slots(v, x, y, applied);
-            st = unpack_state(G(v.mres)[p]);
-        }
-        __syncthreads();
-        const uint32_t s_before = st.s;
-        scan_coop<C, ALGO, 5 * C>(v, frame, lut, px, x, y, applied, sbm, st, active);
-        bool push = false;
-        uint32_t t = 0;
-        if (active && sub == 0) {
-            examined += st.s - s_before;
-            push = finish_pixel<C>(v, p, x, y, st, t);
-        }
-        push_first_mixed(v, push, t, tile_stripe(v, x, y));
-    }
-    block_add<TPB>(examined, v.sc->coop_part);
+    const uint32_t n = s_pre[kContStripes];
+    const bool groups = n <= v.group_limit;
+    if (bid * (groups ? TPB / kGroup : TPB) >= n) return;  // uniform: no item reaches this block
+    if (groups) match_seq_groups<C, ALGO>(v, lut, s_pre, n, bid, nblk);
+    else match_seq_lanes<C, ALGO, KF>(v, lut, s_pre, n, bid, nblk);
 }
 
 // worklist of fix-point iteration k: entry i, and its entry count for every thread of the block (pre:
@@ -1298,30 +1290,24 @@ LV_D uint32_t wl_total(const View& v, uint32_t k, uint32_t* pre) {
     return pre[kContStripes];
 }
 
-// fix-point re-match of worklisted pixels (all lanes call; kGroup lanes per item)
+// fix-point re-match of a wavefront's worklisted pixels i0 .. i0 + 64/kGroup - 1, one group each
 template <int C, int ALGO>
-LV_D void rematch_round(const View& v, const uint8_t* frame, const uint8_t* lut, uint8_t* patch, const uint32_t* pre,
-                        uint32_t n, uint32_t i, uint32_t k, uint32_t* wl_next) {
+LV_D void rematch(const View& v, const uint8_t* lut, GroupLds& L, const uint32_t* pre, uint32_t n, uint32_t i0,
+                  uint32_t k, uint32_t* wl_next) {
+    const uint8_t* frame = v.frame;
+    const uint32_t lane = threadIdx.x & 63u, i = i0 + lane / kGroup;
     const bool active = i < n;
     const uint32_t p = active ? wl_item(v, k, pre, i) : 0u;
     const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
-    PxCtx<C> px;
-    uint32_t applied = 0;
-    uint64_t sbm = 0;
-    __syncthreads();  // previous round's readers of the patch are done
-    if (active) {
-        stage_patch<C>(frame, v.W, x, y, patch, (int)(threadIdx.x & (kGroup - 1)));
-        wave_sync();  // the group's patch bytes, written by its eight lanes
-        build_ctx<C, ALGO, 5 * C>(v, frame, patch, x, y, px);
-        applied = applied_writers_global<true>(v, x, y);
-        sbm = applied_slots(v, x, y, applied);
-    }
-    __syncthreads();
+    uint32_t slot;
+    const uint32_t applied = group_writers<true>(v, x, y, active, slot);
+    PxCtx<C> px{};
+    group_ctx<C, ALGO>(v, frame, x, y, active, L, px);
     ScanState st = scan_init<C>();
-    scan_coop<C, ALGO, 5 * C>(v, frame, lut, px, x, y, applied, sbm, st, active);
+    scan_group<C, ALGO>(v, frame, lut, px, x, y, applied, slot, st, active);
     bool push = false;
     uint32_t t = 0;
-    if (active && (threadIdx.x & (kGroup - 1)) == 0) {
+    if (active && lane % kGroup == 0) {
         G(v.mres)[p] = pack_state(st);
         const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
         const uint8_t old = G(v.dec)[p];
@@ -1336,9 +1322,8 @@ LV_D void rematch_round(const View& v, const uint8_t* frame, const uint8_t* lut,
 // fix-point iteration k (k >= 1): worklist k -> worklist k+1
 template <int C, int ALGO>
 LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k) {
-    const uint8_t* frame = v.frame;
     __shared__ uint8_t lut[256];
-    __shared__ uint8_t patches[TPB / kGroup][25 * C];
+    __shared__ GroupLds L;
     __shared__ uint32_t s_pre[kContStripes + 1];
     // slot k+2 was last read by iteration k-2 (finished); it must be empty before iteration k+1
     // pushes into it, whether or not this iteration has work.
@@ -1355,19 +1340,16 @@ LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k) 
     load_lut(lut, v.sc);
     __syncthreads();
     uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
-    const uint32_t ngroups = nblk * (TPB / kGroup);
-    const uint32_t g0 = (bid * TPB + threadIdx.x) / kGroup;
-    const uint32_t rounds = (n + ngroups - 1) / ngroups;
-    for (uint32_t r = 0; r < rounds; ++r)
-        rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], s_pre, n, g0 + r * ngroups, k, wl_next);
+    const uint32_t step = nblk * (TPB / kGroup);
+    for (uint32_t i0 = (bid * TPB + (threadIdx.x & ~63u)) / kGroup; i0 < n; i0 += step)
+        rematch<C, ALGO>(v, lut, L, s_pre, n, i0, k, wl_next);
 }
 
 // remaining fix-point iterations in one workgroup (normally no work is left)
 template <int C, int ALGO>
 LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k0, uint32_t cap) {
-    const uint8_t* frame = v.frame;
     __shared__ uint8_t lut[256];
-    __shared__ uint8_t patches[256 / kGroup][25 * C];
+    __shared__ GroupLds L;
     __shared__ uint32_t s_pre[kContStripes + 1];
     __shared__ uint32_t s_n;
     load_lut(lut, v.sc);
@@ -1394,10 +1376,8 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
         const uint32_t n = s_n;
         if (n == 0) break;
         uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
-        const uint32_t ngroups = blockDim.x / kGroup, g0 = threadIdx.x / kGroup;
-        const uint32_t rounds = (n + ngroups - 1) / ngroups;
-        for (uint32_t r = 0; r < rounds; ++r)
-            rematch_round<C, ALGO>(v, frame, lut, patches[threadIdx.x / kGroup], s_pre, n, g0 + r * ngroups, k, wl_next);
+        for (uint32_t i0 = (threadIdx.x & ~63u) / kGroup; i0 < n; i0 += TPB / kGroup)
+            rematch<C, ALGO>(v, lut, L, s_pre, n, i0, k, wl_next);
         __threadfence();
     }
 }
@@ -2492,6 +2472,9 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
 }
 
 #define LV_SINGLE_BID ((uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x)), gridDim.x
+// kernels over a list that may fill only the first blocks: in dispatch order, so every XCD gets a share
+// (remapped, 700 busy blocks of 4096 would all run on two XCDs)
+#define LV_LIST_BID blockIdx.x, gridDim.x
 
 template <int C, int ALGO>
 __global__ void __launch_bounds__(TPB) k_describe(View v) { describe_body<C, ALGO>(v, LV_SINGLE_BID); }
@@ -2502,12 +2485,10 @@ __global__ void __launch_bounds__(TPB) LV_MATCH_WAVES(KF) k_match(View v) { matc
 // phase B holds 80 VGPRs at occupancy 6 as well
 template <int C, int ALGO, int KF>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(6))) k_match_seq(View v) {
-    match_seq_body<C, ALGO, KF>(v, LV_SINGLE_BID);
+    match_seq_body<C, ALGO, KF>(v, LV_LIST_BID);
 }
 template <int C, int ALGO>
-__global__ void __launch_bounds__(TPB) k_match_cont(View v) { match_cont_body<C, ALGO>(v, LV_SINGLE_BID); }
-template <int C, int ALGO>
-__global__ void __launch_bounds__(TPB) k_fixpoint(View v, uint32_t k) { fixpoint_body<C, ALGO>(v, LV_SINGLE_BID, k); }
+__global__ void __launch_bounds__(TPB) k_fixpoint(View v, uint32_t k) { fixpoint_body<C, ALGO>(v, LV_LIST_BID, k); }
 template <int C, int ALGO>
 __global__ void __launch_bounds__(256) k_fixpoint_tail(View v, uint32_t k0, uint32_t cap) {
     fixpoint_tail_body<C, ALGO>(v, 0u, 1u, k0, cap);
@@ -2550,7 +2531,6 @@ template <int KF>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(6))) kb_match_seq(BatchArgs b) {
     LV_BATCH_C(match_seq_body, kSuBSENSE, KF);
 }
-__global__ void __launch_bounds__(TPB) kb_match_cont(BatchArgs b) { LV_BATCH_C(match_cont_body, kSuBSENSE); }
 __global__ void __launch_bounds__(TPB) kb_fixpoint(BatchArgs b, uint32_t k) {
     for_batch_block(b, [&](const View& v, uint32_t bid, uint32_t nblk) {
         if (v.C == 3) fixpoint_body<3, kSuBSENSE>(v, bid, nblk, k);
@@ -2595,10 +2575,14 @@ void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]) 
     g[kGridPix] = cdiv(v.npx, TPB);
     g[kGridCell] = !v.lr_scaling ? 0u : cdiv((size_t)v.dsW * v.dsH, TPB);
     g[kGridOne] = 1u;
-    g[kGridFix] = (uint32_t)opt.fixpoint_blocks;
+    // single stream: a block per 1024 pixels (16 groups each; the worklists hold a few per cent of them)
+    g[kGridFix] = opt.fixpoint_blocks > 0 ? (uint32_t)opt.fixpoint_blocks
+                                          : std::max(32u, std::min(1024u, cdiv(v.npx, 1024)));
     if (opt.fix_px_per_block > 0) g[kGridFix] = std::min(g[kGridFix], cdiv(v.npx, (size_t)opt.fix_px_per_block));
     g[kGridSweep] = std::min(cdiv(v.npx, TPB), 128u);
-    g[kGridCont] = (uint32_t)opt.cont_blocks;
+    // single stream: a block per 256 pixels, at most what covers group_limit entries in one round
+    g[kGridCont] = opt.cont_blocks > 0 ? (uint32_t)opt.cont_blocks
+                                       : std::max(64u, std::min(kGroupLimit / (TPB / kGroup), cdiv(v.npx, TPB)));
     if (opt.cont_px_per_block > 0) g[kGridCont] = std::min(g[kGridCont], cdiv(v.npx, (size_t)opt.cont_px_per_block));
 }
 
@@ -2612,15 +2596,15 @@ static void frame_step_t(const View& v, const StepOptions& opt, hipStream_t st) 
     if (opt.fetch_depth == 4) hipLaunchKernelGGL((k_match<C, ALGO, 4>), dim3(g[kGridTile]), dim3(TPB), 0, st, v);
     else hipLaunchKernelGGL((k_match<C, ALGO, 2>), dim3(g[kGridTile]), dim3(TPB), 0, st, v);
     if (opt.timed_stage == 1) (void)hipEventRecord(opt.ev_end, st);
-    // phases B and C finish what phase A left (scans cut at seq_limit, pixels with more than kRepl
-    // overwritten slots); they exit at once when nothing was left
+    // phase B finishes the scans phase A cut; it exits at once when there are none
     if (opt.fetch_depth == 4) hipLaunchKernelGGL((k_match_seq<C, ALGO, 4>), dim3(g[kGridCont]), dim3(TPB), 0, st, v);
     else hipLaunchKernelGGL((k_match_seq<C, ALGO, 2>), dim3(g[kGridCont]), dim3(TPB), 0, st, v);
-    hipLaunchKernelGGL((k_match_cont<C, ALGO>), dim3(g[kGridCont]), dim3(TPB), 0, st, v);
-    for (uint32_t k = 1; k <= (uint32_t)opt.fixpoint_launches; ++k)
+    // the second iteration's worklist is about a hundredth of the first's: on small frames (a dozen entries)
+    // the tail takes it (320x240 126.8 -> 124.8 us; 1920x1080 408 -> 420)
+    const uint32_t launches = opt.fixpoint_launches >= 0 ? (uint32_t)opt.fixpoint_launches : v.npx < 600000u ? 1u : 2u;
+    for (uint32_t k = 1; k <= launches; ++k)
         hipLaunchKernelGGL((k_fixpoint<C, ALGO>), dim3(g[kGridFix]), dim3(TPB), 0, st, v, k);
-    hipLaunchKernelGGL((k_fixpoint_tail<C, ALGO>), dim3(1), dim3(256), 0, st, v, (uint32_t)opt.fixpoint_launches + 1u,
-                       (uint32_t)opt.tail_cap);
+    hipLaunchKernelGGL((k_fixpoint_tail<C, ALGO>), dim3(1), dim3(256), 0, st, v, launches + 1u, (uint32_t)opt.tail_cap);
     if constexpr (ALGO == kSuBSENSE) {
         if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
         hipLaunchKernelGGL((k_update<C, ALGO, true>), dim3(g[kGridTile]), dim3(TPB), 0, st, v);
@@ -2669,7 +2653,6 @@ void batch_step(const View* d_views, int ns, const uint32_t* const prefix[kNumGr
     if (opt.timed_stage == 1) (void)hipEventRecord(opt.ev_end, st);
     if (opt.fetch_depth == 4) hipLaunchKernelGGL(kb_match_seq<4>, dim3(total[kGridCont]), dim3(TPB), 0, st, args(kGridCont));
     else hipLaunchKernelGGL(kb_match_seq<2>, dim3(total[kGridCont]), dim3(TPB), 0, st, args(kGridCont));
-    hipLaunchKernelGGL(kb_match_cont, dim3(total[kGridCont]), dim3(TPB), 0, st, args(kGridCont));
     for (uint32_t k = 1; k <= (uint32_t)opt.fixpoint_launches; ++k)
         hipLaunchKernelGGL(kb_fixpoint, dim3(total[kGridFix]), dim3(TPB), 0, st, args(kGridFix), k);
     hipLaunchKernelGGL(kb_fixpoint_tail, dim3(total[kGridOne]), dim3(256), 0, st, args(kGridOne),

@@ -10,15 +10,20 @@ namespace lvbgs {
 // scan may load past a pixel's last sample
 constexpr int kMaxFetch = 4;
 constexpr int kCtxWords = 20;  // words of a cached match context
+// entries of a continuation list up to which phase B of the match gives each a lane group; the streams of
+// a batch share it
+constexpr uint32_t kGroupLimit = 32768;
 
 struct StepOptions {
-    int fixpoint_launches = 2;   // fix-point iterations launched as full-grid kernels
-    int fixpoint_blocks = 256;   // grid of each fix-point kernel (grid-stride over the worklist)
+    // fix-point iterations launched as full-grid kernels, and their grid (grid-stride over the worklist);
+    // < 0 and 0: the single-stream path's choice by frame size (kernel_grids, frame_step)
+    int fixpoint_launches = -1;
+    int fixpoint_blocks = 0;
     int tail_cap = 1 << 16;      // iteration cap of the single-workgroup tail (error flag if reached)
     int seq_limit = 0;           // samples scanned per pixel by the sequential phase of the match
                                  // (0: the single-stream path's automatic choice)
     int fetch_depth = 4;         // sample loads in flight per lane in the sequential phase (2 or 4)
-    int cont_blocks = 1024;      // grid of the cooperative phase (grid-stride over unfinished pixels)
+    int cont_blocks = 0;         // grid of phase B (grid-stride over unfinished pixels; 0: by frame size)
     int fix_px_per_block = 0;    // > 0: fix-point grid of a stream = ceil(npx / this), at most fixpoint_blocks
     int cont_px_per_block = 0;   // > 0: cooperative grid of a stream = ceil(npx / this), at most cont_blocks
     int timed_stage = 0;         // 0: none, 1: the match kernel (phase A), 2: the whole step, 3: the update kernel

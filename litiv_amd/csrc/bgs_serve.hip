@@ -352,6 +352,7 @@ static int launch_step(lvbgs_server* s) {
             v.out_mask = r.mask;
             v.lr = r.lr;
             v.seq_limit = (uint32_t)s->opt.seq_limit;
+            v.group_limit = kGroupLimit / (uint32_t)n;
             hv[pos] = v;
             uint32_t gk[kNumGrids];
             kernel_grids(c->v, s->opt, gk);

@@ -25,6 +25,7 @@ struct View {
     uint8_t* out_mask;       // optional device W*H output mask
     double lr;               // learning-rate override of apply()
     uint32_t seq_limit;      // samples of the sequential match phase
+    uint32_t group_limit;    // continuation entries up to which phase B works in lane groups
     // roi and model
     const uint8_t* roi;      // W*H, 0 = outside
     uint8_t* last_color;     // W*H*C
@@ -54,7 +55,6 @@ struct View {
     uint32_t* cont_ctx;      // match contexts of the first cont_ctx_region entries of each stripe
                              // (kCtxWords each, stripe k at k * cont_ctx_region)
     uint32_t cont_region, cont_ctx_region;
-    uint32_t* cont2;         // pixels left by the continuation to the cooperative phase
     float *dsLT, *dsST;      // (W/8)*(H/8)*C
     Scalars* sc;
     uint32_t* h_err;         // host-visible copy of Scalars::err_flags (pinned), so a synchronizing

@@ -32,6 +32,23 @@ def test_first_worklist_stripes(algo, c, w, h, schedule):
     run_sequence(algo, flashing(w, h, c, 10), schedule=schedule, lr=None if algo == SUBSENSE else 2.0)
 
 
+@pytest.mark.parametrize("algo,c,schedule", [(SUBSENSE, 3, (1, 1024, 2, 256)), (SUBSENSE, 3, (1, 3, 1, 5)),
+                                             (SUBSENSE, 1, (1, 1024, 2, 256)), (LOBSTER, 3, (1, 2, 2, 256)),
+                                             (LOBSTER, 1, (6, 1, 1, 1)), (SUBSENSE, 3, (11, 1, 1, 1))])
+def test_continuation_lanes_and_groups(algo, c, schedule):
+    # seq_limit 1 on 60 K pixels leaves more entries than phase B takes in lane groups (32 K), later limits
+    # fewer; few blocks make the list loops run several rounds with a ragged last one
+    run_sequence(algo, flashing(301, 205, c, 6), schedule=schedule, lr=None if algo == SUBSENSE else 2.0)
+
+
+@pytest.mark.parametrize("lr,limit", [(1.0, 255), (1.0, 3)])
+def test_more_overwritten_slots_than_entries(lr, limit):
+    # learning rate 1 with 5x5 diffusion: every background pixel writes a neighbour, so some pixels have more
+    # than four overwritten slots and go to the fix point unmatched
+    gpu, _ = run_sequence(SUBSENSE, flashing(484, 325, 3, 7), lr=lr, schedule=(limit, 1024, 2, 256))
+    assert gpu.stats()["fixpoint_work"][1] > 0
+
+
 @pytest.mark.parametrize("pad_in,pad_out", [(0, 0), (7, 0), (0, 5), (3, 9)])
 def test_host_rows_packed_and_padded(pad_in, pad_out):
     # packed rows take one linear copy, padded rows the 2-D copy, in and out independently
