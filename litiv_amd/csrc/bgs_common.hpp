@@ -126,17 +126,17 @@ LV_HD void clamp_coords(int& x, int& y, int border, int w, int h) {
     else if (y >= h - border) y = h - border - 1;
 }
 
-// getSamplePosition_7x7_std2 (opencv.hpp:873-925), border 2
-LV_HD void sample_pos_7x7(uint32_t rnd, int x, int y, int w, int h, int& ox, int& oy) {
+// getSamplePosition_7x7_std2 (opencv.hpp:873-925) of a draw modulo 512, as an offset; the position is
+// then clamped with border 2
+LV_HD void sample_offset_7x7(uint32_t rnd, int& dx, int& dy) {
     int r = 1 + (int)(rnd % 512u);
     int i = 0;
     for (; i < 48; ++i) {
         r -= kSample7x7[i];
         if (r <= 0) break;
     }
-    ox = x + (i % 7) - 3;
-    oy = y + (i / 7) - 3;
-    clamp_coords(ox, oy, 2, w, h);
+    dx = (i % 7) - 3;
+    dy = (i / 7) - 3;
 }
 
 // getNeighborPosition_3x3 / _5x5 (opencv.hpp:928-966), border 2

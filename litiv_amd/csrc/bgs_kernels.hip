@@ -173,11 +173,8 @@ LV_D void load_sample(const View& v, uint32_t s, uint32_t p, uint32_t col[C], ui
 }
 
 template <int C>
-LV_D void store_sample(const View& v, uint32_t s, uint32_t p, const uint32_t col[C], const uint32_t desc[C]) {
+LV_D void store_raw(const View& v, uint32_t s, uint32_t p, uint64_t ra, uint32_t rb) {
     const size_t idx = sample_index(v, s, p);
-    uint64_t ra;
-    uint32_t rb;
-    encode_raw<C>(col, desc, ra, rb);
     // non-temporal: scattered single-record writes gain nothing from being kept in L2
     typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
     if constexpr (C == 3) {
@@ -189,6 +186,14 @@ LV_D void store_sample(const View& v, uint32_t s, uint32_t p, const uint32_t col
     } else {
         __builtin_nontemporal_store((uint32_t)ra, G((uint32_t*)v.sA + idx));
     }
+}
+
+template <int C>
+LV_D void store_sample(const View& v, uint32_t s, uint32_t p, const uint32_t col[C], const uint32_t desc[C]) {
+    uint64_t ra;
+    uint32_t rb;
+    encode_raw<C>(col, desc, ra, rb);
+    store_raw<C>(v, s, p, ra, rb);
 }
 
 // current colour and intra descriptor of pixel q (the value it writes into samples)
@@ -2294,15 +2299,30 @@ LV_D void lobster_end_body(const View& v, uint32_t bid, uint32_t nblk) {
     v.sc->epoch += 1u;
 }
 
-// refreshModel (SUB:80-105; LOB:410-440). pending = 1: auto-reset request from k_decide (also
-// T := 1 everywhere, SUB:592); otherwise an explicit call with the given parameters.
-template <int C, int ALGO>
-LV_D void refresh_pixel(const View& v, uint32_t p, int use_pending, int force_fg, uint32_t frame, uint32_t ev,
-                        uint32_t nref, uint32_t start);
+// What the pixels around a tile offer to refreshModel: colour and descriptor as a sample record, and
+// whether they may be sampled. A 3-pixel halo covers getSamplePosition's 7x7 window (its clamping moves a
+// position towards the pixel). A record serves up to 50 samples of each of the 49 pixels around it, so it is
+// built once here (LOBSTER computes its descriptor) instead of per sample from global memory.
+template <int C>
+struct RefreshTile {
+    static constexpr int LW = TW + 6, LH = TH + 6;
+    uint32_t w0[LW * LH];
+    uint32_t w1[C == 3 ? LW * LH : 1], w2[C == 3 ? LW * LH : 1];
+    uint8_t ok[LW * LH];
+    uint8_t pos[512];  // sample position of each draw % 512: dx + 3 | (dy + 3) << 4
+};
 
-// A grid-stride sweep, so the per-step launch (normally nothing pending) stays small.
+// refreshModel (SUB:80-105; LOB:410-440). pending = 1: auto-reset request from k_decide (also
+// T := 1 everywhere, SUB:592); otherwise an explicit call with the given parameters. outside: pixels
+// outside the ROI get zero samples (initialization writes every sample of the model, so that its memory need
+// not be cleared first). A grid-stride sweep over the tiles, so the per-step launch (normally nothing
+// pending) stays small.
+// Bound by the sample stores and the draws: with a table in LDS for the position (a walk of up to 48
+// entries before) and the tile's records 1305 -> 126 us (4.4 TB/s) for the 553 MB of a
+// 1280x720 RGB model.
 template <int C, int ALGO>
-LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pending, float frac, int force_fg, uint32_t frame, uint32_t ev) {
+LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pending, float frac, int force_fg,
+                       uint32_t frame, uint32_t ev, int outside) {
     if (use_pending) {
         if (!v.sc->refresh_pending) return;
         frac = v.sc->refresh_frac;
@@ -2310,6 +2330,8 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pendi
         frame = v.sc->refresh_frame;
         ev = v.sc->refresh_ev;
     }
+    __shared__ RefreshTile<C> t;
+    constexpr int LW = RefreshTile<C>::LW, LH = RefreshTile<C>::LH;
     const uint32_t N = (uint32_t)v.N;
     const uint32_t nref = frac < 1.0f ? (uint32_t)(frac * (float)N) : N;
     uint32_t start = 0;
@@ -2318,87 +2340,129 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pendi
         draw4(v.seed_lo, v.seed_hi, v.stream_id, frame, PH_REFRESH, ev, 0xFFFFFFFFu, 0, d);
         start = d[0] % N;
     }
-    for (uint32_t p = bid * TPB + threadIdx.x; p < v.npx; p += nblk * TPB)
-        refresh_pixel<C, ALGO>(v, p, use_pending, force_fg, frame, ev, nref, start);
-}
-
-template <int C, int ALGO>
-LV_D void refresh_pixel(const View& v, uint32_t p, int use_pending, int force_fg, uint32_t frame, uint32_t ev,
-                        uint32_t nref, uint32_t start) {
-    if (use_pending && ALGO == kSuBSENSE) G(v.T)[p] = 1.0f;
-    if (!G(v.roi)[p]) return;
-    if (!(force_fg || !G(v.last_fg)[p])) return;
-    const uint32_t N = (uint32_t)v.N;
-    const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
-    uint32_t d[4];
-    for (uint32_t j = 0; j < nref; ++j) {
-        if ((j & 3u) == 0) draw4(v.seed_lo, v.seed_hi, v.stream_id, frame, PH_REFRESH, ev, p, j >> 2, d);
-        int sx, sy;
-        sample_pos_7x7(d[j & 3u], x, y, v.W, v.H, sx, sy);
-        const uint32_t sp = (uint32_t)(sy * v.W + sx);
-        if (!(force_fg || !G(v.last_fg)[sp])) continue;
-        uint32_t col[C], desc[C];
+    for (uint32_t i = threadIdx.x; i < 512u; i += TPB) {
+        int ox, oy;
+        sample_offset_7x7(i, ox, oy);
+        t.pos[i] = (uint8_t)((ox + 3) | ((oy + 3) << 4));
+    }
+    const uint32_t ntx = (uint32_t)((v.W + TW - 1) / TW), ntiles = ntx * (uint32_t)((v.H + TH - 1) / TH);
+    for (uint32_t tile = bid; tile < ntiles; tile += nblk) {
+        const int x0 = (int)(tile % ntx) * TW, y0 = (int)(tile / ntx) * TH;
+        __syncthreads();  // the previous tile's readers are done
+        for (int i = threadIdx.x; i < LW * LH; i += TPB) {
+            const int gx = x0 - 3 + i % LW, gy = y0 - 3 + i / LW;
+            t.ok[i] = 0;
+            if (gx < 2 || gy < 2 || gx >= v.W - 2 || gy >= v.H - 2) continue;  // positions are clamped inside
+            const size_t q = (size_t)gy * v.W + gx;
+            uint32_t col[C], desc[C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            col[c] = G(v.last_color)[(size_t)sp * C + c];
-            if constexpr (ALGO == kLOBSTER) {
-                uint32_t taps[4];
-                taps_from_global<C>(v.last_color, v.W, sx, sy, c, taps);
-                desc[c] = lbsp_threshold_sad(taps, col[c], v.sc->lut[col[c]]);
-            } else {
-                desc[c] = G(v.last_desc)[(size_t)sp * C + c];
+            for (int c = 0; c < C; ++c) {
+                col[c] = G(v.last_color)[q * C + c];
+                if constexpr (ALGO == kLOBSTER) {
+                    uint32_t taps[4];
+                    taps_from_global<C>(v.last_color, v.W, gx, gy, c, taps);
+                    desc[c] = lbsp_threshold_sad(taps, col[c], G(v.sc->lut)[col[c]]);
+                } else {
+                    desc[c] = G(v.last_desc)[q * C + c];
+                }
             }
+            uint64_t ra;
+            uint32_t rb;
+            encode_raw<C>(col, desc, ra, rb);
+            t.w0[i] = (uint32_t)ra;
+            if constexpr (C == 3) {
+                t.w1[i] = (uint32_t)(ra >> 32);
+                t.w2[i] = rb;
+            }
+            t.ok[i] = force_fg || !G(v.last_fg)[q];
         }
-        store_sample<C>(v, (start + j) % N, p, col, desc);
+        __syncthreads();
+        const int x = x0 + (int)threadIdx.x % TW, y = y0 + (int)threadIdx.x / TW;
+        if (x >= v.W || y >= v.H) continue;
+        const uint32_t p = (uint32_t)(y * v.W + x);
+        if (use_pending && ALGO == kSuBSENSE) G(v.T)[p] = 1.0f;
+        const bool in = G(v.roi)[p] != 0 && (force_fg || !G(v.last_fg)[p]);
+        const bool zero = outside && !G(v.roi)[p];
+        if (!in && !zero) continue;
+        uint32_t d[4], slot = start;
+        for (uint32_t j = 0; j < nref; ++j) {
+            if ((j & 3u) == 0) draw4(v.seed_lo, v.seed_hi, v.stream_id, frame, PH_REFRESH, ev, p, j >> 2, d);
+            const uint32_t o = t.pos[d[j & 3u] & 511u];
+            int sx = x + (int)(o & 15u) - 3, sy = y + (int)(o >> 4) - 3;
+            clamp_coords(sx, sy, 2, v.W, v.H);
+            const int li = in ? (sy - y0 + 3) * LW + (sx - x0 + 3) : 0;
+            if (zero || t.ok[li]) {
+                uint64_t ra = t.w0[li];
+                uint32_t rb = 0;
+                if constexpr (C == 3) {
+                    ra |= (uint64_t)t.w1[li] << 32;
+                    rb = t.w2[li];
+                }
+                store_raw<C>(v, slot, p, zero ? 0ull : ra, zero ? 0u : rb);
+            }
+            slot = slot + 1u == N ? 0u : slot + 1u;
+        }
     }
 }
 
 // initial descriptors of the LBSP base (LBS:31-63): strict bounds x>2 && y>2 && x<W-2 && y<H-2
 template <int C>
-__global__ void __launch_bounds__(TPB) k_init_desc(View v, const uint8_t* __restrict__ img) {
-    const uint32_t p = blockIdx.x * TPB + threadIdx.x;
-    if (p >= v.npx) return;
-    const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
-    const bool in = G(v.roi)[p] && x > 2 && y > 2 && x < v.W - 2 && y < v.H - 2;
+LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
+    __shared__ FrameTile<C> tile;
+    __shared__ uint8_t lut[256];
+    const int ntx = (v.W + TW - 1) / TW;
+    const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
+    load_frame_tile<C>(tile, img, v.W, v.H, x0, y0);
+    load_lut(lut, v.sc);
+    __syncthreads();
+    const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
+    if (x >= v.W || y >= v.H) return;
+    const uint32_t p = (uint32_t)(y * v.W + x);
+    const bool roi = G(v.roi)[p] != 0, in = roi && x > 2 && y > 2 && x < v.W - 2 && y < v.H - 2;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        uint16_t d = 0;
-        if (in) {
-            uint32_t taps[4];
-            taps_from_global<C>(img, v.W, x, y, c, taps);
-            const uint32_t ref = img[(size_t)p * C + c];
-            d = (uint16_t)lbsp_threshold_sad(taps, ref, v.sc->lut[ref]);
-        }
-        G(v.last_desc)[(size_t)p * C + c] = d;
-        G(v.last_color)[(size_t)p * C + c] = G(v.roi)[p] ? img[(size_t)p * C + c] : (uint8_t)0;
+        uint32_t taps[4];
+        taps_from_tile<C>(tile, lx, ly, c, taps);
+        const uint32_t ref = tile.px[((ly + 2) * FrameTile<C>::LW + (lx + 2)) * C + c];
+        G(v.last_desc)[(size_t)p * C + c] = (uint16_t)(in ? lbsp_threshold_sad(taps, ref, lut[ref]) : 0u);
+        G(v.last_color)[(size_t)p * C + c] = (uint8_t)(roi ? ref : 0u);
     }
 }
 
 // getBackgroundImage / getBackgroundDescriptorsImage (SUB:614-649): float sum of v/N in sample
-// order, then saturate_cast (round half to even)
-template <int C>
-__global__ void __launch_bounds__(TPB) k_background(View v, uint8_t* __restrict__ out_img, uint16_t* __restrict__ out_desc) {
-    const uint32_t p = blockIdx.x * TPB + threadIdx.x;
+// order, then saturate_cast (round half to even). v/N is the IEEE quotient, from the correctly rounded
+// reciprocal with one residual correction (equal to the division for every v < 2^16 and N <= 255:
+// checked exhaustively), three operations where the division takes about ten.
+LV_HD float quot(float v, float n, float inv) {
+    const float q = v * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q, n, v), inv, q);
+}
+template <int C, bool DESC>
+LV_D void background_body(const View& v, void* out, uint32_t bid) {
+    const uint32_t p = bid * TPB + threadIdx.x;
     if (p >= v.npx) return;
-    float ac[C], ad[C];
+    float acc[C];
 #pragma unroll
-    for (int c = 0; c < C; ++c) ac[c] = ad[c] = 0.0f;
-    const float fN = (float)v.N;
-    for (int s = 0; s < v.N; ++s) {
+    for (int c = 0; c < C; ++c) acc[c] = 0.0f;
+    const float fN = (float)v.N, inv = 1.0f / fN;
+    const uint32_t* rec = rec_base(v, p);
+#pragma unroll 5
+    for (int s = 0; s < v.N; ++s, rec += kSampleStride<C>) {
+        uint64_t ra;
+        uint32_t rb;
+        fetch_at<C>(rec, ra, rb);
         uint32_t col[C], desc[C];
-        load_sample<C>(v, (uint32_t)s, p, col, desc);
+        decode_raw<C>(ra, rb, col, desc);
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            ac[c] += (float)col[c] / fN;
-            ad[c] += (float)desc[c] / fN;
-        }
+        for (int c = 0; c < C; ++c) acc[c] += quot((float)(DESC ? desc[c] : col[c]), fN, inv);
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        if (out_img) out_img[(size_t)p * C + c] = sat_u8(ac[c]);
-        if (out_desc) {
-            const float r = rintf(ad[c]);
-            out_desc[(size_t)p * C + c] = (uint16_t)(r < 0.f ? 0.f : r > 65535.f ? 65535.f : r);
+        if constexpr (DESC) {
+            const float r = rintf(acc[c]);
+            ((uint16_t*)out)[(size_t)p * C + c] = (uint16_t)(r < 0.f ? 0.f : r > 65535.f ? 65535.f : r);
+        } else {
+            ((uint8_t*)out)[(size_t)p * C + c] = sat_u8(acc[c]);
         }
     }
 }
@@ -2512,9 +2576,15 @@ __global__ void __launch_bounds__(256) k_decide(View v) { decide_body(v, 0u, 1u)
 __global__ void __launch_bounds__(64) k_lobster_end(View v) { lobster_end_body(v, 0u, 1u); }
 template <int C, int ALGO>
 __global__ void __launch_bounds__(TPB) k_refresh(View v, int use_pending, float frac, int force_fg, uint32_t frame,
-                                               uint32_t ev) {
-    refresh_body<C, ALGO>(v, LV_SINGLE_BID, use_pending, frac, force_fg, frame, ev);
+                                               uint32_t ev, int outside) {
+    refresh_body<C, ALGO>(v, LV_SINGLE_BID, use_pending, frac, force_fg, frame, ev, outside);
 }
+template <int C>
+__global__ void __launch_bounds__(TPB) k_init_desc(View v, const uint8_t* img) {
+    init_desc_body<C>(v, img, (uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x));
+}
+template <int C, bool DESC>
+__global__ void __launch_bounds__(TPB) k_background(View v, void* out) { background_body<C, DESC>(v, out, blockIdx.x); }
 
 // batched entry points (SuBSENSE; streams of 1 and 3 channels may be mixed)
 #define LV_BATCH_C(body, ...)                                                                \
@@ -2553,8 +2623,8 @@ __global__ void __launch_bounds__(TPB) kb_downsample(BatchArgs b) { LV_BATCH_C(d
 __global__ void __launch_bounds__(256) kb_decide(BatchArgs b) { for_batch_block(b, decide_body); }
 __global__ void __launch_bounds__(TPB) kb_refresh(BatchArgs b) {
     for_batch_block(b, [&](const View& v, uint32_t bid, uint32_t nblk) {
-        if (v.C == 3) refresh_body<3, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u);
-        else refresh_body<1, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u);
+        if (v.C == 3) refresh_body<3, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u, 0);
+        else refresh_body<1, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u, 0);
     });
 }
 
@@ -2579,7 +2649,7 @@ void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]) 
     g[kGridFix] = opt.fixpoint_blocks > 0 ? (uint32_t)opt.fixpoint_blocks
                                           : std::max(32u, std::min(1024u, cdiv(v.npx, 1024)));
     if (opt.fix_px_per_block > 0) g[kGridFix] = std::min(g[kGridFix], cdiv(v.npx, (size_t)opt.fix_px_per_block));
-    g[kGridSweep] = std::min(cdiv(v.npx, TPB), 128u);
+    g[kGridSweep] = std::min(g[kGridTile], 128u);
     // single stream: a block per 256 pixels, at most what covers group_limit entries in one round
     g[kGridCont] = opt.cont_blocks > 0 ? (uint32_t)opt.cont_blocks
                                        : std::max(64u, std::min(kGroupLimit / (TPB / kGroup), cdiv(v.npx, TPB)));
@@ -2616,7 +2686,7 @@ static void frame_step_t(const View& v, const StepOptions& opt, hipStream_t st) 
         hipLaunchKernelGGL(k_dilate_final, dim3(g[kGridPost]), dim3(TPB), 0, st, v);
         if (g[kGridCell]) hipLaunchKernelGGL((k_downsample<C>), dim3(g[kGridCell]), dim3(TPB), 0, st, v);
         hipLaunchKernelGGL(k_decide, dim3(1), dim3(256), 0, st, v);
-        hipLaunchKernelGGL((k_refresh<C, ALGO>), dim3(g[kGridSweep]), dim3(TPB), 0, st, v, 1, 0.f, 0, 0u, 0u);
+        hipLaunchKernelGGL((k_refresh<C, ALGO>), dim3(g[kGridSweep]), dim3(TPB), 0, st, v, 1, 0.f, 0, 0u, 0u, 0);
     } else {
         hipLaunchKernelGGL(k_lobster_raw, dim3(g[kGridPix]), dim3(TPB), 0, st, v);
         if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
@@ -2671,27 +2741,32 @@ void batch_step(const View* d_views, int ns, const uint32_t* const prefix[kNumGr
     if (opt.timed_stage == 2) (void)hipEventRecord(opt.ev_end, st);
 }
 
-void launch_refresh(const View& v, float frac, int force_fg, uint32_t frame, uint32_t ev, hipStream_t st) {
-    const unsigned b = cdiv(v.npx, TPB);
+void launch_refresh(const View& v, float frac, int force_fg, uint32_t frame, uint32_t ev, int outside, hipStream_t st) {
+    const dim3 g(cdiv(v.W, TW) * cdiv(v.H, TH)), t(TPB);
     if (v.algo == kSuBSENSE) {
-        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kSuBSENSE>), dim3(b), dim3(TPB), 0, st, v, 0, frac, force_fg, frame, ev);
-        else hipLaunchKernelGGL((k_refresh<1, kSuBSENSE>), dim3(b), dim3(TPB), 0, st, v, 0, frac, force_fg, frame, ev);
+        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kSuBSENSE>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
+        else hipLaunchKernelGGL((k_refresh<1, kSuBSENSE>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
     } else {
-        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kLOBSTER>), dim3(b), dim3(TPB), 0, st, v, 0, frac, force_fg, frame, ev);
-        else hipLaunchKernelGGL((k_refresh<1, kLOBSTER>), dim3(b), dim3(TPB), 0, st, v, 0, frac, force_fg, frame, ev);
+        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kLOBSTER>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
+        else hipLaunchKernelGGL((k_refresh<1, kLOBSTER>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
     }
 }
 
 void launch_init_desc(const View& v, const uint8_t* img, hipStream_t st) {
-    const unsigned b = cdiv(v.npx, TPB);
+    const unsigned b = cdiv(v.W, TW) * cdiv(v.H, TH);
     if (v.C == 3) hipLaunchKernelGGL(k_init_desc<3>, dim3(b), dim3(TPB), 0, st, v, img);
     else hipLaunchKernelGGL(k_init_desc<1>, dim3(b), dim3(TPB), 0, st, v, img);
 }
 
-void launch_background(const View& v, uint8_t* out_img, uint16_t* out_desc, hipStream_t st) {
+void launch_background(const View& v, uint8_t* out_img, hipStream_t st) {
     const unsigned b = cdiv(v.npx, TPB);
-    if (v.C == 3) hipLaunchKernelGGL(k_background<3>, dim3(b), dim3(TPB), 0, st, v, out_img, out_desc);
-    else hipLaunchKernelGGL(k_background<1>, dim3(b), dim3(TPB), 0, st, v, out_img, out_desc);
+    if (v.C == 3) hipLaunchKernelGGL((k_background<3, false>), dim3(b), dim3(TPB), 0, st, v, (void*)out_img);
+    else hipLaunchKernelGGL((k_background<1, false>), dim3(b), dim3(TPB), 0, st, v, (void*)out_img);
+}
+void launch_background_desc(const View& v, uint16_t* out_desc, hipStream_t st) {
+    const unsigned b = cdiv(v.npx, TPB);
+    if (v.C == 3) hipLaunchKernelGGL((k_background<3, true>), dim3(b), dim3(TPB), 0, st, v, (void*)out_desc);
+    else hipLaunchKernelGGL((k_background<1, true>), dim3(b), dim3(TPB), 0, st, v, (void*)out_desc);
 }
 
 void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st) {

@@ -54,9 +54,11 @@ void frame_step(const View& v, const StepOptions& opt, hipStream_t st);
 // one SuBSENSE step of every stream of a batch (see bgs_kernels.hip)
 void batch_step(const View* d_views, int ns, const uint32_t* const prefix[kNumGrids], const uint32_t total[kNumGrids],
                 const StepOptions& opt, hipStream_t st);
-void launch_refresh(const View& v, float frac, int force_fg, uint32_t frame, uint32_t ev, hipStream_t st);
+// outside: also write zero samples for the pixels outside the ROI
+void launch_refresh(const View& v, float frac, int force_fg, uint32_t frame, uint32_t ev, int outside, hipStream_t st);
 void launch_init_desc(const View& v, const uint8_t* img, hipStream_t st);
-void launch_background(const View& v, uint8_t* out_img, uint16_t* out_desc, hipStream_t st);
+void launch_background(const View& v, uint8_t* out_img, hipStream_t st);
+void launch_background_desc(const View& v, uint16_t* out_desc, hipStream_t st);
 void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st);
 void launch_postprocess_probe(const View& v, hipStream_t st);
 // out[i] = the sticky error bits (Scalars::err_flags) of d_views[i], i < n

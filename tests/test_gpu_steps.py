@@ -79,3 +79,31 @@ def test_validate_roi_border(w, h):
     want = np.zeros((h, w), np.uint8)
     want[2:max(2, h - 2), 2:max(2, w - 2)] = 255
     assert np.array_equal(roi, want)
+
+
+@pytest.mark.parametrize("algo,c,w,h", [(SUBSENSE, 3, 131, 70), (SUBSENSE, 1, 64, 48), (LOBSTER, 3, 70, 67),
+                                        (LOBSTER, 1, 129, 5)])
+def test_reinitialize_over_an_old_model(algo, c, w, h):
+    # the arena is reused and its samples are not cleared: a second initialize with a smaller ROI writes them
+    # all (zeros outside the ROI), and a partial refresh then keeps the foreground's
+    from test_gpu_parity import LOB_STATE, SUB_STATE, _pair
+    frames = flashing(w, h, c, 6, seed=w)
+    roi = np.zeros((h, w), np.uint8)
+    roi[3:h - 1, 9:w - 20] = 255
+    gpu, orc = _pair(algo)
+    for m in (gpu, orc):
+        m.initialize(frames[0])
+        for f in frames[:3]:
+            m.apply(f)
+        m.initialize(frames[3], roi)
+    names = SUB_STATE if algo == SUBSENSE else LOB_STATE
+    for name in names:
+        assert np.array_equal(gpu.state(name), orc.state(name)), name
+    assert np.array_equal(gpu.getBackgroundImage(), orc.background_image())
+    assert np.array_equal(gpu.getBackgroundDescriptorsImage(), orc.background_descriptors())
+    for k, f in enumerate(frames[3:]):
+        assert np.array_equal(gpu.apply(f), orc.apply(f))
+        gpu.refreshModel(0.3, bool(k & 1))
+        orc.refresh_model(0.3, bool(k & 1))
+    for name in names:
+        assert np.array_equal(gpu.state(name), orc.state(name)), name
