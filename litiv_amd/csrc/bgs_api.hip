@@ -190,7 +190,7 @@ static void carve(lvbgs_ctx* c, Arena& ar) {
     float** maps[] = {&v.T, &v.R, &v.V, &v.MLD, &v.DminLT, &v.DminST, &v.RawLT, &v.RawST, &v.FinLT, &v.FinST};
     for (auto m : maps) *m = sub ? ar.take<float>(npx) : nullptr;
     uint8_t** u8s[] = {&v.unstable, &v.blinks, &v.last_raw, &v.last_raw_blink, &v.last_fg, &v.last_dil_inv,
-                       &v.raw, &v.dec};
+                       &v.dec};
     for (auto m : u8s) *m = ar.take<uint8_t>(npx);
     const size_t nz = (size_t)((c->W + 63) / 64) * (size_t)((c->H + 63) / 64);
     v.zbits = ar.take<uint64_t>(nz * 64);
@@ -760,7 +760,7 @@ extern "C" long long lvbgs_get_state(lvbgs_ctx* c, const char* name, void* out, 
                           {"blinks", v.blinks, npx},               {"last_raw", v.last_raw, npx},
                           {"last_raw_blink", v.last_raw_blink, npx}, {"last_dil_inv", v.last_dil_inv, npx},
                           {"dsLT", v.dsLT, nds},                   {"dsST", v.dsST, nds},
-                          {"raw", v.raw, npx},                     {"dec", v.dec, npx},
+                          {"raw", v.last_raw, npx},                {"dec", v.dec, npx},
                           {"mres", v.mres, npx * 4},               {"rec", v.rec, npx * 4},
                           {"desc_cur", v.desc_cur, npx * C * 2}};
     for (const auto& it : items)
@@ -928,9 +928,9 @@ extern "C" int lvbgs_debug_postprocess(lvbgs_ctx* c, const uint8_t* host_raw, ui
     if (!c->initialized) return set_err(c, LVBGS_ERR_STATE, "algo & model must be initialized first");
     if (c->algo != LVBGS_SUBSENSE) return set_err(c, LVBGS_ERR_ARG, "post-processing check is for SuBSENSE");
     (void)hipSetDevice(c->device);
-    int rc = hip_check(c, hipMemcpyAsync(c->v.raw, host_raw, c->npx, hipMemcpyHostToDevice, c->stream), "raw copy");
+    int rc = hip_check(c, hipMemcpyAsync(c->d_mask, host_raw, c->npx, hipMemcpyHostToDevice, c->stream), "raw copy");
     if (rc) return rc;
-    launch_postprocess_probe(c->v, c->stream);
+    launch_postprocess_probe(c->v, c->d_mask, c->stream);
     rc = hip_check(c, hipMemcpyAsync(host_last_fg, c->v.last_fg, c->npx, hipMemcpyDeviceToHost, c->stream), "mask copy");
     if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "sync");
     return rc;

@@ -193,6 +193,7 @@ struct alignas(128) Scalars {
     uint32_t iters;              // per-frame: fix-point iterations that had work
     uint32_t max_iter_seen;      // largest fix-point iteration index that had work (sticky)
     uint32_t epoch;              // steps since allocation (kept in checkpoints)
+    uint32_t fix_done;           // blocks of the last fix-point launch that are done (zero between launches)
     uint32_t wl_work[8];         // per-frame: worklist size of fix-point iterations 1..7
     uint8_t lut[256];            // LBSP threshold LUT (m_anLBSPThreshold_8bitLUT)
     // per-frame: pixels handed to the match continuation, stripe k at cont_cnt[k * kContStride]

@@ -850,22 +850,27 @@ LV_D int pred_dy(uint32_t i) { return (int)(i / 5u) - 2; }
 
 // Writers of p applied by the match: bit i of the result is set when predecessor i targets p with an
 // open forward gate and its decision is background (CURRENT: the decisions of the fix point, else those of
-// the previous frame). slot = the sample slot lane i's predecessor writes. Every lane of the wavefront calls.
+// the previous frame). slot = the sample slot lane i's predecessor writes; turned (CURRENT) = the group
+// has a candidate writer of a slot below `below` whose decision is not the guessed one. Every lane of the
+// wavefront calls.
 template <bool CURRENT>
-LV_D uint32_t group_writers(const View& v, int x, int y, bool active, uint32_t& slot) {
+LV_D uint32_t group_writers(const View& v, int x, int y, bool active, uint32_t& slot, uint32_t below, bool& turned) {
     const int lane = (int)(threadIdx.x & 63u), gbase = lane & ~(kGroup - 1);
     const uint32_t sub = (uint32_t)(lane & (kGroup - 1));
-    bool on = false;
+    bool on = false, other = false;
     slot = 0;
     if (active && sub < 12u) {
         const int dx = pred_dx(sub), dy = pred_dy(sub);
         const uint32_t q = (uint32_t)((y + dy) * v.W + (x + dx));
         const uint32_t r = G(v.rec)[q];
-        const uint8_t d = CURRENT ? __hip_atomic_load(&v.dec[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                  : G(v.last_raw)[q];
-        on = rec_tgt(r) == (uint32_t)((2 - dy) * 5 + (2 - dx)) && fwd_gate(r) && d == 0;
+        const uint8_t guess = G(v.last_raw)[q];
+        const uint8_t d = CURRENT ? __hip_atomic_load(&v.dec[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : guess;
+        const bool writer = rec_tgt(r) == (uint32_t)((2 - dy) * 5 + (2 - dx)) && fwd_gate(r);
         slot = rec_slot_diff(r);
+        on = writer && d == 0;
+        other = writer && (d == 0) != (guess == 0) && slot < below;
     }
+    if constexpr (CURRENT) turned = ((uint32_t)(__ballot(other) >> gbase) & 0xFFFu) != 0u;
     return (uint32_t)(__ballot(on) >> gbase) & 0xFFFu;
 }
 
@@ -1251,7 +1256,8 @@ LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_
             st = unpack_state(G(v.mres)[p]);
         }
         uint32_t slot;
-        const uint32_t applied = group_writers<false>(v, x, y, active, slot);
+        bool turned;
+        const uint32_t applied = group_writers<false>(v, x, y, active, slot, 0u, turned);
         const uint32_t s0 = st.s;
         scan_group<C, ALGO>(v, frame, lut, px, x, y, applied, slot, st, active);
         bool push = false;
@@ -1295,69 +1301,48 @@ LV_D uint32_t wl_total(const View& v, uint32_t k, uint32_t* pre) {
     return pre[kContStripes];
 }
 
-// fix-point re-match of a wavefront's worklisted pixels i0 .. i0 + 64/kGroup - 1, one group each
+// result of a fix-point re-match; true when the decision changed and the pixel has a forward target
+LV_D bool rematch_done(const View& v, uint32_t p, int x, int y, const ScanState& st, uint32_t& t) {
+    G(v.mres)[p] = pack_state(st);
+    const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
+    if (fg == G(v.dec)[p]) return false;
+    __hip_atomic_store(&v.dec[p], fg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return forward_target(v, G(v.rec)[p], x, y, t);
+}
+
+// Fix-point re-match of a wavefront's worklisted pixels i0 .. i0 + 64/kGroup - 1, one group each. In iteration 1
+// a pixel whose wrongly guessed writers all write slots that its speculative scan never reached keeps its
+// result (a background pixel examines 2 to 5 of 50 samples, so nine in ten do): only the records and decisions
+// around it are read. A writer that turns later pushes the pixel again, and later iterations match in full.
 template <int C, int ALGO>
 LV_D void rematch(const View& v, const uint8_t* lut, GroupLds& L, const uint32_t* pre, uint32_t n, uint32_t i0,
                   uint32_t k, uint32_t* wl_next) {
     const uint8_t* frame = v.frame;
     const uint32_t lane = threadIdx.x & 63u, i = i0 + lane / kGroup;
-    const bool active = i < n;
+    bool active = i < n;
     const uint32_t p = active ? wl_item(v, k, pre, i) : 0u;
     const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
+    // samples its result rests on; 0 = not matched yet
+    const uint32_t seen = active && k == 1u ? G(v.mres)[p] >> 24 : 0u;
     uint32_t slot;
-    const uint32_t applied = group_writers<true>(v, x, y, active, slot);
+    bool turned;
+    const uint32_t applied = group_writers<true>(v, x, y, active, slot, seen, turned);
+    active = active && (seen == 0u || turned);
+    if (__ballot(active) == 0ull) return;
     PxCtx<C> px{};
     group_ctx<C, ALGO>(v, frame, x, y, active, L, px);
     ScanState st = scan_init<C>();
     scan_group<C, ALGO>(v, frame, lut, px, x, y, applied, slot, st, active);
     bool push = false;
     uint32_t t = 0;
-    if (active && lane % kGroup == 0) {
-        G(v.mres)[p] = pack_state(st);
-        const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
-        const uint8_t old = G(v.dec)[p];
-        if (fg != old) {
-            __hip_atomic_store(&v.dec[p], fg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            push = forward_target(v, G(v.rec)[p], x, y, t);
-        }
-    }
+    if (active && lane % kGroup == 0) push = rematch_done(v, p, x, y, st, t);
     push_next(v, push, t, k + 1u, wl_next);
 }
 
-// fix-point iteration k (k >= 1): worklist k -> worklist k+1
+// fix-point iterations from k0 on in one workgroup (normally no work is left)
 template <int C, int ALGO>
-LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k) {
-    __shared__ uint8_t lut[256];
-    __shared__ GroupLds L;
-    __shared__ uint32_t s_pre[kContStripes + 1];
-    // slot k+2 was last read by iteration k-2 (finished); it must be empty before iteration k+1
-    // pushes into it, whether or not this iteration has work.
-    if (bid == 0 && threadIdx.x == 0)
-        __hip_atomic_store(&v.sc->wl_count[(k + 2) % kWlRing], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t n = wl_total(v, k, s_pre);
-    if (n == 0) return;
-    if (bid == 0 && threadIdx.x == 0) {
-        atomicAdd(&v.sc->iters, 1u);
-        atomicMax(&v.sc->max_iter_seen, k);
-        if (k < 8) v.sc->wl_work[k] = n;
-    }
-    if (bid * (TPB / kGroup) >= n) return;  // uniform: no item reaches this block
-    load_lut(lut, v.sc);
-    __syncthreads();
-    uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
-    const uint32_t step = nblk * (TPB / kGroup);
-    for (uint32_t i0 = (bid * TPB + (threadIdx.x & ~63u)) / kGroup; i0 < n; i0 += step)
-        rematch<C, ALGO>(v, lut, L, s_pre, n, i0, k, wl_next);
-}
-
-// remaining fix-point iterations in one workgroup (normally no work is left)
-template <int C, int ALGO>
-LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k0, uint32_t cap) {
-    __shared__ uint8_t lut[256];
-    __shared__ GroupLds L;
-    __shared__ uint32_t s_pre[kContStripes + 1];
+LV_D void fixpoint_tail(const View& v, const uint8_t* lut, GroupLds& L, uint32_t* s_pre, uint32_t k0, uint32_t cap) {
     __shared__ uint32_t s_n;
-    load_lut(lut, v.sc);
     for (uint32_t k = k0;; ++k) {
         __syncthreads();
         const uint32_t total = wl_total(v, k, s_pre);
@@ -1371,8 +1356,8 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
                 } else {
                     __hip_atomic_store(&v.sc->wl_count[(k + 2) % kWlRing], 0u, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
-                    v.sc->iters += 1u;
-                    v.sc->max_iter_seen = k > v.sc->max_iter_seen ? k : v.sc->max_iter_seen;
+                    atomicAdd(&v.sc->iters, 1u);
+                    atomicMax(&v.sc->max_iter_seen, k);
                     if (k < 8) v.sc->wl_work[k] = s_n;
                 }
             }
@@ -1384,6 +1369,53 @@ LV_D void fixpoint_tail_body(const View& v, uint32_t bid, uint32_t nblk, uint32_
         for (uint32_t i0 = (threadIdx.x & ~63u) / kGroup; i0 < n; i0 += TPB / kGroup)
             rematch<C, ALGO>(v, lut, L, s_pre, n, i0, k, wl_next);
         __threadfence();
+    }
+}
+
+// Fix-point iteration k: worklist k -> worklist k+1 (k >= 1). LAST: the block that finishes last goes on with
+// the iterations left (fixpoint_tail): blocks with work count themselves when done, behind a
+// device-scope fence; nobody waits for another block. Batches end with a launch of one block per
+// stream instead (TAIL): there the fences of thousands of blocks cost more (151 us) than the launch (20 us).
+enum FixKind : int { kFixMore, kFixLast, kFixTail };
+template <int C, int ALGO, int KIND>
+LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k, uint32_t cap) {
+    __shared__ uint8_t lut[256];
+    __shared__ GroupLds L;
+    __shared__ uint32_t s_pre[kContStripes + 1];
+    if constexpr (KIND == kFixTail) {
+        load_lut(lut, v.sc);
+        fixpoint_tail<C, ALGO>(v, lut, L, s_pre, k, cap);
+    } else {
+        // slot k+2 was last read by iteration k-2 (finished); it must be empty before iteration k+1
+        // pushes into it, whether or not this iteration has work.
+        if (bid == 0 && threadIdx.x == 0)
+            __hip_atomic_store(&v.sc->wl_count[(k + 2) % kWlRing], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t n = wl_total(v, k, s_pre);
+        if (n == 0) return;
+        if (bid == 0 && threadIdx.x == 0) {
+            atomicAdd(&v.sc->iters, 1u);
+            atomicMax(&v.sc->max_iter_seen, k);
+            if (k < 8) v.sc->wl_work[k] = n;
+        }
+        constexpr uint32_t kPerBlock = TPB / kGroup;
+        if (bid * kPerBlock >= n) return;  // uniform: no item reaches this block
+        load_lut(lut, v.sc);
+        __syncthreads();
+        uint32_t* wl_next = (k & 1u) ? v.wl0 : v.wl1;
+        for (uint32_t i0 = (bid * TPB + (threadIdx.x & ~63u)) / kGroup; i0 < n; i0 += nblk * kPerBlock)
+            rematch<C, ALGO>(v, lut, L, s_pre, n, i0, k, wl_next);
+        if constexpr (KIND == kFixLast) {
+            __shared__ uint32_t s_done;
+            const uint32_t blocks = (n + kPerBlock - 1) / kPerBlock, nwork = blocks < nblk ? blocks : nblk;
+            __threadfence();
+            __syncthreads();
+            // the counter wraps back to zero with the last block
+            if (threadIdx.x == 0) s_done = atomicInc(&v.sc->fix_done, nwork - 1u);
+            __syncthreads();
+            if (s_done != nwork - 1u) return;
+            __threadfence();
+            fixpoint_tail<C, ALGO>(v, lut, L, s_pre, k + 1u, cap);
+        }
     }
 }
 
@@ -1487,34 +1519,18 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, float& rst_out, float& m
     const uint8_t cb = raw ^ G(v.last_raw)[p];
     G(v.blinks)[p] = cb | G(v.last_raw_blink)[p];
     G(v.last_raw_blink)[p] = cb;
-    G(v.last_raw)[p] = raw;
-    G(v.raw)[p] = raw;
+    G(v.last_raw)[p] = raw;  // this frame's raw mask from here on
     return examined;
-}
-
-// LOBSTER: raw mask (LOB:496-497, :554-555) and previous-raw bookkeeping for the next speculation
-LV_D void lobster_raw_body(const View& v, uint32_t bid, uint32_t nblk) {
-    const uint32_t p = bid * TPB + threadIdx.x;
-    uint32_t examined = 0;
-    if (p < v.npx) {
-        uint8_t raw = 0;
-        if (G(v.roi)[p]) {
-            raw = G(v.dec)[p] ? 255 : 0;
-            examined = G(v.mres)[p] >> 24;
-        }
-        G(v.raw)[p] = raw;
-        G(v.last_raw)[p] = raw;
-    }
-    block_add<TPB>(examined, v.sc->ex_part);
 }
 
 // ----------------------------------------------------------------------------------------------
 // model update: every pixel of the inner rectangle gathers the writes aimed at its samples, in
 // the raster order of the writers; the last write of each slot wins (SUB:406-449, LOB:498-512).
 // ----------------------------------------------------------------------------------------------
-// FUSED (SuBSENSE): the feedback maps of the thread's pixel are updated first, in the same pass
-// (they depend on the pixel alone), and the ghost test uses the new values from registers.
-template <int C, int ALGO, bool FUSED>
+// SuBSENSE: the feedback maps of the thread's pixel are updated first, in the same pass
+// (they depend on the pixel alone), and the ghost test uses the new values from registers. LOBSTER: the raw
+// mask (LOB:496-497, :554-555) and the last colour frame (LOB:580) are written in the same pass.
+template <int C, int ALGO>
 LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
     const uint8_t* frame = v.frame;
     constexpr int LW = TW + 4, LH = TH + 4, NT = (LW * LH + TPB - 1) / TPB;
@@ -1547,7 +1563,7 @@ LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
     const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
     uint32_t nw = 0, examined = 0;
     float rst = 0.f, mld = 1.f;
-    if constexpr (FUSED)
+    if constexpr (ALGO == kSuBSENSE)
         if (x < v.W && y < v.H) examined = feedback_pixel<C>(v, (uint32_t)(y * v.W + x), rst, mld);
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
@@ -1563,12 +1579,21 @@ LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
         }
     }
     __syncthreads();
+    if constexpr (ALGO == kLOBSTER) {
+        if (x < v.W && y < v.H) {
+            const uint32_t p = (uint32_t)(y * v.W + x);
+            const bool roi = rec_tgt(s_rec[ly + 2][lx + 2]) != kRecNone;
+            G(v.last_raw)[p] = roi && !s_bg[ly + 2][lx + 2] ? 255 : 0;
+            if (roi) examined = G(v.mres)[p] >> 24;
+#pragma unroll
+            for (int c = 0; c < C; ++c) G(v.last_color)[(size_t)p * C + c] = s_col[ly + 2][(lx + 2) * C + c];
+        }
+    }
     if (x >= 2 && y >= 2 && x < v.W - 2 && y < v.H - 2) {
         const uint32_t p = (uint32_t)(y * v.W + x);
         // ghost test of writers at or after p reads p's updated maps (SUB:438-441)
         bool ghost_new = false;
-        if constexpr (FUSED) ghost_new = rst > 0.995f && mld < 0.010f;
-        else if constexpr (ALGO == kSuBSENSE) ghost_new = G(v.RawST)[p] > 0.995f && G(v.MLD)[p] < 0.010f;
+        if constexpr (ALGO == kSuBSENSE) ghost_new = rst > 0.995f && mld < 0.010f;
         // Writes landing on p, as bits in sequential order: writer j of the 5x5 window (raster
         // order) owns bit 2j (its self update, j == 12 only) and bit 2j+1 (its diffusion into p).
         uint64_t wm = 0;
@@ -1611,15 +1636,7 @@ LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
         }
     }
     block_add<TPB>(nw, v.sc->wr_part);
-    if constexpr (FUSED) block_add<TPB>(examined, v.sc->ex_part);  // workload counter (sum of k_p)
-}
-
-// LOBSTER: last colour frame := input (LOB:580)
-template <int C>
-LV_D void copy_last_color_body(const View& v, uint32_t bid, uint32_t nblk) {
-    const uint8_t* frame = v.frame;
-    const uint32_t i = bid * TPB + threadIdx.x;
-    if (i < v.npx * (uint32_t)C) G(v.last_color)[i] = G(frame)[i];
+    block_add<TPB>(examined, v.sc->ex_part);  // workload counter (sum of k_p)
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -1722,7 +1739,9 @@ LV_D void zone_close_body(const View& v, uint32_t bid, uint32_t nblk) {
     const int z = (int)bid * ZPB + wv;
     if (z >= nz) return;  // whole wavefronts only; nothing below synchronizes the block
     const int x0 = (z % nzx) * ZS, y0 = (z / nzx) * ZS;
-    const uint8_t* raw = v.raw;
+    // the raw mask is the decisions (zero outside the ROI): they are final before the model update, so
+    // this runs beside it
+    const uint8_t* raw = v.dec;
     // raw rows y0-2+r as 64-bit masks: lane = column for the loads, one ballot per row; lane y
     // keeps row y, lanes 0..3 also rows 64..67
     const int gx = x0 + lane;
@@ -1937,6 +1956,16 @@ LV_D void store_mask_word(uint8_t* m, int W, int H, int gx, int gy, uint32_t w) 
     for (int i = 0; i < 4 && gx + i < W; ++i) row[gx + i] = (uint8_t)(w >> (8 * i));
 }
 
+// the same into the caller's mask, which may have any alignment
+LV_D void store_out_word(uint8_t* m, int W, int H, int gx, int gy, uint32_t w) {
+    if (((uintptr_t)m & 3u) == 0) {
+        store_mask_word(m, W, H, gx, gy, w);
+        return;
+    }
+    if (gy >= H) return;
+    for (int i = 0; i < 4 && gx + i < W; ++i) m[(size_t)gy * (size_t)W + gx + i] = (uint8_t)(w >> (8 * i));
+}
+
 // bits (gx..gx+3, gy) of a zone bitmap (gx % 4 == 0), zero outside the image
 LV_D uint32_t zone_bits4(const uint64_t* bits, int W, int H, int gx, int gy) {
     if (gx < 0 || gy < 0 || gx >= W || gy >= H) return 0u;
@@ -2005,10 +2034,10 @@ LV_D void median_body(const View& v, uint32_t bid, uint32_t nblk) {
             uint32_t e = s_eh[ly][j];
 #pragma unroll
             for (int a = 1; a <= 2 * HE; ++a) e &= s_eh[ly + a][j];
-            m = (load_mask_word(v.raw, W, H, gx, gy, 0u) | expand4(zone_bits4(v.hbits, W, H, gx, gy)) | e) &
+            m = (load_mask_word(v.last_raw, W, H, gx, gy, 0u) | expand4(zone_bits4(v.hbits, W, H, gx, gy)) | e) &
                 in_image_bytes(W, H, gx, gy);
         } else {
-            m = load_mask_word(v.raw, W, H, gx, gy, 0u);
+            m = load_mask_word(v.last_raw, W, H, gx, gy, 0u);
         }
         s_mask[ly][j] = m & 0x01010101u;
     }
@@ -2037,19 +2066,56 @@ LV_D void median_body(const View& v, uint32_t bid, uint32_t nblk) {
         }
         const uint32_t bits = ((s + bias) >> 7) & 0x01010101u;
         store_mask_word(v.last_fg, W, H, x0 + 4 * q, y0 + ly, bits * 255u);
+        if constexpr (!SUBSENSE)
+            if (v.out_mask) store_out_word(v.out_mask, W, H, x0 + 4 * q, y0 + ly, bits * 255u);
+    }
+    if constexpr (!SUBSENSE) {
+        if (bid == 0 && threadIdx.x == 0) {  // end of the LOBSTER step
+            v.sc->frame_idx += 1u;
+            v.sc->epoch += 1u;
+        }
     }
 }
 
+// What the pixels around a tile offer to refreshModel: colour and descriptor as a sample record, and
+// whether they may be sampled. A 3-pixel halo covers getSamplePosition's 7x7 window (its clamping moves a
+// position towards the pixel). A record serves up to 50 samples of each of the 49 pixels around it, so it is
+// built once here (LOBSTER computes its descriptor) instead of per sample from global memory.
+struct RefreshTile {
+    static constexpr int LW = TW + 6, LH = TH + 6;
+    uint32_t w0[LW * LH], w1[LW * LH], w2[LW * LH];  // w0 alone with one channel
+    uint8_t ok[LW * LH];
+    uint8_t pos[512];  // sample position of each draw % 512: dx + 3 | (dy + 3) << 4
+};
+
+struct DilateTile {
+    static constexpr int H3 = 3;
+    static constexpr int FWW = (PW + 8) / 4;  // last_fg words: columns x0-4 .. x0+PW+3
+    static constexpr int LH = PH + 2 * H3;    // rows y0-3 .. y0+PH+2
+    static constexpr int OWW = PW / 4;
+    uint32_t fg[LH][FWW], h[LH][OWW];
+};
+
+// one allocation for the two kinds of block of the dilation launch, whichever channel counts it instantiates
+// (separate arrays took 16.6 KB and the dilation of a batch 220 us instead of 189)
+union SweepLds {
+    RefreshTile refresh;
+    DilateTile dilate;
+};
+LV_D SweepLds& sweep_lds() {
+    __shared__ SweepLds m;
+    return m;
+}
+
 // dilate7(last_fg), blink masks (SUB:548-551), final-segmentation averages (SUB:553-554) and the
-// output mask. addWeighted(.., CV_32F) is evaluated as the double-precision scalar form.
+// output mask. addWeighted(.., CV_32F) is evaluated as the double-precision scalar form. Runs after the
+// controller, which has advanced the frame index.
 LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
     uint8_t* out_mask = v.out_mask;
-    constexpr int H3 = 3;
-    constexpr int FWW = (PW + 8) / 4;  // last_fg words: columns x0-4 .. x0+PW+3
-    constexpr int LH = PH + 2 * H3;    // rows y0-3 .. y0+PH+2
-    constexpr int OWW = PW / 4;
-    __shared__ uint32_t s_fg[LH][FWW];
-    __shared__ uint32_t s_h[LH][OWW];
+    constexpr int H3 = DilateTile::H3, FWW = DilateTile::FWW, LH = DilateTile::LH, OWW = DilateTile::OWW;
+    DilateTile& t = sweep_lds().dilate;
+    auto& s_fg = t.fg;
+    auto& s_h = t.h;
     const int W = v.W, H = v.H;
     const int ntx = (W + PW - 1) / PW;
     const int tid = (int)bid;
@@ -2064,7 +2130,7 @@ LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
         s_h[ly][q] = dilate7_word(s_fg[ly][q], s_fg[ly][q + 1], s_fg[ly][q + 2]);
     }
     __syncthreads();
-    const uint32_t frame_no = cur_frame(v), mvn = v.mv_avgs;
+    const uint32_t frame_no = v.sc->frame_idx, mvn = v.mv_avgs;
     const float aLT = 1.0f / (float)(frame_no < mvn ? frame_no : mvn);
     const float aST = 1.0f / (float)(frame_no < mvn / 4u ? frame_no : mvn / 4u);
     const double alt = (double)(1.0f - aLT), blt = (1.0 / 255) * (double)aLT;
@@ -2115,13 +2181,6 @@ LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
             }
         }
     }
-}
-
-LV_D void copy_mask_body(const View& v, uint32_t bid, uint32_t nblk) {
-    uint8_t* out_mask = v.out_mask;
-    if (!out_mask) return;
-    const uint32_t p = bid * TPB + threadIdx.x;
-    if (p < v.npx) out_mask[p] = G(v.last_fg)[p];
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -2292,46 +2351,17 @@ LV_D void decide_body(const View& v, uint32_t bid, uint32_t nblk) {
     sc->epoch += 1u;
 }
 
-// LOBSTER end of step: frame counter and worklist epoch
-LV_D void lobster_end_body(const View& v, uint32_t bid, uint32_t nblk) {
-    if (threadIdx.x != 0) return;
-    v.sc->frame_idx += 1u;
-    v.sc->epoch += 1u;
-}
-
-// What the pixels around a tile offer to refreshModel: colour and descriptor as a sample record, and
-// whether they may be sampled. A 3-pixel halo covers getSamplePosition's 7x7 window (its clamping moves a
-// position towards the pixel). A record serves up to 50 samples of each of the 49 pixels around it, so it is
-// built once here (LOBSTER computes its descriptor) instead of per sample from global memory.
-template <int C>
-struct RefreshTile {
-    static constexpr int LW = TW + 6, LH = TH + 6;
-    uint32_t w0[LW * LH];
-    uint32_t w1[C == 3 ? LW * LH : 1], w2[C == 3 ? LW * LH : 1];
-    uint8_t ok[LW * LH];
-    uint8_t pos[512];  // sample position of each draw % 512: dx + 3 | (dy + 3) << 4
-};
-
-// refreshModel (SUB:80-105; LOB:410-440). pending = 1: auto-reset request from k_decide (also
-// T := 1 everywhere, SUB:592); otherwise an explicit call with the given parameters. outside: pixels
-// outside the ROI get zero samples (initialization writes every sample of the model, so that its memory need
-// not be cleared first). A grid-stride sweep over the tiles, so the per-step launch (normally nothing
-// pending) stays small.
+// refreshModel (SUB:80-105; LOB:410-440) over the tiles bid, bid + nblk, ... reset: the automatic reset's, which
+// also sets T := 1 everywhere (SUB:592). outside: pixels outside the ROI get zero samples
+// (initialization writes every sample of the model, so that its memory need not be cleared first).
 // Bound by the sample stores and the draws: with a table in LDS for the position (a walk of up to 48
 // entries before) and the tile's records 1305 -> 126 us (4.4 TB/s) for the 553 MB of a
 // 1280x720 RGB model.
 template <int C, int ALGO>
-LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pending, float frac, int force_fg,
-                       uint32_t frame, uint32_t ev, int outside) {
-    if (use_pending) {
-        if (!v.sc->refresh_pending) return;
-        frac = v.sc->refresh_frac;
-        force_fg = v.sc->refresh_force_fg;
-        frame = v.sc->refresh_frame;
-        ev = v.sc->refresh_ev;
-    }
-    __shared__ RefreshTile<C> t;
-    constexpr int LW = RefreshTile<C>::LW, LH = RefreshTile<C>::LH;
+LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int reset, float frac, int force_fg, uint32_t frame,
+                       uint32_t ev, int outside) {
+    RefreshTile& t = sweep_lds().refresh;
+    constexpr int LW = RefreshTile::LW, LH = RefreshTile::LH;
     const uint32_t N = (uint32_t)v.N;
     const uint32_t nref = frac < 1.0f ? (uint32_t)(frac * (float)N) : N;
     uint32_t start = 0;
@@ -2380,7 +2410,7 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pendi
         const int x = x0 + (int)threadIdx.x % TW, y = y0 + (int)threadIdx.x / TW;
         if (x >= v.W || y >= v.H) continue;
         const uint32_t p = (uint32_t)(y * v.W + x);
-        if (use_pending && ALGO == kSuBSENSE) G(v.T)[p] = 1.0f;
+        if (reset) G(v.T)[p] = 1.0f;
         const bool in = G(v.roi)[p] != 0 && (force_fg || !G(v.last_fg)[p]);
         const bool zero = outside && !G(v.roi)[p];
         if (!in && !zero) continue;
@@ -2403,6 +2433,15 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int use_pendi
             slot = slot + 1u == N ? 0u : slot + 1u;
         }
     }
+}
+
+// the automatic reset the controller asked for in this step, by the blocks of the dilation (a launch
+// of its own, or blocks of their own, cost 9 to 30 us per step of a 64-stream batch with nothing pending)
+template <int C>
+LV_D void refresh_pending(const View& v, uint32_t bid, uint32_t nblk) {
+    __syncthreads();  // the dilation's readers of the shared LDS are done
+    refresh_body<C, kSuBSENSE>(v, bid, nblk, 1, v.sc->refresh_frac, v.sc->refresh_force_fg, v.sc->refresh_frame,
+                               v.sc->refresh_ev, 0);
 }
 
 // initial descriptors of the LBSP base (LBS:31-63): strict bounds x>2 && y>2 && x<W-2 && y<H-2
@@ -2521,9 +2560,10 @@ struct BatchArgs {
     int ns;
 };
 
+// block bid of nblk of a grid
 template <class F>
-LV_D void for_batch_block(const BatchArgs& b, F&& f) {
-    const uint32_t lb = (uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x);
+LV_D void for_batch_block(const BatchArgs& b, uint32_t bid, uint32_t nblk, F&& f) {
+    const uint32_t lb = (uint32_t)xcd_tile((int)bid, (int)nblk);
     int lo = 0, hi = b.ns;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -2535,6 +2575,14 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
     f(v, lb - b.prefix[lo], b.prefix[lo + 1] - b.prefix[lo]);
 }
 
+template <class F>
+LV_D void for_batch_block(const BatchArgs& b, F&& f) {
+    for_batch_block(b, blockIdx.x, gridDim.x, f);
+}
+
+// Several kernels take two or three kinds of work in one launch: the small, latency-bound kinds in the
+// first blocks, so that they run beside the kind that fills the chip instead of before or after it with a
+// launch of their own (4 to 5 us each on an idle chip, and the zones 25 us).
 #define LV_SINGLE_BID ((uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x)), gridDim.x
 // kernels over a list that may fill only the first blocks: in dispatch order, so every XCD gets a share
 // (remapped, 700 busy blocks of 4096 would all run on two XCDs)
@@ -2551,33 +2599,47 @@ template <int C, int ALGO, int KF>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(6))) k_match_seq(View v) {
     match_seq_body<C, ALGO, KF>(v, LV_LIST_BID);
 }
-template <int C, int ALGO>
-__global__ void __launch_bounds__(TPB) k_fixpoint(View v, uint32_t k) { fixpoint_body<C, ALGO>(v, LV_LIST_BID, k); }
-template <int C, int ALGO>
-__global__ void __launch_bounds__(256) k_fixpoint_tail(View v, uint32_t k0, uint32_t cap) {
-    fixpoint_tail_body<C, ALGO>(v, 0u, 1u, k0, cap);
+template <int C, int ALGO, int KIND>
+__global__ void __launch_bounds__(TPB) k_fixpoint(View v, uint32_t k, uint32_t cap) {
+    fixpoint_body<C, ALGO, KIND>(v, LV_LIST_BID, k, cap);
 }
 
-__global__ void __launch_bounds__(TPB) k_lobster_raw(View v) { lobster_raw_body(v, LV_SINGLE_BID); }
-template <int C, int ALGO, bool FUSED>
-__global__ void __launch_bounds__(TPB) k_update(View v) { update_body<C, ALGO, FUSED>(v, LV_SINGLE_BID); }
-template <int C>
-__global__ void __launch_bounds__(TPB) k_copy_last_color(View v) { copy_last_color_body<C>(v, LV_SINGLE_BID); }
+// the zones' closing and the frame-level cells beside the model update (SuBSENSE; nzone = ncell = 0 else)
+template <int C, int ALGO>
+__global__ void __launch_bounds__(TPB) k_update(View v, uint32_t nzone, uint32_t ncell) {
+    const uint32_t b = blockIdx.x, rest = gridDim.x - nzone - ncell;
+    if constexpr (ALGO == kSuBSENSE) {
+        if (b < nzone) {
+            zone_close_body(v, b, nzone);
+            return;
+        }
+        if (b < nzone + ncell) {
+            downsample_body<C>(v, b - nzone, ncell);
+            return;
+        }
+    }
+    update_body<C, ALGO>(v, (uint32_t)xcd_tile((int)(b - nzone - ncell), (int)rest), rest);
+}
 __global__ void __launch_bounds__(TPB) k_zone_close(View v) { zone_close_body(v, LV_SINGLE_BID); }
 __global__ void __launch_bounds__(TPB) k_zone_link(View v) { zone_link_body(v, LV_SINGLE_BID); }
-__global__ void __launch_bounds__(TPB) k_zone_holes(View v) { zone_holes_body(v, LV_SINGLE_BID); }
+// the frame controller (ndecide = 1) beside the zones' holes
+__global__ void __launch_bounds__(TPB) k_zone_holes(View v, uint32_t ndecide) {
+    if (blockIdx.x < ndecide) decide_body(v, 0u, 1u);
+    else zone_holes_body(v, blockIdx.x - ndecide, gridDim.x - ndecide);
+}
 template <bool SUB>
 __global__ void __launch_bounds__(TPB) k_median(View v) { median_body<SUB>(v, LV_SINGLE_BID); }
-__global__ void __launch_bounds__(TPB) k_dilate_final(View v) { dilate_final_body(v, LV_SINGLE_BID); }
-__global__ void __launch_bounds__(TPB) k_copy_mask(View v) { copy_mask_body(v, LV_SINGLE_BID); }
 template <int C>
-__global__ void __launch_bounds__(TPB) k_downsample(View v) { downsample_body<C>(v, LV_SINGLE_BID); }
-__global__ void __launch_bounds__(256) k_decide(View v) { decide_body(v, 0u, 1u); }
-__global__ void __launch_bounds__(64) k_lobster_end(View v) { lobster_end_body(v, 0u, 1u); }
+__global__ void __launch_bounds__(TPB) k_dilate_final(View v) {
+    const uint32_t bid = (uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int pending = v.sc->refresh_pending;  // loaded before the tile, not behind its stores
+    dilate_final_body(v, bid, gridDim.x);
+    if (pending) refresh_pending<C>(v, bid, gridDim.x);
+}
 template <int C, int ALGO>
-__global__ void __launch_bounds__(TPB) k_refresh(View v, int use_pending, float frac, int force_fg, uint32_t frame,
-                                               uint32_t ev, int outside) {
-    refresh_body<C, ALGO>(v, LV_SINGLE_BID, use_pending, frac, force_fg, frame, ev, outside);
+__global__ void __launch_bounds__(TPB) k_refresh(View v, float frac, int force_fg, uint32_t frame, uint32_t ev,
+                                               int outside) {
+    refresh_body<C, ALGO>(v, LV_SINGLE_BID, 0, frac, force_fg, frame, ev, outside);
 }
 template <int C>
 __global__ void __launch_bounds__(TPB) k_init_desc(View v, const uint8_t* img) {
@@ -2601,30 +2663,44 @@ template <int KF>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(6))) kb_match_seq(BatchArgs b) {
     LV_BATCH_C(match_seq_body, kSuBSENSE, KF);
 }
-__global__ void __launch_bounds__(TPB) kb_fixpoint(BatchArgs b, uint32_t k) {
+template <int KIND>
+__global__ void __launch_bounds__(TPB) kb_fixpoint(BatchArgs b, uint32_t k, uint32_t cap) {
     for_batch_block(b, [&](const View& v, uint32_t bid, uint32_t nblk) {
-        if (v.C == 3) fixpoint_body<3, kSuBSENSE>(v, bid, nblk, k);
-        else fixpoint_body<1, kSuBSENSE>(v, bid, nblk, k);
+        if (v.C == 3) fixpoint_body<3, kSuBSENSE, KIND>(v, bid, nblk, k, cap);
+        else fixpoint_body<1, kSuBSENSE, KIND>(v, bid, nblk, k, cap);
     });
 }
-__global__ void __launch_bounds__(256) kb_fixpoint_tail(BatchArgs b, uint32_t k0, uint32_t cap) {
-    for_batch_block(b, [&](const View& v, uint32_t bid, uint32_t nblk) {
-        if (v.C == 3) fixpoint_tail_body<3, kSuBSENSE>(v, bid, nblk, k0, cap);
-        else fixpoint_tail_body<1, kSuBSENSE>(v, bid, nblk, k0, cap);
-    });
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7))) kb_update(BatchArgs zone, uint32_t nzone, BatchArgs cell, uint32_t ncell,
+                                                 BatchArgs tile) {
+    const uint32_t b = blockIdx.x;
+    if (b < nzone) {
+        for_batch_block(zone, b, nzone, zone_close_body);
+    } else if (b < nzone + ncell) {
+        for_batch_block(cell, b - nzone, ncell, [&](const View& v, uint32_t bid, uint32_t nblk) {
+            if (v.C == 3) downsample_body<3>(v, bid, nblk);
+            else downsample_body<1>(v, bid, nblk);
+        });
+    } else {
+        for_batch_block(tile, b - nzone - ncell, gridDim.x - nzone - ncell,
+                        [&](const View& v, uint32_t bid, uint32_t nblk) {
+                            if (v.C == 3) update_body<3, kSuBSENSE>(v, bid, nblk);
+                            else update_body<1, kSuBSENSE>(v, bid, nblk);
+                        });
+    }
 }
-__global__ void __launch_bounds__(TPB) kb_update(BatchArgs b) { LV_BATCH_C(update_body, kSuBSENSE, true); }
-__global__ void __launch_bounds__(TPB) kb_zone_close(BatchArgs b) { for_batch_block(b, zone_close_body); }
 __global__ void __launch_bounds__(TPB) kb_zone_link(BatchArgs b) { for_batch_block(b, zone_link_body); }
-__global__ void __launch_bounds__(TPB) kb_zone_holes(BatchArgs b) { for_batch_block(b, zone_holes_body); }
+__global__ void __launch_bounds__(TPB) kb_zone_holes(BatchArgs one, uint32_t none, BatchArgs zone) {
+    if (blockIdx.x < none) for_batch_block(one, blockIdx.x, none, decide_body);
+    else for_batch_block(zone, blockIdx.x - none, gridDim.x - none, zone_holes_body);
+}
 __global__ void __launch_bounds__(TPB) kb_median(BatchArgs b) { for_batch_block(b, median_body<true>); }
-__global__ void __launch_bounds__(TPB) kb_dilate_final(BatchArgs b) { for_batch_block(b, dilate_final_body); }
-__global__ void __launch_bounds__(TPB) kb_downsample(BatchArgs b) { LV_BATCH_C(downsample_body); }
-__global__ void __launch_bounds__(256) kb_decide(BatchArgs b) { for_batch_block(b, decide_body); }
-__global__ void __launch_bounds__(TPB) kb_refresh(BatchArgs b) {
+__global__ void __launch_bounds__(TPB) kb_dilate_final(BatchArgs b) {
     for_batch_block(b, [&](const View& v, uint32_t bid, uint32_t nblk) {
-        if (v.C == 3) refresh_body<3, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u, 0);
-        else refresh_body<1, kSuBSENSE>(v, bid, nblk, 1, 0.f, 0, 0u, 0u, 0);
+        const int pending = v.sc->refresh_pending;
+        dilate_final_body(v, bid, nblk);
+        if (!pending) return;
+        if (v.C == 3) refresh_pending<3>(v, bid, nblk);
+        else refresh_pending<1>(v, bid, nblk);
     });
 }
 
@@ -2642,14 +2718,12 @@ void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]) 
     g[kGridTile] = cdiv(v.W, TW) * cdiv(v.H, TH);
     g[kGridPost] = cdiv(v.W, PW) * cdiv(v.H, PH);
     g[kGridZone] = cdiv((size_t)cdiv(v.W, ZS) * cdiv(v.H, ZS), ZPB);
-    g[kGridPix] = cdiv(v.npx, TPB);
     g[kGridCell] = !v.lr_scaling ? 0u : cdiv((size_t)v.dsW * v.dsH, TPB);
     g[kGridOne] = 1u;
     // single stream: a block per 1024 pixels (16 groups each; the worklists hold a few per cent of them)
     g[kGridFix] = opt.fixpoint_blocks > 0 ? (uint32_t)opt.fixpoint_blocks
                                           : std::max(32u, std::min(1024u, cdiv(v.npx, 1024)));
     if (opt.fix_px_per_block > 0) g[kGridFix] = std::min(g[kGridFix], cdiv(v.npx, (size_t)opt.fix_px_per_block));
-    g[kGridSweep] = std::min(g[kGridTile], 128u);
     // single stream: a block per 256 pixels, at most what covers group_limit entries in one round
     g[kGridCont] = opt.cont_blocks > 0 ? (uint32_t)opt.cont_blocks
                                        : std::max(64u, std::min(kGroupLimit / (TPB / kGroup), cdiv(v.npx, TPB)));
@@ -2672,30 +2746,23 @@ static void frame_step_t(const View& v, const StepOptions& opt, hipStream_t st) 
     // the second iteration's worklist is about a hundredth of the first's: on small frames (a dozen entries)
     // the tail takes it (320x240 126.8 -> 124.8 us; 1920x1080 408 -> 420)
     const uint32_t launches = opt.fixpoint_launches >= 0 ? (uint32_t)opt.fixpoint_launches : v.npx < 600000u ? 1u : 2u;
-    for (uint32_t k = 1; k <= launches; ++k)
-        hipLaunchKernelGGL((k_fixpoint<C, ALGO>), dim3(g[kGridFix]), dim3(TPB), 0, st, v, k);
-    hipLaunchKernelGGL((k_fixpoint_tail<C, ALGO>), dim3(1), dim3(256), 0, st, v, launches + 1u, (uint32_t)opt.tail_cap);
-    if constexpr (ALGO == kSuBSENSE) {
-        if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
-        hipLaunchKernelGGL((k_update<C, ALGO, true>), dim3(g[kGridTile]), dim3(TPB), 0, st, v);
-        if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
-        hipLaunchKernelGGL(k_zone_close, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL(k_zone_link, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL(k_zone_holes, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
+    const uint32_t cap = (uint32_t)opt.tail_cap;
+    for (uint32_t k = 1; k < launches; ++k)
+        hipLaunchKernelGGL((k_fixpoint<C, ALGO, kFixMore>), dim3(g[kGridFix]), dim3(TPB), 0, st, v, k, cap);
+    if (launches) hipLaunchKernelGGL((k_fixpoint<C, ALGO, kFixLast>), dim3(g[kGridFix]), dim3(TPB), 0, st, v, launches, cap);
+    else hipLaunchKernelGGL((k_fixpoint<C, ALGO, kFixTail>), dim3(1), dim3(TPB), 0, st, v, 1u, cap);
+    constexpr bool kSub = ALGO == kSuBSENSE;
+    const uint32_t nzone = kSub ? g[kGridZone] : 0u, ncell = kSub ? g[kGridCell] : 0u;
+    if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
+    hipLaunchKernelGGL((k_update<C, ALGO>), dim3(nzone + ncell + g[kGridTile]), dim3(TPB), 0, st, v, nzone, ncell);
+    if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
+    if constexpr (kSub) {
+        hipLaunchKernelGGL(k_zone_link, dim3(nzone), dim3(TPB), 0, st, v);
+        hipLaunchKernelGGL(k_zone_holes, dim3(1 + nzone), dim3(TPB), 0, st, v, 1u);
         hipLaunchKernelGGL((k_median<true>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL(k_dilate_final, dim3(g[kGridPost]), dim3(TPB), 0, st, v);
-        if (g[kGridCell]) hipLaunchKernelGGL((k_downsample<C>), dim3(g[kGridCell]), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL(k_decide, dim3(1), dim3(256), 0, st, v);
-        hipLaunchKernelGGL((k_refresh<C, ALGO>), dim3(g[kGridSweep]), dim3(TPB), 0, st, v, 1, 0.f, 0, 0u, 0u, 0);
+        hipLaunchKernelGGL((k_dilate_final<C>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
     } else {
-        hipLaunchKernelGGL(k_lobster_raw, dim3(g[kGridPix]), dim3(TPB), 0, st, v);
-        if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
-        hipLaunchKernelGGL((k_update<C, ALGO, false>), dim3(g[kGridTile]), dim3(TPB), 0, st, v);
-        if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
         hipLaunchKernelGGL((k_median<false>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
-        if (v.out_mask) hipLaunchKernelGGL(k_copy_mask, dim3(g[kGridPix]), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL((k_copy_last_color<C>), dim3(cdiv((size_t)v.npx * C, TPB)), dim3(TPB), 0, st, v);
-        hipLaunchKernelGGL(k_lobster_end, dim3(1), dim3(64), 0, st, v);
     }
     if (opt.timed_stage == 2) (void)hipEventRecord(opt.ev_end, st);
 }
@@ -2723,32 +2790,30 @@ void batch_step(const View* d_views, int ns, const uint32_t* const prefix[kNumGr
     if (opt.timed_stage == 1) (void)hipEventRecord(opt.ev_end, st);
     if (opt.fetch_depth == 4) hipLaunchKernelGGL(kb_match_seq<4>, dim3(total[kGridCont]), dim3(TPB), 0, st, args(kGridCont));
     else hipLaunchKernelGGL(kb_match_seq<2>, dim3(total[kGridCont]), dim3(TPB), 0, st, args(kGridCont));
-    for (uint32_t k = 1; k <= (uint32_t)opt.fixpoint_launches; ++k)
-        hipLaunchKernelGGL(kb_fixpoint, dim3(total[kGridFix]), dim3(TPB), 0, st, args(kGridFix), k);
-    hipLaunchKernelGGL(kb_fixpoint_tail, dim3(total[kGridOne]), dim3(256), 0, st, args(kGridOne),
-                       (uint32_t)opt.fixpoint_launches + 1u, (uint32_t)opt.tail_cap);
+    const uint32_t launches = (uint32_t)opt.fixpoint_launches, cap = (uint32_t)opt.tail_cap;
+    for (uint32_t k = 1; k <= launches; ++k)
+        hipLaunchKernelGGL(kb_fixpoint<kFixMore>, dim3(total[kGridFix]), dim3(TPB), 0, st, args(kGridFix), k, cap);
+    hipLaunchKernelGGL(kb_fixpoint<kFixTail>, dim3(total[kGridOne]), dim3(TPB), 0, st, args(kGridOne), launches + 1u, cap);
+    const uint32_t nzone = total[kGridZone], ncell = total[kGridCell], none = total[kGridOne];
     if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_begin, st);
-    hipLaunchKernelGGL(kb_update, dim3(total[kGridTile]), dim3(TPB), 0, st, args(kGridTile));
+    hipLaunchKernelGGL(kb_update, dim3(nzone + ncell + total[kGridTile]), dim3(TPB), 0, st, args(kGridZone), nzone,
+                       args(kGridCell), ncell, args(kGridTile));
     if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
-    hipLaunchKernelGGL(kb_zone_close, dim3(total[kGridZone]), dim3(TPB), 0, st, args(kGridZone));
-    hipLaunchKernelGGL(kb_zone_link, dim3(total[kGridZone]), dim3(TPB), 0, st, args(kGridZone));
-    hipLaunchKernelGGL(kb_zone_holes, dim3(total[kGridZone]), dim3(TPB), 0, st, args(kGridZone));
+    hipLaunchKernelGGL(kb_zone_link, dim3(nzone), dim3(TPB), 0, st, args(kGridZone));
+    hipLaunchKernelGGL(kb_zone_holes, dim3(none + nzone), dim3(TPB), 0, st, args(kGridOne), none, args(kGridZone));
     hipLaunchKernelGGL(kb_median, dim3(total[kGridPost]), dim3(TPB), 0, st, args(kGridPost));
     hipLaunchKernelGGL(kb_dilate_final, dim3(total[kGridPost]), dim3(TPB), 0, st, args(kGridPost));
-    if (total[kGridCell]) hipLaunchKernelGGL(kb_downsample, dim3(total[kGridCell]), dim3(TPB), 0, st, args(kGridCell));
-    hipLaunchKernelGGL(kb_decide, dim3(total[kGridOne]), dim3(256), 0, st, args(kGridOne));
-    hipLaunchKernelGGL(kb_refresh, dim3(total[kGridSweep]), dim3(TPB), 0, st, args(kGridSweep));
     if (opt.timed_stage == 2) (void)hipEventRecord(opt.ev_end, st);
 }
 
 void launch_refresh(const View& v, float frac, int force_fg, uint32_t frame, uint32_t ev, int outside, hipStream_t st) {
     const dim3 g(cdiv(v.W, TW) * cdiv(v.H, TH)), t(TPB);
     if (v.algo == kSuBSENSE) {
-        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kSuBSENSE>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
-        else hipLaunchKernelGGL((k_refresh<1, kSuBSENSE>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
+        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kSuBSENSE>), g, t, 0, st, v, frac, force_fg, frame, ev, outside);
+        else hipLaunchKernelGGL((k_refresh<1, kSuBSENSE>), g, t, 0, st, v, frac, force_fg, frame, ev, outside);
     } else {
-        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kLOBSTER>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
-        else hipLaunchKernelGGL((k_refresh<1, kLOBSTER>), g, t, 0, st, v, 0, frac, force_fg, frame, ev, outside);
+        if (v.C == 3) hipLaunchKernelGGL((k_refresh<3, kLOBSTER>), g, t, 0, st, v, frac, force_fg, frame, ev, outside);
+        else hipLaunchKernelGGL((k_refresh<1, kLOBSTER>), g, t, 0, st, v, frac, force_fg, frame, ev, outside);
     }
 }
 
@@ -2780,13 +2845,15 @@ void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16
     }
 }
 
-// the SuBSENSE hole-filling and median kernels alone, on whatever v.raw holds
-void launch_postprocess_probe(const View& v, hipStream_t st) {
+// the SuBSENSE hole-filling and median kernels alone, on a raw mask
+void launch_postprocess_probe(const View& view, uint8_t* raw, hipStream_t st) {
+    View v = view;
+    v.dec = v.last_raw = raw;
     uint32_t g[kNumGrids];
     kernel_grids(v, StepOptions{}, g);
     hipLaunchKernelGGL(k_zone_close, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
     hipLaunchKernelGGL(k_zone_link, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
-    hipLaunchKernelGGL(k_zone_holes, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
+    hipLaunchKernelGGL(k_zone_holes, dim3(g[kGridZone]), dim3(TPB), 0, st, v, 0u);
     hipLaunchKernelGGL((k_median<true>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
 }
 

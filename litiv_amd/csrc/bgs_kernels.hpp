@@ -35,12 +35,10 @@ enum GridKind : int {
     kGridTile = 0,   // 64x4 pixel tiles (describe, match, update)
     kGridPost,       // 64x16 tiles (median, dilate)
     kGridZone,       // 64x64 hole-filling zones, four per block
-    kGridPix,        // 256 pixels per block
     kGridCell,       // 256 frame-level cells per block (0 when learning-rate scaling is off)
     kGridOne,        // one block per stream
     kGridFix,        // fix-point iteration grid
     kGridCont,       // cooperative match grid
-    kGridSweep,      // grid-stride sweep over the pixels (pending model refresh; mostly idle)
     kNumGrids
 };
 void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]);
@@ -60,7 +58,7 @@ void launch_init_desc(const View& v, const uint8_t* img, hipStream_t st);
 void launch_background(const View& v, uint8_t* out_img, hipStream_t st);
 void launch_background_desc(const View& v, uint16_t* out_desc, hipStream_t st);
 void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st);
-void launch_postprocess_probe(const View& v, hipStream_t st);
+void launch_postprocess_probe(const View& v, uint8_t* raw, hipStream_t st);
 // out[i] = the sticky error bits (Scalars::err_flags) of d_views[i], i < n
 void launch_gather_errors(const View* d_views, int n, uint32_t* d_out, hipStream_t st);
 void launch_rng_probe(const View& v, uint32_t frame, uint32_t phase, uint32_t ev, uint32_t n, uint32_t* out,

@@ -37,7 +37,6 @@ struct View {
     // u8 W*H maps
     uint8_t *unstable, *blinks, *last_raw, *last_raw_blink, *last_fg, *last_dil_inv;
     // per-frame scratch
-    uint8_t* raw;            // W*H raw segmentation (0/255)
     // hole filling on 64x64 zones (row-major zone grid): bit x of word 64*z+y is pixel (x, y) of
     // zone z; zbits = zero pixels of the closed mask, hbits = holes
     uint64_t *zbits, *hbits;
@@ -47,7 +46,7 @@ struct View {
     uint16_t* desc_cur;      // W*H*C intra descriptors of the current frame
     uint32_t* rec;           // W*H update records
     uint32_t* mres;          // W*H match results
-    uint8_t* dec;            // W*H raw decisions (1 = foreground)
+    uint8_t* dec;            // W*H raw decisions (1 = foreground; 0 outside the ROI)
     uint32_t* wl0;           // fix-point worklists: of even iterations (W*H entries), of odd ones
     uint32_t* wl1;           // (iteration 1 in stripes of cont_region entries like cont)
     uint32_t* cont;          // pixels left by the speculative match to the continuation: stripe k's
