@@ -295,6 +295,15 @@ static int setup_geometry(lvbgs_ctx* c, int w, int h, int ch, size_t orig, size_
     v.H = h;
     v.C = ch;
     v.N = (int)c->p.bg_samples;
+    {
+        // 2^s <= N < 2^(s+1): n_mul = ceil(2^(32+s) / N) fits 32 bits and its error times a draw stays below
+        // 2^(32+s); a power of two takes s - 1
+        uint32_t n = (uint32_t)v.N, sh = 0;
+        while ((2u << sh) <= n) ++sh;
+        if (n > 1 && (n & (n - 1)) == 0) --sh;
+        v.n_shift = sh;
+        v.n_mul = n > 1 ? (uint32_t)((((uint64_t)1 << (32 + sh)) + n - 1) / n) : 0u;
+    }
     v.REQ = (int)c->p.required_bg_samples;
     v.algo = c->algo;
     v.npx = (uint32_t)npx;

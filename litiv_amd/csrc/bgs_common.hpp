@@ -54,6 +54,23 @@ LV_HD uint32_t mod64(uint32_t d, uint64_t m) {
     return d % (uint32_t)m;
 }
 
+// True iff the 31-bit draw d is a multiple of m (1 <= m <= kDividesMax). Two rounds of a float quotient by
+// a reciprocal (within one ulp, as v_rcp_f32 gives it): the first leaves a remainder of at most 512 + m/2 in
+// magnitude (d has 31 bits, a float 24), exact in integers; the second is exact in floats, and its
+// remainder is zero iff m divides d. 19 issue slots against about 36 for the integer remainder.
+constexpr uint32_t kDividesMax = 1u << 22;
+LV_HD bool divides31(uint32_t d, uint32_t m) {
+    const float mf = (float)m;
+#ifdef __HIP_DEVICE_COMPILE__
+    const float r = __builtin_amdgcn_rcpf(mf);
+#else
+    const float r = 1.0f / mf;
+#endif
+    const uint32_t q = (uint32_t)rintf((float)d * r);
+    const float rem = (float)(int32_t)(d - q * m);
+    return __builtin_fmaf(-rintf(rem * r), mf, rem) == 0.0f;
+}
+
 // ------------------------------------------------------------------------------------------
 // LBSP 16-bit double cross (LBSP.hpp:275-298): bit n compares the centre with (x+DX[n], y+DY[n]).
 // ------------------------------------------------------------------------------------------
@@ -113,12 +130,6 @@ LV_D uint32_t lbsp_threshold_packed(const uint32_t taps[4], uint32_t ref, uint32
 constexpr int kSample7x7[49] = {2, 4, 6,  7,  6,  4,  2,  4, 8,  12, 14, 12, 8, 4, 6, 12, 21,
                                                    25, 21, 12, 6, 7, 14, 25, 28, 25, 14, 7, 6, 12, 21, 25, 21, 12,
                                                    6, 4, 8,  12, 14, 12, 8, 4, 2,  4,  6,  7,  6,  4,  2};
-constexpr int kNb3[8][2] = {{-1, 1}, {0, 1}, {1, 1}, {-1, 0}, {1, 0}, {-1, -1}, {0, -1}, {1, -1}};
-constexpr int kNb5[24][2] = {{-2, 2}, {-1, 2}, {0, 2},  {1, 2},  {2, 2},   {-2, 1},
-                                                {-1, 1}, {0, 1},  {1, 1},  {2, 1},  {-2, 0},  {-1, 0},
-                                                {1, 0},  {2, 0},  {-2, -1}, {-1, -1}, {0, -1}, {1, -1},
-                                                {2, -1}, {-2, -2}, {-1, -2}, {0, -2}, {1, -2}, {2, -2}};
-
 LV_HD void clamp_coords(int& x, int& y, int border, int w, int h) {
     if (x < border) x = border;
     else if (x >= w - border) x = w - border - 1;
@@ -139,17 +150,15 @@ LV_HD void sample_offset_7x7(uint32_t rnd, int& dx, int& dy) {
     dy = (i / 7) - 3;
 }
 
-// getNeighborPosition_3x3 / _5x5 (opencv.hpp:928-966), border 2
+// getNeighborPosition_3x3 / _5x5 (opencv.hpp:928-966), border 2. Both tables list the window's rows
+// from the bottom up without the centre, so entry i is cell i, past the centre i + 1 (two dependent table loads
+// otherwise).
 LV_HD void neighbor_pos(uint32_t rnd, bool use3, int x, int y, int w, int h, int& ox, int& oy) {
-    if (use3) {
-        const int r = (int)(rnd % 8u);
-        ox = x + kNb3[r][0];
-        oy = y + kNb3[r][1];
-    } else {
-        const int r = (int)(rnd % 24u);
-        ox = x + kNb5[r][0];
-        oy = y + kNb5[r][1];
-    }
+    const uint32_t r3 = rnd % 8u, r5 = rnd % 24u;
+    const uint32_t i3 = r3 + (r3 >= 4u ? 1u : 0u), i5 = r5 + (r5 >= 12u ? 1u : 0u);
+    const uint32_t row3 = (i3 * 11u) >> 5, row5 = (i5 * 13u) >> 6;  // i3 / 3 (i3 < 9), i5 / 5 (i5 < 25)
+    ox = x + (use3 ? (int)(i3 - 3u * row3) - 1 : (int)(i5 - 5u * row5) - 2);
+    oy = y + (use3 ? 1 - (int)row3 : 2 - (int)row5);
     clamp_coords(ox, oy, 2, w, h);
 }
 

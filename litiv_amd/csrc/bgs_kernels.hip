@@ -23,6 +23,8 @@
 #include <cmath>
 
 #include <algorithm>
+#include <cstddef>
+#include <type_traits>
 
 #include "bgs_kernels.hpp"
 
@@ -44,24 +46,48 @@ LV_D uint32_t absdiff(uint32_t a, uint32_t b) { return a > b ? a - b : b - a; }
 LV_D float fmin_ref(float a, float b) { return (b < a) ? b : a; }  // std::min
 LV_D float fmax_ref(float a, float b) { return (a < b) ? b : a; }  // std::max
 
-// Workgroup sum of one value per thread, added to stripe blockIdx % kStripes of a counter array.
-// Every thread of the workgroup must call it. The closing barrier keeps the wavefront partials in
-// LDS until thread 0 has summed them, so a second call right after (the model update adds two
-// counters) cannot overwrite them early.
-template <int NT>
-LV_D void block_add(unsigned long long value, unsigned long long* stripes) {
-    __shared__ unsigned long long part[NT / 64];
+// Sum of one value per lane over the wavefront, in lane 63 (DPP row shifts and broadcasts: six adds, no LDS).
+LV_D uint32_t wave_sum_last(uint32_t x) {
+    auto step = [&](auto ctrl, auto rows) {
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
+    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});  // row_shr:2
+    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});  // row_shr:4
+    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});  // row_shr:8
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31
+    return x;
+}
+
+// Workgroup sums of K 32-bit values per thread (each below 2^24), added to stripe blockIdx % kStripes of K
+// counter arrays. Every thread of the workgroup must call it, once per kernel.
+template <int NT, int K>
+LV_D void block_add(const uint32_t (&value)[K], unsigned long long* const (&stripes)[K]) {
+    __shared__ uint32_t part[NT / 64][K];
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) value += __shfl_down(value, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = value;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long s = 0;
-#pragma unroll
-        for (int i = 0; i < NT / 64; ++i) s += part[i];
-        if (s) atomicAdd(&stripes[blockIdx.x % kStripes], s);
+    for (int k = 0; k < K; ++k) {
+        const uint32_t t = wave_sum_last(value[k]);
+        if (lane == 63) part[wave][k] = t;
     }
     __syncthreads();
+    if (threadIdx.x < (uint32_t)K) {
+        uint32_t t = 0;
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) t += part[i][threadIdx.x];
+        unsigned long long* s = stripes[0];
+#pragma unroll
+        for (int k = 1; k < K; ++k) s = threadIdx.x == (uint32_t)k ? stripes[k] : s;
+        if (t) atomicAdd(&s[blockIdx.x % kStripes], (unsigned long long)t);
+    }
+}
+template <int NT>
+LV_D void block_add(uint32_t value, unsigned long long* stripes) {
+    const uint32_t v1[1] = {value};
+    unsigned long long* const s1[1] = {stripes};
+    block_add<NT, 1>(v1, s1);
 }
 
 LV_HD unsigned long long sum_stripes(const unsigned long long* s) {
@@ -97,6 +123,14 @@ using gptr = __attribute__((address_space(1))) T*;
 template <typename T>
 LV_D gptr<T> G(T* p) {
     return (gptr<T>)p;
+}
+
+// element i of a per-pixel array, through a 32-bit byte offset: every per-pixel array is below 4 GiB (at most 2^28
+// pixels of 6 bytes), so a load takes its base from scalar registers and its offset from one vector
+// register, where a 64-bit index costs two or three vector adds per access
+template <typename T, typename I>
+LV_D gptr<T> at(T* base, I i) {
+    return (gptr<T>)((gptr<const uint8_t>)base + (uint32_t)((uint32_t)i * (uint32_t)sizeof(T)));
 }
 
 // wavefront-local LDS exchange: the lanes' stores above are visible to the loads below
@@ -201,42 +235,69 @@ template <int C>
 LV_D void current_value(const View& v, const uint8_t* frame, uint32_t q, uint32_t col[C], uint32_t desc[C]) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        col[c] = G(frame)[(size_t)q * C + c];
-        desc[c] = G(v.desc_cur)[(size_t)q * C + c];
+        col[c] = *at(frame, q * C + c);
+        desc[c] = *at(v.desc_cur, q * C + c);
     }
 }
 
 // ----------------------------------------------------------------------------------------------
 // LDS frame tile with a 2-pixel halo (the 5x5 LBSP patch)
 // ----------------------------------------------------------------------------------------------
+// Rows are loaded as 32-bit words from 8 (RGB) or 4 (grey) bytes left of the tile, so a halo row is 52 or 18
+// loads instead of 204 or 68 byte loads; PITCH is a row's bytes in LDS and OFF where its first pixel lies.
 template <int C>
 struct FrameTile {
-    static constexpr int LW = TW + 4, LH = TH + 4;
-    uint8_t px[LW * LH * C];
+    static constexpr int LW = TW + 4, LH = TH + 4, OFF = 2, WORDS = C == 3 ? 52 : 18, PITCH = 4 * WORDS;
+    alignas(4) uint8_t px[LH * PITCH];
+    // byte of channel c of halo pixel (lx, ly)
+    static constexpr int at(int lx, int ly, int c) { return ly * PITCH + OFF + lx * C + c; }
 };
+
+// a 32-bit word at any byte offset of a buffer of `total` bytes (4 at least), zeros outside it. Global loads need
+// no alignment here; the last bytes of a buffer come from its last whole word.
+struct __attribute__((packed, aligned(1))) UnalignedU32 {
+    uint32_t v;
+};
+LV_D uint32_t word_at(const uint8_t* base, int off, int total) {
+    const int o = off < 0 ? 0 : off > total - 4 ? total - 4 : off;
+    const uint32_t w = ((gptr<const UnalignedU32>)((gptr<const uint8_t>)base + (uint32_t)o))->v;
+    const int beyond = off - o;  // < 0: left of the buffer, > 0: bytes to drop
+    return beyond < 0 || beyond > 3 ? 0u : w >> (8 * beyond);
+}
 
 template <int C>
 LV_D void load_frame_tile(FrameTile<C>& t, const uint8_t* frame, int W, int H, int x0, int y0) {
-    constexpr int LW = FrameTile<C>::LW, LH = FrameTile<C>::LH;
-    for (int i = threadIdx.x; i < LW * LH; i += TPB) {
-        const int ly = i / LW, lx = i % LW, gx = x0 + lx - 2, gy = y0 + ly - 2;
-        const bool in = gx >= 0 && gx < W && gy >= 0 && gy < H;
+    using T = FrameTile<C>;
+    const int total = W * H * C, left = C == 3 ? 8 : 4;
+    if constexpr (C == 3) {  // a wavefront per row
+        const int l = (int)(threadIdx.x & 63u);
 #pragma unroll
-        for (int c = 0; c < C; ++c) t.px[i * C + c] = in ? G(frame)[((size_t)gy * W + gx) * C + c] : (uint8_t)0;
+        for (int k = 0; k < T::LH / 4; ++k) {
+            const int r = (int)(threadIdx.x >> 6) + 4 * k, gy = y0 + r - 2;
+            if (l < T::WORDS) {
+                const uint32_t w = gy >= 0 && gy < H ? word_at(frame, (gy * W + x0) * C - left + 4 * l, total) : 0u;
+                *(uint32_t*)&t.px[r * T::PITCH + 4 * l] = w;
+            }
+        }
+    } else {
+        const int r = (int)threadIdx.x / T::WORDS, l = (int)threadIdx.x % T::WORDS, gy = y0 + r - 2;
+        if (r < T::LH) {
+            const uint32_t w = gy >= 0 && gy < H ? word_at(frame, gy * W + x0 - left + 4 * l, total) : 0u;
+            *(uint32_t*)&t.px[r * T::PITCH + 4 * l] = w;
+        }
     }
 }
 
 // packed 16 taps of channel c around tile-local (lx,ly) (centre coordinates, halo excluded)
 template <int C>
 LV_D void taps_from_tile(const FrameTile<C>& t, int lx, int ly, int c, uint32_t taps[4]) {
-    constexpr int LW = FrameTile<C>::LW;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         uint32_t acc = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int n = 4 * w + k;
-            acc |= (uint32_t)t.px[((ly + 2 + kLbspDY[n]) * LW + (lx + 2 + kLbspDX[n])) * C + c] << (8 * k);
+            acc |= (uint32_t)t.px[FrameTile<C>::at(lx + 2 + kLbspDX[n], ly + 2 + kLbspDY[n], c)] << (8 * k);
         }
         taps[w] = acc;
     }
@@ -250,15 +311,16 @@ LV_D void taps_from_global(const uint8_t* frame, int W, int x, int y, int c, uin
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int n = 4 * w + k;
-            acc |= (uint32_t)G(frame)[((size_t)(y + kLbspDY[n]) * W + (x + kLbspDX[n])) * C + c] << (8 * k);
+            acc |= (uint32_t)*at(frame, ((y + kLbspDY[n]) * W + (x + kLbspDX[n])) * C + c) << (8 * k);
         }
         taps[w] = acc;
     }
 }
 
+// lut_lds: 4-byte aligned
 LV_D void load_lut(uint8_t* lut_lds, const Scalars* sc) {
-    const gptr<const uint8_t> src = G(sc->lut);
-    for (int i = threadIdx.x; i < 256; i += blockDim.x) lut_lds[i] = src[i];
+    static_assert(offsetof(Scalars, lut) % 4 == 0, "the LUT is read in words");
+    if (threadIdx.x < 64u) ((uint32_t*)lut_lds)[threadIdx.x] = *at((const uint32_t*)sc->lut, threadIdx.x);
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -589,7 +651,13 @@ LV_D bool forward_target(const View& v, uint32_t r, int x, int y, uint32_t& t) {
     const int dx = tgt_dx(tg), dy = tgt_dy(tg);
     if (!(dy > 0 || (dy == 0 && dx > 0))) return false;
     t = (uint32_t)((y + dy) * v.W + (x + dx));
-    return G(v.roi)[t] != 0;
+    return *at(v.roi, t) != 0;
+}
+
+// draw % N, with the reciprocal of N laid out in the View
+LV_D uint32_t mod_n(const View& v, uint32_t d) {
+    const uint32_t q = __umulhi(d, v.n_mul) >> v.n_shift;
+    return v.N == 1 ? 0u : d - q * (uint32_t)v.N;
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -601,7 +669,7 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     const uint8_t* frame = v.frame;
     const double lr = v.lr;
     __shared__ FrameTile<C> tile;
-    __shared__ uint8_t lut[256];
+    __shared__ alignas(4) uint8_t lut[256];
     const int ntx = (v.W + TW - 1) / TW;
     const int tid = (int)bid;
     const int x0 = (tid % ntx) * TW, y0 = (tid / ntx) * TH;
@@ -625,13 +693,13 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     const bool inside = x < v.W && y < v.H;
     // the pixel's own state is loaded first, so these loads run alongside the tile's
     const uint32_t pp = inside ? (uint32_t)(y * v.W + x) : 0u;
-    const uint8_t roi_p = G(v.roi)[pp];
+    const uint8_t roi_p = *at(v.roi, pp);
     float Rv = 0.f, Tv = 0.f, d_lt = 0.f, d_st = 0.f;
     if constexpr (ALGO == kSuBSENSE) {
-        Rv = G(v.R)[pp];
-        Tv = G(v.T)[pp];
-        d_lt = G(v.RawLT)[pp] - G(v.FinLT)[pp];
-        d_st = G(v.RawST)[pp] - G(v.FinST)[pp];
+        Rv = *at(v.R, pp);
+        Tv = *at(v.T, pp);
+        d_lt = *at(v.RawLT, pp) - *at(v.FinLT, pp);
+        d_st = *at(v.RawST, pp) - *at(v.FinST, pp);
     }
     load_frame_tile<C>(tile, frame, v.W, v.H, x0, y0);
     load_lut(lut, v.sc);
@@ -640,7 +708,7 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     if (inside) {
         const uint32_t p = pp;
         if (!roi_p) {
-            G(v.rec)[p] = kRecNone;
+            *at(v.rec, p) = kRecNone;
         } else {
             uint32_t pc = 0;
             uint32_t intra[C];
@@ -648,59 +716,66 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
             for (int c = 0; c < C; ++c) {
                 uint32_t taps[4];
                 taps_from_tile<C>(tile, lx, ly, c, taps);
-                const uint32_t ref = tile.px[((ly + 2) * FrameTile<C>::LW + (lx + 2)) * C + c];
+                const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
                 intra[c] = lbsp_threshold_sad(taps, ref, lut[ref]);
-                G(v.desc_cur)[(size_t)p * C + c] = (uint16_t)intra[c];
+                *at(v.desc_cur, p * C + c) = (uint16_t)intra[c];
                 pc += popc(intra[c]);
             }
             nz = pc >= (C == 1 ? 2u : 4u);
             const uint32_t frame_no = cur_frame(v);
             uint32_t d[4];
             draw4(v.seed_lo, v.seed_hi, v.stream_id, frame_no, PH_APPLY, 0, p, 0, d);
-            const uint32_t N = (uint32_t)v.N;
             // draw 4 (group 1) is the diffusion slot: drawn only when a diffusion gate is open
             auto diff_slot = [&]() {
                 uint32_t d4[4];
                 draw4(v.seed_lo, v.seed_hi, v.stream_id, frame_no, PH_APPLY, 0, p, 1, d4);
-                return mod64(d4[0], N);
+                return mod_n(v, d4[0]);
             };
+            // learning rates beyond the exact range of divides31 (uniform; infinity among them)
+            const bool slow = lr > (double)kDividesMax;
             uint32_t r;
             if constexpr (ALGO == kSuBSENSE) {
                 const uint32_t unst_new = (Rv > 3.0f || d_lt > 0.1f || d_st > 0.1f) ? 1u : 0u;
-                const uint64_t L = isinf(lr) ? ~0ull : (lr > 0 ? (uint64_t)ceil(lr) : (uint64_t)ceilf(Tv));
-                const bool self_bg = mod64(d[0], L) == 0u;
-                const bool self_fg = v.sc->cooldown != 0u && (d[0] % 2u) == 0u;
                 const bool use3 = v.use3x3 && !unst_new;
+                bool self_bg, gate_a;
+                if (slow) {
+                    const uint64_t L = isinf(lr) ? ~0ull : (uint64_t)ceil(lr);
+                    self_bg = mod64(d[0], L) == 0u;
+                    gate_a = mod64(d[3], use3 ? L : L / 2u + 1u) == 0u;
+                } else {
+                    const uint32_t L = lr > 0 ? (uint32_t)ceil(lr) : (uint32_t)ceilf(Tv);
+                    self_bg = divides31(d[0], L);
+                    gate_a = divides31(d[3], use3 ? L : L / 2u + 1u);
+                }
+                const bool self_fg = v.sc->cooldown != 0u && (d[0] % 2u) == 0u;
                 int tx, ty;
                 neighbor_pos(d[2], use3, x, y, v.W, v.H, tx, ty);
-                const uint64_t spread = use3 ? L : L / 2u + 1u;
-                const bool gate_a = mod64(d[3], spread) == 0u;
-                const uint64_t lcap = (uint64_t)v.sc->lower_cap;
-                const bool gate_b = mod64(d[3], lcap) == 0u;
+                const uint32_t lcap = (uint32_t)v.sc->lower_cap;  // 1, 2 or 4
+                const bool gate_b = (lcap & (lcap - 1u)) == 0u ? (d[3] & (lcap - 1u)) == 0u : d[3] % lcap == 0u;
                 bool ghost_fwd = false;
                 if (ty > y || (ty == y && tx > x)) {
                     const uint32_t t = (uint32_t)(ty * v.W + tx);
-                    ghost_fwd = G(v.RawST)[t] > 0.995f && G(v.MLD)[t] < 0.010f;
+                    ghost_fwd = *at(v.RawST, t) > 0.995f && *at(v.MLD, t) < 0.010f;
                 }
                 const uint32_t tg = (uint32_t)((ty - y + 2) * 5 + (tx - x + 2));
                 const uint32_t sd = (gate_a || gate_b) ? diff_slot() : 0u;
                 r = tg | ((uint32_t)gate_a << 5) | ((uint32_t)gate_b << 6) | ((uint32_t)ghost_fwd << 7) |
-                    ((uint32_t)self_bg << 8) | ((uint32_t)self_fg << 9) | (unst_new << 10) | (mod64(d[1], N) << 16) |
+                    ((uint32_t)self_bg << 8) | ((uint32_t)self_fg << 9) | (unst_new << 10) | (mod_n(v, d[1]) << 16) |
                     (sd << 24);
             } else {
                 const uint64_t L = isinf(lr) ? ~0ull : (uint64_t)ceil(lr);
-                const bool self_bg = mod64(d[0], L) == 0u;
-                const bool gate_a = mod64(d[2], L) == 0u;
+                const bool self_bg = slow ? mod64(d[0], L) == 0u : divides31(d[0], (uint32_t)L);
+                const bool gate_a = slow ? mod64(d[2], L) == 0u : divides31(d[2], (uint32_t)L);
                 int tx, ty;
                 neighbor_pos(d[3], true, x, y, v.W, v.H, tx, ty);
                 const uint32_t tg = (uint32_t)((ty - y + 2) * 5 + (tx - x + 2));
                 const uint32_t sd = gate_a ? diff_slot() : 0u;
-                r = tg | ((uint32_t)gate_a << 5) | ((uint32_t)self_bg << 8) | (mod64(d[1], N) << 16) | (sd << 24);
+                r = tg | ((uint32_t)gate_a << 5) | ((uint32_t)self_bg << 8) | (mod_n(v, d[1]) << 16) | (sd << 24);
             }
-            G(v.rec)[p] = r;
+            *at(v.rec, p) = r;
         }
     }
-    if constexpr (ALGO == kSuBSENSE) block_add<TPB>(nz ? 1ull : 0ull, v.sc->nz_part);
+    if constexpr (ALGO == kSuBSENSE) block_add<TPB>(nz ? 1u : 0u, v.sc->nz_part);
 }
 
 // a tile pixel's per-frame match inputs, loaded together with the tile and staged in LDS (the
@@ -715,12 +790,12 @@ struct PxIn {
 template <int C, int ALGO>
 LV_D PxIn<C> load_px_in(const View& v, uint32_t q, bool in) {
     PxIn<C> r;
-    r.roi = in ? G(v.roi)[q] : (uint8_t)0;
+    r.roi = in ? *at(v.roi, q) : (uint8_t)0;
 #pragma unroll
-    for (int c = 0; c < C; ++c) r.desc[c] = G(v.desc_cur)[(size_t)q * C + c];
+    for (int c = 0; c < C; ++c) r.desc[c] = *at(v.desc_cur, q * C + c);
     if constexpr (ALGO == kSuBSENSE) {
-        r.R = G(v.R)[q];
-        r.unst = G(v.unstable)[q];
+        r.R = *at(v.R, q);
+        r.unst = *at(v.unstable, q);
     } else {
         r.R = 0.f;
         r.unst = 0;
@@ -817,8 +892,8 @@ LV_D void build_ctx_global(const View& v, const uint8_t* frame, int x, int y, Px
     const uint32_t p = (uint32_t)(y * v.W + x);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        px.cur[c] = G(frame)[(size_t)p * C + c];
-        px.intra[c] = G(v.desc_cur)[(size_t)p * C + c];
+        px.cur[c] = *at(frame, p * C + c);
+        px.intra[c] = *at(v.desc_cur, p * C + c);
     }
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -828,11 +903,11 @@ LV_D void build_ctx_global(const View& v, const uint8_t* frame, int x, int y, Px
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int n = 4 * w + k;
-                acc |= (uint32_t)G(frame)[((size_t)(y + kLbspDY[n]) * v.W + (x + kLbspDX[n])) * C + c] << (8 * k);
+                acc |= (uint32_t)*at(frame, ((y + kLbspDY[n]) * v.W + (x + kLbspDX[n])) * C + c) << (8 * k);
             }
             px.taps[c][w] = acc;
         }
-    if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, G(v.R)[p], G(v.unstable)[p], px);
+    if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, *at(v.R, p), *at(v.unstable, p), px);
     else lobster_thresholds<C>(v, px);
 }
 
@@ -862,8 +937,8 @@ LV_D uint32_t group_writers(const View& v, int x, int y, bool active, uint32_t& 
     if (active && sub < 12u) {
         const int dx = pred_dx(sub), dy = pred_dy(sub);
         const uint32_t q = (uint32_t)((y + dy) * v.W + (x + dx));
-        const uint32_t r = G(v.rec)[q];
-        const uint8_t guess = G(v.last_raw)[q];
+        const uint32_t r = *at(v.rec, q);
+        const uint8_t guess = *at(v.last_raw, q);
         const uint8_t d = CURRENT ? __hip_atomic_load(&v.dec[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : guess;
         const bool writer = rec_tgt(r) == (uint32_t)((2 - dy) * 5 + (2 - dx)) && fwd_gate(r);
         slot = rec_slot_diff(r);
@@ -946,17 +1021,17 @@ LV_D void group_ctx(const View& v, const uint8_t* frame, int x, int y, bool acti
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int dx = (int)((ks >> (8 * k)) & 15u) - 2, dy = (int)((ks >> (8 * k + 4)) & 15u) - 2;
-            acc |= (uint32_t)G(frame)[((size_t)(y + dy) * v.W + (x + dx)) * C + c] << (8 * k);
+            acc |= (uint32_t)*at(frame, ((y + dy) * v.W + (x + dx)) * C + c) << (8 * k);
         }
         L.taps[g][sub] = acc;
     }
     if (active) {
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            px.cur[c] = G(frame)[(size_t)p * C + c];
-            px.intra[c] = G(v.desc_cur)[(size_t)p * C + c];
+            px.cur[c] = *at(frame, p * C + c);
+            px.intra[c] = *at(v.desc_cur, p * C + c);
         }
-        if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, G(v.R)[p], G(v.unstable)[p], px);
+        if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, *at(v.R, p), *at(v.unstable, p), px);
         else lobster_thresholds<C>(v, px);
     }
     wave_sync();
@@ -989,8 +1064,8 @@ LV_D void load_pred_tile(PredTile& t, const View& v, int x0, int y0) {
         const int ly = i / PredTile::LW, lx = i % PredTile::LW, gx = x0 + lx - 2, gy = y0 + ly - 2;
         const bool in = gx >= 0 && gx < v.W && gy >= 0 && gy < v.H;
         const size_t q = (size_t)gy * v.W + gx;
-        t.rec[ly][lx] = in ? G(v.rec)[q] : kRecNone;
-        t.guess[ly][lx] = in ? (G(v.last_raw)[q] ? 1 : 0) : 1;
+        t.rec[ly][lx] = in ? *at(v.rec, q) : kRecNone;
+        t.guess[ly][lx] = in ? (*at(v.last_raw, q) ? 1 : 0) : 1;
     }
 }
 
@@ -1017,7 +1092,7 @@ struct MatchLds {
         FrameTile<1> c1;
     } tile;
     PredTile pred;
-    uint8_t lut[256];
+    alignas(4) uint8_t lut[256];
     uint16_t perm[TPB];
     uint32_t nfg[TPB / 64];
     union {
@@ -1137,13 +1212,13 @@ LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, c
     const uint8_t guess = pred.guess[ly + 2][lx + 2];
     const bool fits = build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
     const uint32_t limit = !fits ? 0u : seq_limit < N ? seq_limit : N;
-    build_ctx_staged<C, ALGO, FrameTile<C>::LW * C>(v, &tile.px[(ly * FrameTile<C>::LW + lx) * C], in, px);
-    scan_seq<C, ALGO, FrameTile<C>::LW * C, KF>(v, lut, px, x, y, sbm, nrep, st, limit);
+    build_ctx_staged<C, ALGO, FrameTile<C>::PITCH>(v, &tile.px[FrameTile<C>::at(lx, ly, 0)], in, px);
+    scan_seq<C, ALGO, FrameTile<C>::PITCH, KF>(v, lut, px, x, y, sbm, nrep, st, limit);
     examined = st.s;
-    G(v.mres)[p] = pack_state(st);
+    *at(v.mres, p) = pack_state(st);
     if (fits && st.good < (uint32_t)v.REQ && st.s < N) return false;
     const uint8_t fg = !fits ? guess : st.good < (uint32_t)v.REQ ? 1 : 0;
-    G(v.dec)[p] = fg;
+    *at(v.dec, p) = fg;
     push = fg != guess && forward_target(v, pred.rec[ly + 2][lx + 2], x, y, target);
     if (!fits) {
         push = true;
@@ -1158,7 +1233,7 @@ LV_D uint32_t applied_writers_global(const View& v, int x, int y) {
 #pragma unroll
     for (int i = 0; i < 12; ++i) {
         const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
-        const uint32_t r = G(v.rec)[q];
+        const uint32_t r = *at(v.rec, q);
         const uint32_t code = (uint32_t)((2 - kPredDY[i]) * 5 + (2 - kPredDX[i]));
         if (rec_tgt(r) == code && fwd_gate(r)) m |= 1u << i;
     }
@@ -1166,7 +1241,7 @@ LV_D uint32_t applied_writers_global(const View& v, int x, int y) {
     for (; m; m &= m - 1) {
         const int i = __builtin_ctz(m);
         const uint32_t q = (uint32_t)((y + pred_dy((uint32_t)i)) * v.W + (x + pred_dx((uint32_t)i)));
-        if (G(v.last_raw)[q] == 0) applied |= 1u << i;
+        if (*at(v.last_raw, q) == 0) applied |= 1u << i;
     }
     return applied;
 }
@@ -1175,11 +1250,11 @@ LV_D uint32_t applied_writers_global(const View& v, int x, int y) {
 // speculative guess and the pixel has a forward target (for the first fix-point worklist)
 template <int C>
 LV_D bool finish_pixel(const View& v, uint32_t p, int x, int y, const ScanState& st, uint32_t& t) {
-    G(v.mres)[p] = pack_state(st);
+    *at(v.mres, p) = pack_state(st);
     const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
-    G(v.dec)[p] = fg;
-    const uint8_t guess = G(v.last_raw)[p] ? 1 : 0;
-    return fg != guess && forward_target(v, G(v.rec)[p], x, y, t);
+    *at(v.dec, p) = fg;
+    const uint8_t guess = *at(v.last_raw, p) ? 1 : 0;
+    return fg != guess && forward_target(v, *at(v.rec, p), x, y, t);
 }
 
 // push_first for lanes of different stripes: one append per stripe present in the wavefront
@@ -1217,10 +1292,10 @@ LV_D void match_seq_lanes(const View& v, const uint8_t* lut, const uint32_t* s_p
         const uint32_t applied = applied_writers_global(v, x, y);
         uint64_t sbm;
         int nrep;
-        auto rec_of = [&](int i) { return G(v.rec)[(size_t)(y + kPredDY[i]) * v.W + (x + kPredDX[i])]; };
+        auto rec_of = [&](int i) { return *at(v.rec, (y + kPredDY[i]) * v.W + (x + kPredDX[i])); };
         // at most kRepl slots: phase A keeps the others (same writers, same guesses)
         (void)build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
-        ScanState st = unpack_state(G(v.mres)[p]);
+        ScanState st = unpack_state(*at(v.mres, p));
         const uint32_t s0 = st.s;
         scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
         examined += st.s - s0;
@@ -1253,7 +1328,7 @@ LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_
             y = (int)(p / (uint32_t)v.W);
             if (j < v.cont_ctx_region) load_ctx<C>(v.cont_ctx + ((size_t)k * v.cont_ctx_region + j) * kCtxWords, px);
             else build_ctx_global<C, ALGO>(v, frame, x, y, px);
-            st = unpack_state(G(v.mres)[p]);
+            st = unpack_state(*at(v.mres, p));
         }
         uint32_t slot;
         bool turned;
@@ -1273,7 +1348,7 @@ LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_
 
 template <int C, int ALGO, int KF>
 LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
-    __shared__ uint8_t lut[256];
+    __shared__ alignas(4) uint8_t lut[256];
     __shared__ uint32_t s_pre[kContStripes + 1];  // exclusive prefix of the stripe counts
     stripe_prefix(v.sc->cont_cnt, s_pre);
     load_lut(lut, v.sc);
@@ -1303,11 +1378,11 @@ LV_D uint32_t wl_total(const View& v, uint32_t k, uint32_t* pre) {
 
 // result of a fix-point re-match; true when the decision changed and the pixel has a forward target
 LV_D bool rematch_done(const View& v, uint32_t p, int x, int y, const ScanState& st, uint32_t& t) {
-    G(v.mres)[p] = pack_state(st);
+    *at(v.mres, p) = pack_state(st);
     const uint8_t fg = st.good < (uint32_t)v.REQ ? 1 : 0;
-    if (fg == G(v.dec)[p]) return false;
+    if (fg == *at(v.dec, p)) return false;
     __hip_atomic_store(&v.dec[p], fg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return forward_target(v, G(v.rec)[p], x, y, t);
+    return forward_target(v, *at(v.rec, p), x, y, t);
 }
 
 // Fix-point re-match of a wavefront's worklisted pixels i0 .. i0 + 64/kGroup - 1, one group each. In iteration 1
@@ -1323,7 +1398,7 @@ LV_D void rematch(const View& v, const uint8_t* lut, GroupLds& L, const uint32_t
     const uint32_t p = active ? wl_item(v, k, pre, i) : 0u;
     const int x = (int)(p % (uint32_t)v.W), y = (int)(p / (uint32_t)v.W);
     // samples its result rests on; 0 = not matched yet
-    const uint32_t seen = active && k == 1u ? G(v.mres)[p] >> 24 : 0u;
+    const uint32_t seen = active && k == 1u ? *at(v.mres, p) >> 24 : 0u;
     uint32_t slot;
     bool turned;
     const uint32_t applied = group_writers<true>(v, x, y, active, slot, seen, turned);
@@ -1379,7 +1454,7 @@ LV_D void fixpoint_tail(const View& v, const uint8_t* lut, GroupLds& L, uint32_t
 enum FixKind : int { kFixMore, kFixLast, kFixTail };
 template <int C, int ALGO, int KIND>
 LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k, uint32_t cap) {
-    __shared__ uint8_t lut[256];
+    __shared__ alignas(4) uint8_t lut[256];
     __shared__ GroupLds L;
     __shared__ uint32_t s_pre[kContStripes + 1];
     if constexpr (KIND == kFixTail) {
@@ -1423,80 +1498,140 @@ LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k, 
 // SuBSENSE feedback maps (SUB:396-420, :451-480; 1ch :254-329), raw mask and blink bookkeeping
 // (SUB:536-539). Whole image: pixels outside the ROI get raw = 0.
 // ----------------------------------------------------------------------------------------------
-// One pixel (p < npx). Returns p's samples examined (k_p) and its RawST / MLD after the update
-// (the values the model update's ghost test reads).
+// v / n as the IEEE quotient, from the correctly rounded reciprocal inv = 1 / n with one residual correction:
+// equal to the division for every whole v < 2^16 and whole n <= 255 as well as 765 (checked exhaustively),
+// three operations where the division takes about ten
+LV_HD float quot(float v, float n, float inv) {
+    const float q = v * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q, n, v), inv, q);
+}
+
+// A pixel's state of the previous frame, loaded ahead of the tile barrier. The last colour and descriptor are
+// read as one and two words (a byte or two past them lies in the same allocation).
 template <int C>
-LV_D uint32_t feedback_pixel(const View& v, uint32_t p, float& rst_out, float& mld_out) {
-    const uint8_t* frame = v.frame;
+struct PxState {
+    uint32_t last_color, last_desc[C == 3 ? 2 : 1];
+    float mld, dlt, dst, rlt, rst, T, V, R;
+    uint32_t mres;
+    uint8_t roi, last_fg, blinks, last_raw, last_raw_blink;
+};
+struct __attribute__((packed, aligned(1))) UnalignedU16 {
+    uint16_t v;
+};
+template <typename W, typename T>
+LV_D auto peek(T* base, uint32_t byte) {
+    return ((gptr<const W>)((gptr<const uint8_t>)base + byte))->v;
+}
+template <typename W, typename T, typename V>
+LV_D void poke(T* base, uint32_t byte, V value) {
+    ((gptr<W>)((gptr<uint8_t>)base + byte))->v = value;
+}
+
+template <int C>
+LV_D void load_px_state(const View& v, uint32_t p, PxState<C>& s) {
+    s.roi = *at(v.roi, p);
+    s.mres = *at(v.mres, p);
+    if constexpr (C == 3) {
+        s.last_color = peek<UnalignedU32>(v.last_color, 3u * p);
+        s.last_desc[0] = peek<UnalignedU32>(v.last_desc, 6u * p);
+        s.last_desc[1 % (C == 3 ? 2 : 1)] = peek<UnalignedU16>(v.last_desc, 6u * p + 4u);
+    } else {
+        s.last_color = *at(v.last_color, p);
+        s.last_desc[0] = *at(v.last_desc, p);
+    }
+    s.mld = *at(v.MLD, p);
+    s.dlt = *at(v.DminLT, p);
+    s.dst = *at(v.DminST, p);
+    s.rlt = *at(v.RawLT, p);
+    s.rst = *at(v.RawST, p);
+    s.T = *at(v.T, p);
+    s.V = *at(v.V, p);
+    s.R = *at(v.R, p);
+    s.last_fg = *at(v.last_fg, p);
+    s.blinks = *at(v.blinks, p);
+    s.last_raw = *at(v.last_raw, p);
+    s.last_raw_blink = *at(v.last_raw_blink, p);
+}
+
+template <int C>
+LV_D void store_last(const View& v, uint32_t p, const uint32_t cur[C], const uint32_t intra[C]) {
+    if constexpr (C == 3) {
+        poke<UnalignedU16>(v.last_color, 3u * p, (uint16_t)(cur[0] | cur[1] << 8));
+        *at(v.last_color, 3u * p + 2u) = (uint8_t)cur[2 % C];
+        poke<UnalignedU32>(v.last_desc, 6u * p, intra[0] | intra[1 % C] << 16);
+        poke<UnalignedU16>(v.last_desc, 6u * p + 4u, (uint16_t)intra[2 % C]);
+    } else {
+        *at(v.last_color, p) = (uint8_t)cur[0];
+        *at(v.last_desc, p) = (uint16_t)intra[0];
+    }
+}
+
+// One pixel (p < npx) with its current colour, descriptor, record and decision. Returns p's samples examined
+// (k_p); s.rst and s.mld become the updated values the model update's ghost test reads.
+template <int C>
+LV_D uint32_t feedback_pixel(const View& v, uint32_t p, PxState<C>& s, const uint32_t cur[C], const uint32_t intra[C],
+                             bool unstable, bool fg) {
     uint32_t examined = 0;
     uint8_t raw = 0;
-    if (!G(v.roi)[p]) {
-        rst_out = G(v.RawST)[p];
-        mld_out = G(v.MLD)[p];
-    } else {
+    if (s.roi) {
         const uint32_t frame_no = cur_frame(v);
         const uint32_t mvn = v.mv_avgs;
         const float aLT = 1.0f / (float)(frame_no < mvn ? frame_no : mvn);
         const float aST = 1.0f / (float)(frame_no < mvn / 4u ? frame_no : mvn / 4u);
-        const uint32_t mr = G(v.mres)[p];
-        const uint32_t good = mr & 255u, md = (mr >> 8) & 63u, ms = (mr >> 14) & 1023u;
-        examined = mr >> 24;
-        const bool fg = G(v.dec)[p] != 0;
-        const uint32_t r = G(v.rec)[p];
-        const uint32_t unst_new = rec_unstable(r) ? 1u : 0u;
-        const float col_max = (float)(C * 255), desc_max = (float)(C * 16);
+        const uint32_t good = s.mres & 255u, md = (s.mres >> 8) & 63u, ms = (s.mres >> 14) & 1023u;
+        examined = s.mres >> 24;
+        constexpr float col_max = (float)(C * 255), desc_max = (float)(C * 16);
+        constexpr float inv_col = 1.0f / col_max, inv_desc = 1.0f / desc_max;
         // D_last (SUB:396-397): L1dist<3> accumulates in uchar (wraps mod 256)
         uint32_t l1 = 0, hd = 0;
-        uint32_t cur[C], intra[C];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            cur[c] = G(frame)[(size_t)p * C + c];
-            intra[c] = G(v.desc_cur)[(size_t)p * C + c];
-            l1 += absdiff(G(v.last_color)[(size_t)p * C + c], cur[c]);
-            hd += popc((uint32_t)G(v.last_desc)[(size_t)p * C + c] ^ intra[c]);
+            l1 = __builtin_amdgcn_sad_u8((s.last_color >> (8 * c)) & 255u, cur[c], l1);
+            hd += popc(((s.last_desc[c / 2] >> (16 * (c & 1))) & 0xFFFFu) ^ intra[c]);
         }
         l1 &= 255u;
-        const float nld = ((float)l1 / col_max + (float)hd / desc_max) / 2.0f;
-        const float mld = G(v.MLD)[p] * (1.0f - aST) + nld * aST;
-        G(v.MLD)[p] = mld;
-        float dlt = G(v.DminLT)[p], dst = G(v.DminST)[p], rlt = G(v.RawLT)[p], rst = G(v.RawST)[p];
+        const float nld = (quot((float)l1, col_max, inv_col) + quot((float)hd, desc_max, inv_desc)) / 2.0f;
+        const float mld = s.mld * (1.0f - aST) + nld * aST;
+        *at(v.MLD, p) = mld;
+        float dlt = s.dlt, dst = s.dst, rlt = s.rlt, rst = s.rst;
         const uint32_t REQ = (uint32_t)v.REQ;
+        float nmd = (quot((float)ms, col_max, inv_col) + quot((float)md, desc_max, inv_desc)) / 2.0f;
         if (fg) {
-            const float nmd = fmin_ref(1.0f, ((float)ms / col_max + (float)md / desc_max) / 2.0f +
-                                                 (float)(REQ - good) / (float)REQ);
-            dlt = dlt * (1.0f - aLT) + nmd * aLT;
-            dst = dst * (1.0f - aST) + nmd * aST;
-            rlt = rlt * (1.0f - aLT) + aLT;
-            rst = rst * (1.0f - aST) + aST;
+            nmd = fmin_ref(1.0f, nmd + (float)(REQ - good) / (float)REQ);
             raw = 255;
-        } else {
-            const float nmd = ((float)ms / col_max + (float)md / desc_max) / 2.0f;
-            dlt = dlt * (1.0f - aLT) + nmd * aLT;
-            dst = dst * (1.0f - aST) + nmd * aST;
-            rlt = rlt * (1.0f - aLT);
-            rst = rst * (1.0f - aST);
         }
-        G(v.DminLT)[p] = dlt;
-        G(v.DminST)[p] = dst;
-        G(v.RawLT)[p] = rlt;
-        G(v.RawST)[p] = rst;
-        rst_out = rst;
-        mld_out = mld;
+        dlt = dlt * (1.0f - aLT) + nmd * aLT;
+        dst = dst * (1.0f - aST) + nmd * aST;
+        rlt = rlt * (1.0f - aLT);
+        rst = rst * (1.0f - aST);
+        if (fg) {
+            rlt = rlt + aLT;
+            rst = rst + aST;
+        }
+        *at(v.DminLT, p) = dlt;
+        *at(v.DminST, p) = dst;
+        *at(v.RawLT, p) = rlt;
+        *at(v.RawST, p) = rst;
+        s.rst = rst;
+        s.mld = mld;
         const float lcap = v.sc->lower_cap, ucap = v.sc->upper_cap;
         const float mn = fmin_ref(dlt, dst), mx = fmax_ref(dlt, dst);
-        const bool last_fg = G(v.last_fg)[p] != 0;
-        float T = G(v.T)[p], V = G(v.V)[p], R = G(v.R)[p];
-        if (last_fg || (mn < 0.1f && raw)) {
-            if (T < ucap) T += 0.5f / (mx * V);
+        const bool last_fg = s.last_fg != 0;
+        float T = s.T, V = s.V, R = s.R;
+        // T += 0.5 / (mx * V) or T -= 0.25 * V / mx, one division for both
+        const bool up = last_fg || (mn < 0.1f && raw);
+        const float step = (up ? 0.5f : 0.25f * V) / (up ? mx * V : mx);
+        if (up) {
+            if (T < ucap) T += step;
         } else if (T > lcap) {
-            T -= 0.25f * V / mx;
+            T -= step;
         }
         if (T < lcap) T = lcap;
         else if (T > ucap) T = ucap;
-        if (mx > 0.1f && G(v.blinks)[p]) {
+        if (mx > 0.1f && s.blinks) {
             V += 1.0f;
         } else if (V > 0.1f) {
-            V -= last_fg ? 0.1f / 4 : unst_new ? 0.1f / 2 : 0.1f;
+            V -= last_fg ? 0.1f / 4 : unstable ? 0.1f / 2 : 0.1f;
             if (V < 0.1f) V = 0.1f;
         }
         const float base = 1.0f + mn * 2.0f;
@@ -1506,20 +1641,16 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, float& rst_out, float& m
             R -= 0.01f / V;
             if (R < 1.0f) R = 1.0f;
         }
-        G(v.T)[p] = T;
-        G(v.V)[p] = V;
-        G(v.R)[p] = R;
-        G(v.unstable)[p] = (uint8_t)unst_new;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            G(v.last_color)[(size_t)p * C + c] = (uint8_t)cur[c];
-            G(v.last_desc)[(size_t)p * C + c] = (uint16_t)intra[c];
-        }
+        *at(v.T, p) = T;
+        *at(v.V, p) = V;
+        *at(v.R, p) = R;
+        *at(v.unstable, p) = (uint8_t)unstable;
+        store_last<C>(v, p, cur, intra);
     }
-    const uint8_t cb = raw ^ G(v.last_raw)[p];
-    G(v.blinks)[p] = cb | G(v.last_raw_blink)[p];
-    G(v.last_raw_blink)[p] = cb;
-    G(v.last_raw)[p] = raw;  // this frame's raw mask from here on
+    const uint8_t cb = raw ^ s.last_raw;
+    *at(v.blinks, p) = cb | s.last_raw_blink;
+    *at(v.last_raw_blink, p) = cb;
+    *at(v.last_raw, p) = raw;  // this frame's raw mask from here on
     return examined;
 }
 
@@ -1527,116 +1658,126 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, float& rst_out, float& m
 // model update: every pixel of the inner rectangle gathers the writes aimed at its samples, in
 // the raster order of the writers; the last write of each slot wins (SUB:406-449, LOB:498-512).
 // ----------------------------------------------------------------------------------------------
-// SuBSENSE: the feedback maps of the thread's pixel are updated first, in the same pass
-// (they depend on the pixel alone), and the ghost test uses the new values from registers. LOBSTER: the raw
-// mask (LOB:496-497, :554-555) and the last colour frame (LOB:580) are written in the same pass.
+// The tile's 5x5 neighbourhood in LDS, a wavefront per row: records with the tests of a write folded into their
+// free bits (a writer is then one masked compare instead of two reads and four tests), and the writers' current
+// colours and intra descriptors (the values they write) as the rows' bytes.
+constexpr uint32_t kRecBg = 1u << 11;   // decided background
+constexpr uint32_t kRecFwd = 1u << 12;  // fwd_gate
+constexpr uint32_t kRecAny = 1u << 13;  // gate a or gate b
+template <int C>
+struct UpdateTile {
+    static constexpr int LW = TW + 4, LH = TH + 4;
+    static constexpr int DW = LW * 2 * C / 4;  // words of a descriptor row
+    uint32_t rec[LH][LW];
+    uint32_t desc[LH][DW];
+    FrameTile<C> px;
+};
+
+// SuBSENSE: the feedback maps of the thread's pixel are updated in the same pass (they depend on the pixel
+// alone), and the ghost test uses the new values from registers. LOBSTER: the raw mask (LOB:496-497,
+// :554-555) and the last colour frame (LOB:580) are written in the same pass.
 template <int C, int ALGO>
 LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
-    const uint8_t* frame = v.frame;
-    constexpr int LW = TW + 4, LH = TH + 4, NT = (LW * LH + TPB - 1) / TPB;
-    // the tile's 5x5 neighbourhood: records (tgt = kRecNone outside the image), "writer decided
-    // background", and the writers' current colour and intra descriptor (the values they write)
-    __shared__ uint32_t s_rec[LH][LW];
-    __shared__ uint8_t s_bg[LH][LW];
-    __shared__ uint8_t s_col[LH][LW * C];
-    __shared__ uint16_t s_desc[LH][LW * C];
+    using Tile = UpdateTile<C>;
+    __shared__ Tile t;
+    constexpr int LW = Tile::LW, LH = Tile::LH, DW = Tile::DW;
     const int ntx = (v.W + TW - 1) / TW;
-    const int tid = (int)bid;
-    const int x0 = (tid % ntx) * TW, y0 = (tid / ntx) * TH;
-    // neighbourhood loads first, into registers: their latency overlaps the feedback pass below
-    uint32_t t_rec[NT], t_col[NT][C], t_desc[NT][C];
-    uint8_t t_dec[NT];
+    const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
+    const int lx = (int)threadIdx.x % TW, ly = (int)threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
+    const bool inside = x < v.W && y < v.H;
+    const uint32_t p = inside ? (uint32_t)(y * v.W + x) : 0u;
+    auto stage_rec = [&](int r, int c) {
+        const int gx = x0 + c - 2, gy = y0 + r - 2;
+        uint32_t w = kRecNone;
+        if (gx >= 0 && gx < v.W && gy >= 0 && gy < v.H) {
+            const uint32_t q = (uint32_t)(gy * v.W + gx);
+            w = *at(v.rec, q);
+            w |= (*at(v.dec, q) == 0 ? kRecBg : 0u) | (fwd_gate(w) ? kRecFwd : 0u) |
+                 (rec_gate_a(w) || rec_gate_b(w) ? kRecAny : 0u);
+        }
+        t.rec[r][c] = w;
+    };
+    const int total = (int)v.npx * 2 * C;
 #pragma unroll
-    for (int k = 0; k < NT; ++k) {
-        const int i = (int)threadIdx.x + k * TPB;
-        const int ly = i / LW, lx = i % LW, gx = x0 + lx - 2, gy = y0 + ly - 2;
-        const bool in = i < LW * LH && gx >= 0 && gx < v.W && gy >= 0 && gy < v.H;
-        const size_t q = in ? (size_t)gy * v.W + gx : 0;
-        t_rec[k] = in ? G(v.rec)[q] : kRecNone;
-        t_dec[k] = G(v.dec)[q];
+    for (int k = 0; k < LH / 4; ++k) {
+        const int r = ly + 4 * k, gy = y0 + r - 2;
+        stage_rec(r, lx);
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            t_col[k][c] = G(frame)[q * C + c];
-            t_desc[k][c] = G(v.desc_cur)[q * C + c];
+        for (int j = 0; j < (DW + 63) / 64; ++j) {
+            const int w = lx + 64 * j;
+            if (w < DW)
+                t.desc[r][w] = gy >= 0 && gy < v.H
+                                   ? word_at((const uint8_t*)v.desc_cur, (gy * v.W + x0 - 2) * 2 * C + 4 * w, total)
+                                   : 0u;
         }
     }
-    const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
-    uint32_t nw = 0, examined = 0;
-    float rst = 0.f, mld = 1.f;
-    if constexpr (ALGO == kSuBSENSE)
-        if (x < v.W && y < v.H) examined = feedback_pixel<C>(v, (uint32_t)(y * v.W + x), rst, mld);
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-        const int i = (int)threadIdx.x + k * TPB;
-        if (i >= LW * LH) break;
-        const int ly2 = i / LW, lx2 = i % LW;
-        s_rec[ly2][lx2] = t_rec[k];
-        s_bg[ly2][lx2] = (rec_tgt(t_rec[k]) != kRecNone && t_dec[k] == 0) ? 1 : 0;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            s_col[ly2][lx2 * C + c] = (uint8_t)t_col[k][c];
-            s_desc[ly2][lx2 * C + c] = (uint16_t)t_desc[k][c];
-        }
-    }
+    if (threadIdx.x < 4 * LH) stage_rec((int)threadIdx.x / 4, TW + (int)threadIdx.x % 4);
+    load_frame_tile<C>(t.px, v.frame, v.W, v.H, x0, y0);
+    PxState<C> s;
+    if constexpr (ALGO == kSuBSENSE) load_px_state<C>(v, p, s);
     __syncthreads();
-    if constexpr (ALGO == kLOBSTER) {
-        if (x < v.W && y < v.H) {
-            const uint32_t p = (uint32_t)(y * v.W + x);
-            const bool roi = rec_tgt(s_rec[ly + 2][lx + 2]) != kRecNone;
-            G(v.last_raw)[p] = roi && !s_bg[ly + 2][lx + 2] ? 255 : 0;
-            if (roi) examined = G(v.mres)[p] >> 24;
+    auto colour = [&](int hx, int hy, int c) { return (uint32_t)t.px.px[FrameTile<C>::at(hx, hy, c)]; };
+    auto descriptor = [&](int hx, int hy, int c) { return (uint32_t)((const uint16_t*)t.desc[hy])[hx * C + c]; };
+    const uint32_t own = t.rec[ly + 2][lx + 2];
+    const bool own_bg = (own & kRecBg) != 0;
+    uint32_t nw = 0, examined = 0;
+    bool ghost_new = false;  // writers at or after p read p's updated maps (SUB:438-441)
+    if (inside) {
+        uint32_t cur[C], intra[C];
 #pragma unroll
-            for (int c = 0; c < C; ++c) G(v.last_color)[(size_t)p * C + c] = s_col[ly + 2][(lx + 2) * C + c];
+        for (int c = 0; c < C; ++c) {
+            cur[c] = colour(lx + 2, ly + 2, c);
+            intra[c] = descriptor(lx + 2, ly + 2, c);
+        }
+        if constexpr (ALGO == kSuBSENSE) {
+            examined = feedback_pixel<C>(v, p, s, cur, intra, rec_unstable(own), !own_bg);
+            ghost_new = s.rst > 0.995f && s.mld < 0.010f;
+        } else {
+            const bool roi = rec_tgt(own) != kRecNone;
+            *at(v.last_raw, p) = roi && !own_bg ? 255 : 0;
+            if (roi) examined = *at(v.mres, p) >> 24;
+#pragma unroll
+            for (int c = 0; c < C; ++c) *at(v.last_color, p * C + c) = (uint8_t)cur[c];
         }
     }
     if (x >= 2 && y >= 2 && x < v.W - 2 && y < v.H - 2) {
-        const uint32_t p = (uint32_t)(y * v.W + x);
-        // ghost test of writers at or after p reads p's updated maps (SUB:438-441)
-        bool ghost_new = false;
-        if constexpr (ALGO == kSuBSENSE) ghost_new = rst > 0.995f && mld < 0.010f;
-        // Writes landing on p, as bits in sequential order: writer j of the 5x5 window (raster
-        // order) owns bit 2j (its self update, j == 12 only) and bit 2j+1 (its diffusion into p).
-        uint64_t wm = 0;
+        // Writes landing on p, as bits in sequential order: writer j of the 5x5 window (raster order), bit j
+        // for j < 12 and j + 1 from 12 on; bit 12 is p's self update
+        const uint32_t late = 31u | kRecBg | (ghost_new ? kRecAny : 1u << 5);
+        constexpr uint32_t early = 31u | kRecBg | kRecFwd;
+        uint32_t wm = 0;
 #pragma unroll
         for (int j = 0; j < 25; ++j) {
             const int dy = j / 5 - 2, dx = j % 5 - 2;
-            const uint32_t r = s_rec[ly + 2 + dy][lx + 2 + dx];
-            const bool bg = s_bg[ly + 2 + dy][lx + 2 + dx] != 0;
-            if (j == 12 && rec_tgt(r) != kRecNone && (bg ? rec_self_bg(r) : (ALGO == kSuBSENSE && rec_self_fg(r))))
-                wm |= 1ull << (2 * j);
-            if (bg && rec_tgt(r) == (uint32_t)((2 - dy) * 5 + (2 - dx)) &&
-                (j < 12 ? fwd_gate(r) : (rec_gate_a(r) || (rec_gate_b(r) && ghost_new))))
-                wm |= 1ull << (2 * j + 1);
+            const uint32_t r = t.rec[ly + 2 + dy][lx + 2 + dx];
+            const uint32_t code = (uint32_t)((2 - dy) * 5 + (2 - dx));
+            const bool hit = j < 12 ? (r & early) == (code | kRecBg | kRecFwd) : ((r ^ ~31u) & late) == code;
+            wm |= hit ? 1u << (j < 12 ? j : j + 1) : 0u;
         }
-        // Visited from the last write back, so the first write seen for a slot is the one the
-        // sequential loop leaves in place; earlier writes to a written slot are skipped.
-        uint64_t done0 = 0, done1 = 0, done2 = 0, done3 = 0;  // slots already final (N <= 255)
-        nw = (uint32_t)__popcll(wm);
+        if (rec_tgt(own) != kRecNone && (own_bg ? rec_self_bg(own) : (ALGO == kSuBSENSE && rec_self_fg(own)))) wm |= 1u << 12;
+        nw = (uint32_t)popc(wm);
+        // in sequential order: a later write to the same slot overwrites the earlier one, as stores of one
+        // lane to one address do
         while (wm) {
-            const int b = 63 - __clzll((long long)wm);
-            wm &= ~(1ull << b);
-            const int j = b >> 1, dy = j / 5 - 2, dx = j % 5 - 2;
-            const uint32_t r = s_rec[ly + 2 + dy][lx + 2 + dx];
-            const uint32_t sl = (b & 1) ? rec_slot_diff(r) : rec_slot_self(r);
-            const uint64_t bit = 1ull << (sl & 63u);
-            const uint32_t word = sl >> 6;
-            const uint64_t dw = word == 0 ? done0 : word == 1 ? done1 : word == 2 ? done2 : done3;
-            if (dw & bit) continue;
-            if (word == 0) done0 |= bit;
-            else if (word == 1) done1 |= bit;
-            else if (word == 2) done2 |= bit;
-            else done3 |= bit;
+            const int b = __builtin_ctz(wm);
+            wm &= wm - 1u;
+            const int j = b < 12 ? b : b == 12 ? 12 : b - 1;
+            const int hy = ly + j / 5, hx = lx + j % 5;
+            const uint32_t r = t.rec[hy][hx];
+            const uint32_t sl = b == 12 ? rec_slot_self(r) : rec_slot_diff(r);
             uint32_t col[C], desc[C];
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                col[c] = s_col[ly + 2 + dy][(lx + 2 + dx) * C + c];
-                desc[c] = s_desc[ly + 2 + dy][(lx + 2 + dx) * C + c];
+                col[c] = colour(hx, hy, c);
+                desc[c] = descriptor(hx, hy, c);
             }
             store_sample<C>(v, sl, p, col, desc);
         }
     }
-    block_add<TPB>(nw, v.sc->wr_part);
-    block_add<TPB>(examined, v.sc->ex_part);  // workload counter (sum of k_p)
+    // workload counters: sample writes (w_p) and samples examined (k_p)
+    const uint32_t sums[2] = {nw, examined};
+    unsigned long long* const to[2] = {v.sc->wr_part, v.sc->ex_part};
+    block_add<TPB, 2>(sums, to);
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -2172,11 +2313,11 @@ LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
             for (int u = 0; u < 4 && gx + u < W; ++u) {
                 const size_t pu = p + u;
                 const uint8_t iu = (uint8_t)(inv >> (8 * u)), fu = (uint8_t)(fg >> (8 * u));
-                G(v.blinks)[pu] = (uint8_t)(G(v.blinks)[pu] & G(v.last_dil_inv)[pu] & iu);
-                G(v.last_dil_inv)[pu] = iu;
+                *at(v.blinks, pu) = (uint8_t)(*at(v.blinks, pu) & *at(v.last_dil_inv, pu) & iu);
+                *at(v.last_dil_inv, pu) = iu;
                 const double f = (double)fu;
-                G(v.FinLT)[pu] = (float)((double)G(v.FinLT)[pu] * alt + f * blt + 0.0);
-                G(v.FinST)[pu] = (float)((double)G(v.FinST)[pu] * ast + f * bst + 0.0);
+                *at(v.FinLT, pu) = (float)((double)*at(v.FinLT, pu) * alt + f * blt + 0.0);
+                *at(v.FinST, pu) = (float)((double)*at(v.FinST, pu) * ast + f * bst + 0.0);
                 if (out_mask) out_mask[pu] = fu;
             }
         }
@@ -2263,7 +2404,7 @@ LV_D void downsample_body(const View& v, uint32_t bid, uint32_t nblk) {
                 int sum = 0;
                 for (int yy = 0; yy < sy; ++yy)
                     for (int xx = 0; xx < sx; ++xx)
-                        sum += G(frame)[((size_t)(dy * sy + yy) * v.W + (dx * sx + xx)) * C + c];
+                        sum += *at(frame, ((dy * sy + yy) * v.W + (dx * sx + xx)) * C + c);
                 m = sat_u8((float)sum * (1.f / (float)(sx * sy)));
             } else {
                 const double sx = (double)v.W / v.dsW, sy = (double)v.H / v.dsH;
@@ -2273,7 +2414,7 @@ LV_D void downsample_body(const View& v, uint32_t bid, uint32_t nblk) {
                     const double wy = fmin((double)(yy + 1), ye) - fmax((double)yy, yb);
                     for (int xx = (int)xb; xx < v.W && (double)xx < xe; ++xx) {
                         const double wx = fmin((double)(xx + 1), xe) - fmax((double)xx, xb);
-                        acc += (double)G(frame)[((size_t)yy * v.W + xx) * C + c] * (wy * wx);
+                        acc += (double)*at(frame, (yy * v.W + xx) * C + c) * (wy * wx);
                     }
                 }
                 m = sat_u8((float)(acc / (sx * sy)));
@@ -2387,13 +2528,13 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int reset, fl
             uint32_t col[C], desc[C];
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                col[c] = G(v.last_color)[q * C + c];
+                col[c] = *at(v.last_color, q * C + c);
                 if constexpr (ALGO == kLOBSTER) {
                     uint32_t taps[4];
                     taps_from_global<C>(v.last_color, v.W, gx, gy, c, taps);
-                    desc[c] = lbsp_threshold_sad(taps, col[c], G(v.sc->lut)[col[c]]);
+                    desc[c] = lbsp_threshold_sad(taps, col[c], *at(v.sc->lut, col[c]));
                 } else {
-                    desc[c] = G(v.last_desc)[q * C + c];
+                    desc[c] = *at(v.last_desc, q * C + c);
                 }
             }
             uint64_t ra;
@@ -2404,15 +2545,15 @@ LV_D void refresh_body(const View& v, uint32_t bid, uint32_t nblk, int reset, fl
                 t.w1[i] = (uint32_t)(ra >> 32);
                 t.w2[i] = rb;
             }
-            t.ok[i] = force_fg || !G(v.last_fg)[q];
+            t.ok[i] = force_fg || !*at(v.last_fg, q);
         }
         __syncthreads();
         const int x = x0 + (int)threadIdx.x % TW, y = y0 + (int)threadIdx.x / TW;
         if (x >= v.W || y >= v.H) continue;
         const uint32_t p = (uint32_t)(y * v.W + x);
-        if (reset) G(v.T)[p] = 1.0f;
-        const bool in = G(v.roi)[p] != 0 && (force_fg || !G(v.last_fg)[p]);
-        const bool zero = outside && !G(v.roi)[p];
+        if (reset) *at(v.T, p) = 1.0f;
+        const bool in = *at(v.roi, p) != 0 && (force_fg || !*at(v.last_fg, p));
+        const bool zero = outside && !*at(v.roi, p);
         if (!in && !zero) continue;
         uint32_t d[4], slot = start;
         for (uint32_t j = 0; j < nref; ++j) {
@@ -2448,7 +2589,7 @@ LV_D void refresh_pending(const View& v, uint32_t bid, uint32_t nblk) {
 template <int C>
 LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
     __shared__ FrameTile<C> tile;
-    __shared__ uint8_t lut[256];
+    __shared__ alignas(4) uint8_t lut[256];
     const int ntx = (v.W + TW - 1) / TW;
     const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
     load_frame_tile<C>(tile, img, v.W, v.H, x0, y0);
@@ -2457,25 +2598,19 @@ LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
     const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
     if (x >= v.W || y >= v.H) return;
     const uint32_t p = (uint32_t)(y * v.W + x);
-    const bool roi = G(v.roi)[p] != 0, in = roi && x > 2 && y > 2 && x < v.W - 2 && y < v.H - 2;
+    const bool roi = *at(v.roi, p) != 0, in = roi && x > 2 && y > 2 && x < v.W - 2 && y < v.H - 2;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         uint32_t taps[4];
         taps_from_tile<C>(tile, lx, ly, c, taps);
-        const uint32_t ref = tile.px[((ly + 2) * FrameTile<C>::LW + (lx + 2)) * C + c];
-        G(v.last_desc)[(size_t)p * C + c] = (uint16_t)(in ? lbsp_threshold_sad(taps, ref, lut[ref]) : 0u);
-        G(v.last_color)[(size_t)p * C + c] = (uint8_t)(roi ? ref : 0u);
+        const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
+        *at(v.last_desc, p * C + c) = (uint16_t)(in ? lbsp_threshold_sad(taps, ref, lut[ref]) : 0u);
+        *at(v.last_color, p * C + c) = (uint8_t)(roi ? ref : 0u);
     }
 }
 
 // getBackgroundImage / getBackgroundDescriptorsImage (SUB:614-649): float sum of v/N in sample
-// order, then saturate_cast (round half to even). v/N is the IEEE quotient, from the correctly rounded
-// reciprocal with one residual correction (equal to the division for every v < 2^16 and N <= 255:
-// checked exhaustively), three operations where the division takes about ten.
-LV_HD float quot(float v, float n, float inv) {
-    const float q = v * inv;
-    return __builtin_fmaf(__builtin_fmaf(-q, n, v), inv, q);
-}
+// order, then saturate_cast (round half to even)
 template <int C, bool DESC>
 LV_D void background_body(const View& v, void* out, uint32_t bid) {
     const uint32_t p = bid * TPB + threadIdx.x;
@@ -2526,7 +2661,7 @@ __global__ void __launch_bounds__(TPB) k_lbsp_abs(const uint8_t* __restrict__ im
         if (in) {
             uint32_t taps[4];
             taps_from_tile<C>(tile, lx, ly, c, taps);
-            const uint32_t ref = tile.px[((ly + 2) * FrameTile<C>::LW + (lx + 2)) * C + c];
+            const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
             d = (uint16_t)(PACKED ? lbsp_threshold_packed(taps, ref, t) : lbsp_threshold_sad(taps, ref, t));
         }
         out[((size_t)y * W + x) * C + c] = d;
@@ -2606,7 +2741,7 @@ __global__ void __launch_bounds__(TPB) k_fixpoint(View v, uint32_t k, uint32_t c
 
 // the zones' closing and the frame-level cells beside the model update (SuBSENSE; nzone = ncell = 0 else)
 template <int C, int ALGO>
-__global__ void __launch_bounds__(TPB) k_update(View v, uint32_t nzone, uint32_t ncell) {
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7))) k_update(View v, uint32_t nzone, uint32_t ncell) {
     const uint32_t b = blockIdx.x, rest = gridDim.x - nzone - ncell;
     if constexpr (ALGO == kSuBSENSE) {
         if (b < nzone) {

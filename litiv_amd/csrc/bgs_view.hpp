@@ -20,6 +20,7 @@ struct View {
     float rel_lbsp;          // m_fRelLBSPThreshold
     uint32_t seed_lo, seed_hi, stream_id;
     int use3x3, median_k, lr_scaling, dsW, dsH;
+    uint32_t n_mul, n_shift; // draw / N = mulhi(draw, n_mul) >> n_shift for 31-bit draws, N > 1
     // per-step inputs
     const uint8_t* frame;    // current input frame, device W*H*C
     uint8_t* out_mask;       // optional device W*H output mask

@@ -143,3 +143,46 @@ def test_batch_model_reset(groups):
     for i in range(3):
         for name in SUB_STATE:
             assert np.array_equal(gpus[i].state(name), orcs[i].state(name)), (i, name)
+
+
+@pytest.mark.parametrize("algo,c", [(SUBSENSE, 3), (SUBSENSE, 1), (LOBSTER, 3), (LOBSTER, 1)])
+@pytest.mark.parametrize("w,h", [(5, 5), (6, 7), (63, 5), (65, 6), (67, 9), (131, 10)])
+def test_tile_rows_at_small_and_ragged_sizes(algo, c, w, h):
+    # tile rows are read in words at any alignment: frames whose rows and whole size are no multiple of a word,
+    # tiles with one to three columns
+    run_sequence(algo, flashing(w, h, c, 6, seed=w * h), lr=None if algo == SUBSENSE else 2.0)
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("c", [1, 3])
+def test_unaligned_device_frames(offset, c):
+    import torch
+
+    from test_gpu_parity import _pair
+    w, h = 77, 21
+    gpu, orc = _pair(SUBSENSE)
+    frames = flashing(w, h, c, 5, seed=offset)
+    gpu.initialize(frames[0])
+    orc.initialize(frames[0])
+    buf = torch.zeros(w * h * c + 8, dtype=torch.uint8, device="cuda")
+    mask = torch.zeros(w * h + 8, dtype=torch.uint8, device="cuda")
+    for f in frames:
+        buf[offset:offset + f.size].copy_(torch.from_numpy(f.reshape(-1)))
+        torch.cuda.synchronize()
+        gpu.apply_device(buf.data_ptr() + offset, mask.data_ptr() + offset)
+        gpu.synchronize()
+        m = mask.cpu().numpy()
+        assert np.array_equal(m[offset:offset + w * h].reshape(h, w), orc.apply(f))
+        assert not m[:offset].any() and not m[offset + w * h:].any()
+
+
+@pytest.mark.parametrize("lr", [1.0, 5.0, 4194303.5, 4194304.0, 4194304.5, 3e9, 1e12])
+@pytest.mark.parametrize("algo", [SUBSENSE, LOBSTER])
+def test_learning_rates_around_the_divisibility_range(algo, lr):
+    run_sequence(algo, flashing(90, 40, 1, 5), lr=lr)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 32, 33, 64, 65, 127, 128, 255])
+def test_sample_counts(n):
+    # the slot draw's reciprocal (powers of two and their neighbours), slots past 64
+    run_sequence(SUBSENSE, flashing(70, 30, 3, 5), bg_samples=n, required_bg_samples=min(n, 2), lr=1.0)
