@@ -133,6 +133,18 @@ LV_D gptr<T> at(T* base, I i) {
     return (gptr<T>)((gptr<const uint8_t>)base + (uint32_t)((uint32_t)i * (uint32_t)sizeof(T)));
 }
 
+// Stores element i unless every lane of the wavefront that is here holds the value already stored (old). Most of
+// the state of a settled background pixel does not change from frame to frame (raw averages at 0, v at its
+// floor, T at a cap, no blinks), and a row of 64 unchanged values need not be written; whole rows keep
+// the store's lines whole.
+template <typename T, typename I>
+LV_D void store_changed(T* base, I i, T value, T old) {
+    bool same;
+    if constexpr (sizeof(T) == 4) same = __builtin_bit_cast(uint32_t, value) == __builtin_bit_cast(uint32_t, old);
+    else same = value == old;
+    if (__ballot(!same) != 0ull) *at(base, i) = value;
+}
+
 // wavefront-local LDS exchange: the lanes' stores above are visible to the loads below
 LV_D void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1610,8 +1622,8 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, PxState<C>& s, const uin
         }
         *at(v.DminLT, p) = dlt;
         *at(v.DminST, p) = dst;
-        *at(v.RawLT, p) = rlt;
-        *at(v.RawST, p) = rst;
+        store_changed(v.RawLT, p, rlt, s.rlt);
+        store_changed(v.RawST, p, rst, s.rst);
         s.rst = rst;
         s.mld = mld;
         const float lcap = v.sc->lower_cap, ucap = v.sc->upper_cap;
@@ -1641,16 +1653,16 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, PxState<C>& s, const uin
             R -= 0.01f / V;
             if (R < 1.0f) R = 1.0f;
         }
-        *at(v.T, p) = T;
-        *at(v.V, p) = V;
-        *at(v.R, p) = R;
+        store_changed(v.T, p, T, s.T);
+        store_changed(v.V, p, V, s.V);
+        store_changed(v.R, p, R, s.R);
         *at(v.unstable, p) = (uint8_t)unstable;
         store_last<C>(v, p, cur, intra);
     }
     const uint8_t cb = raw ^ s.last_raw;
-    *at(v.blinks, p) = cb | s.last_raw_blink;
-    *at(v.last_raw_blink, p) = cb;
-    *at(v.last_raw, p) = raw;  // this frame's raw mask from here on
+    store_changed(v.blinks, p, (uint8_t)(cb | s.last_raw_blink), s.blinks);
+    store_changed(v.last_raw_blink, p, cb, s.last_raw_blink);
+    store_changed(v.last_raw, p, raw, s.last_raw);  // this frame's raw mask from here on
     return examined;
 }
 
@@ -2285,13 +2297,15 @@ LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
         const uint32_t inv = ~d, fg = s_fg[ly + H3][q + 1];
         const size_t p = (size_t)gy * W + gx;
         if ((W & 3) == 0) {
-            uint32_t* bl = (uint32_t*)(v.blinks + p);
-            uint32_t* ldi = (uint32_t*)(v.last_dil_inv + p);
-            *bl = *bl & *ldi & inv;
-            *ldi = inv;
-            float4* lt = (float4*)(v.FinLT + p);
-            float4* st = (float4*)(v.FinST + p);
-            float4 a = *lt, b = *st;
+            uint32_t* const bl = (uint32_t*)v.blinks;
+            uint32_t* const ldi = (uint32_t*)v.last_dil_inv;
+            const uint32_t w = (uint32_t)(p >> 2), bl0 = *at(bl, w), ldi0 = *at(ldi, w);
+            store_changed(bl, w, bl0 & ldi0 & inv, bl0);
+            store_changed(ldi, w, inv, ldi0);
+            typedef float f32x4 __attribute__((ext_vector_type(4)));
+            const gptr<f32x4> lt = at((f32x4*)v.FinLT, w), st = at((f32x4*)v.FinST, w);
+            const f32x4 a0 = *lt, b0 = *st;
+            f32x4 a = a0, b = b0;
             const double f0 = (double)(fg & 255u), f1 = (double)((fg >> 8) & 255u);
             const double f2 = (double)((fg >> 16) & 255u), f3 = (double)(fg >> 24);
             a.x = (float)((double)a.x * alt + f0 * blt + 0.0);
@@ -2302,8 +2316,13 @@ LV_D void dilate_final_body(const View& v, uint32_t bid, uint32_t nblk) {
             b.y = (float)((double)b.y * ast + f1 * bst + 0.0);
             b.z = (float)((double)b.z * ast + f2 * bst + 0.0);
             b.w = (float)((double)b.w * ast + f3 * bst + 0.0);
-            *lt = a;
-            *st = b;
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            auto differ = [](f32x4 m, f32x4 n) {
+                const u32x4 d = __builtin_bit_cast(u32x4, m) ^ __builtin_bit_cast(u32x4, n);
+                return (d.x | d.y | d.z | d.w) != 0u;
+            };
+            if (__ballot(differ(a, a0)) != 0ull) *lt = a;
+            if (__ballot(differ(b, b0)) != 0ull) *st = b;
             if (out_mask) {
                 if (((uintptr_t)out_mask & 3u) == 0) *(uint32_t*)(out_mask + p) = fg;  // caller's buffer
                 else
