@@ -42,7 +42,7 @@ LV_D int xcd_tile(int bid, int nblocks) {
 }
 
 LV_D uint32_t popc(uint32_t v) { return (uint32_t)__builtin_popcount(v); }
-LV_D uint32_t absdiff(uint32_t a, uint32_t b) { return a > b ? a - b : b - a; }
+LV_D uint32_t absdiff(uint32_t a, uint32_t b) { return __builtin_amdgcn_sad_u8(a, b, 0u); }  // of bytes
 LV_D float fmin_ref(float a, float b) { return (b < a) ? b : a; }  // std::min
 LV_D float fmax_ref(float a, float b) { return (a < b) ? b : a; }  // std::max
 
@@ -242,76 +242,134 @@ LV_D void store_sample(const View& v, uint32_t s, uint32_t p, const uint32_t col
     store_raw<C>(v, s, p, ra, rb);
 }
 
-// current colour and intra descriptor of pixel q (the value it writes into samples)
+// unaligned words of global memory (global accesses need no alignment on this device)
+struct __attribute__((packed, aligned(1))) UnalignedU32 {
+    uint32_t v;
+};
+struct __attribute__((packed, aligned(1))) UnalignedU16 {
+    uint16_t v;
+};
+template <typename W, typename T>
+LV_D auto peek(T* base, uint32_t byte) {
+    return ((gptr<const W>)((gptr<const uint8_t>)base + byte))->v;
+}
+template <typename W, typename T, typename V>
+LV_D void poke(T* base, uint32_t byte, V value) {
+    ((gptr<W>)((gptr<uint8_t>)base + byte))->v = value;
+}
+
+// intra descriptors of pixel q, RGB as {d0 | d1 << 16, d2}, grey as {d0}
 template <int C>
-LV_D void current_value(const View& v, const uint8_t* frame, uint32_t q, uint32_t col[C], uint32_t desc[C]) {
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        col[c] = *at(frame, q * C + c);
-        desc[c] = *at(v.desc_cur, q * C + c);
+struct DescWords {
+    uint32_t w0, w1;
+};
+template <int C>
+LV_D DescWords<C> load_desc(const uint16_t* desc, uint32_t q) {
+    if constexpr (C == 3) return {peek<UnalignedU32>(desc, 6u * q), peek<UnalignedU16>(desc, 6u * q + 4u)};
+    else return {*at(desc, q), 0u};
+}
+// a pixel's sample record (the value it writes into samples) from its packed colour and descriptor words
+template <int C>
+LV_D void record_of(uint32_t colour, DescWords<C> d, uint64_t& ra, uint32_t& rb) {
+    if constexpr (C == 3) {
+        ra = (uint64_t)d.w0 | ((uint64_t)(d.w1 | colour << 16) << 32);
+        rb = colour >> 16;
+    } else {
+        ra = (uint64_t)(d.w0 | colour << 16);
+        rb = 0;
     }
+}
+// the packed colour of pixel q from global memory (bytes, so that nothing past the frame is read)
+template <int C>
+LV_D uint32_t load_colour(const uint8_t* frame, uint32_t q) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) w |= (uint32_t)*at(frame, q * C + c) << (8 * c);
+    return w;
 }
 
 // ----------------------------------------------------------------------------------------------
 // LDS frame tile with a 2-pixel halo (the 5x5 LBSP patch)
 // ----------------------------------------------------------------------------------------------
-// Rows are loaded as 32-bit words from 8 (RGB) or 4 (grey) bytes left of the tile, so a halo row is 52 or 18
-// loads instead of 204 or 68 byte loads; PITCH is a row's bytes in LDS and OFF where its first pixel lies.
+// RGB: one word per pixel (c0 | c1 << 8 | c2 << 16), so a tap is one LDS read for the three channels and a
+// halo row one 3-byte-strided word load per pixel. Grey: bytes, loaded as words from 4 bytes left of the tile.
 template <int C>
-struct FrameTile {
-    static constexpr int LW = TW + 4, LH = TH + 4, OFF = 2, WORDS = C == 3 ? 52 : 18, PITCH = 4 * WORDS;
-    alignas(4) uint8_t px[LH * PITCH];
-    // byte of channel c of halo pixel (lx, ly)
-    static constexpr int at(int lx, int ly, int c) { return ly * PITCH + OFF + lx * C + c; }
+struct FrameTile;
+template <>
+struct FrameTile<3> {
+    static constexpr int LW = TW + 4, LH = TH + 4;
+    uint32_t px[LH][LW];
+};
+template <>
+struct FrameTile<1> {
+    static constexpr int LW = TW + 4, LH = TH + 4, OFF = 2, WORDS = 18, PITCH = 4 * WORDS;
+    alignas(4) uint8_t px[LH][PITCH];
 };
 
-// a 32-bit word at any byte offset of a buffer of `total` bytes (4 at least), zeros outside it. Global loads need
-// no alignment here; the last bytes of a buffer come from its last whole word.
-struct __attribute__((packed, aligned(1))) UnalignedU32 {
-    uint32_t v;
-};
+// a 32-bit word at any byte offset of a buffer of `total` bytes (4 at least), zeros outside it; the last bytes
+// of a buffer come from its last whole word
 LV_D uint32_t word_at(const uint8_t* base, int off, int total) {
     const int o = off < 0 ? 0 : off > total - 4 ? total - 4 : off;
-    const uint32_t w = ((gptr<const UnalignedU32>)((gptr<const uint8_t>)base + (uint32_t)o))->v;
+    const uint32_t w = peek<UnalignedU32>(base, (uint32_t)o);
     const int beyond = off - o;  // < 0: left of the buffer, > 0: bytes to drop
     return beyond < 0 || beyond > 3 ? 0u : w >> (8 * beyond);
 }
 
+// Pixels left and right of the image come out as whatever lies beside them in the frame: no pixel of the ROI
+// reaches them.
 template <int C>
 LV_D void load_frame_tile(FrameTile<C>& t, const uint8_t* frame, int W, int H, int x0, int y0) {
     using T = FrameTile<C>;
-    const int total = W * H * C, left = C == 3 ? 8 : 4;
-    if constexpr (C == 3) {  // a wavefront per row
-        const int l = (int)(threadIdx.x & 63u);
+    const int total = W * H * C;
+    if constexpr (C == 3) {
+        auto put = [&](int r, int c) {
+            const int gy = y0 + r - 2;
+            t.px[r][c] = gy >= 0 && gy < H ? word_at(frame, (gy * W + x0 + c - 2) * 3, total) & 0xFFFFFFu : 0u;
+        };
+        const int lx = (int)threadIdx.x % TW, ly = (int)threadIdx.x / TW;
 #pragma unroll
-        for (int k = 0; k < T::LH / 4; ++k) {
-            const int r = (int)(threadIdx.x >> 6) + 4 * k, gy = y0 + r - 2;
-            if (l < T::WORDS) {
-                const uint32_t w = gy >= 0 && gy < H ? word_at(frame, (gy * W + x0) * C - left + 4 * l, total) : 0u;
-                *(uint32_t*)&t.px[r * T::PITCH + 4 * l] = w;
-            }
-        }
+        for (int k = 0; k < T::LH / TH; ++k) put(ly + TH * k, lx);
+        if (threadIdx.x < 4u * T::LH) put((int)threadIdx.x / 4, TW + (int)threadIdx.x % 4);
     } else {
         const int r = (int)threadIdx.x / T::WORDS, l = (int)threadIdx.x % T::WORDS, gy = y0 + r - 2;
         if (r < T::LH) {
-            const uint32_t w = gy >= 0 && gy < H ? word_at(frame, gy * W + x0 - left + 4 * l, total) : 0u;
-            *(uint32_t*)&t.px[r * T::PITCH + 4 * l] = w;
+            const uint32_t w = gy >= 0 && gy < H ? word_at(frame, gy * W + x0 - 4 + 4 * l, total) : 0u;
+            *(uint32_t*)&t.px[r][4 * l] = w;
         }
     }
 }
 
-// packed 16 taps of channel c around tile-local (lx,ly) (centre coordinates, halo excluded)
-template <int C>
-LV_D void taps_from_tile(const FrameTile<C>& t, int lx, int ly, int c, uint32_t taps[4]) {
+// packed colour of halo pixel (hx, hy)
+LV_D uint32_t tile_colour(const FrameTile<3>& t, int hx, int hy) { return t.px[hy][hx]; }
+LV_D uint32_t tile_colour(const FrameTile<1>& t, int hx, int hy) { return t.px[hy][FrameTile<1>::OFF + hx]; }
+
+// packed 16 taps of every channel around tile-local (lx, ly) (centre coordinates, halo excluded). RGB: four
+// pixel words become three tap words by a byte transposition (seven v_perm; 16 LDS reads and 28 permutes
+// where single bytes took 48 reads and 36 shifts).
+LV_D void tile_taps(const FrameTile<3>& t, int lx, int ly, uint32_t (&taps)[3][4]) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        uint32_t q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] = t.px[ly + 2 + kLbspDY[4 * w + k]][lx + 2 + kLbspDX[4 * w + k]];
+        // v_perm_b32(hi, lo): bytes 0-3 select lo's, 4-7 hi's
+        const uint32_t a = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u);  // q0.0 q1.0 q0.1 q1.1
+        const uint32_t b = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u);
+        const uint32_t c = __builtin_amdgcn_perm(q[1], q[0], 0x0C0C0602u);  // q0.2 q1.2
+        const uint32_t d = __builtin_amdgcn_perm(q[3], q[2], 0x0C0C0602u);
+        taps[0][w] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        taps[1][w] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        taps[2][w] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+    }
+}
+LV_D void tile_taps(const FrameTile<1>& t, int lx, int ly, uint32_t (&taps)[1][4]) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         uint32_t acc = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int n = 4 * w + k;
-            acc |= (uint32_t)t.px[FrameTile<C>::at(lx + 2 + kLbspDX[n], ly + 2 + kLbspDY[n], c)] << (8 * k);
-        }
-        taps[w] = acc;
+        for (int k = 0; k < 4; ++k)
+            acc |= (uint32_t)t.px[ly + 2 + kLbspDY[4 * w + k]][FrameTile<1>::OFF + lx + 2 + kLbspDX[4 * w + k]] << (8 * k);
+        taps[0][w] = acc;
     }
 }
 
@@ -346,25 +404,24 @@ struct PxCtx {
     uint32_t t_col, t_desc;                // 1ch thresholds
 };
 
-LV_D uint32_t clamp_u32(uint64_t v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)v; }
-
-// SuBSENSE per-pixel thresholds from the previous unstable flag (SUB:355-359, 1ch :222-223)
+// SuBSENSE per-pixel thresholds from the previous unstable flag (SUB:355-359, 1ch :222-223). The reference
+// computes them in size_t; a threshold is only compared with distances of at most 765, so bounds that are
+// far above those (2^28 for the colour, 2^20 for the power of two) give the same tests in 32 bits: the
+// parameters are below 2^24, so nothing overflows.
 template <int C>
 LV_D void subsense_thresholds(const View& v, float R, uint32_t unst_old, PxCtx<C>& px) {
-    const float colf = R * (float)v.color_thr - (float)((uint64_t)(unst_old ? 0u : 1u) * (uint64_t)(v.color_thr / 5u));
-    uint64_t col = (uint64_t)colf;
-    const uint64_t shift = (uint64_t)floorf(R + 0.5f);
-    const uint64_t desc = (1ull << (shift & 63u)) + (uint64_t)v.desc_thr + (uint64_t)unst_old * (uint64_t)v.desc_thr;
+    const float colf = R * (float)v.color_thr - (unst_old ? 0.0f : (float)(v.color_thr / 5u));
+    const uint32_t col = (uint32_t)fminf(colf, 268435456.0f);
+    const uint32_t shift = (uint32_t)floorf(R + 0.5f) & 63u;
+    const uint32_t desc = (1u << (shift < 20u ? shift : 20u)) + v.desc_thr + unst_old * v.desc_thr;
     if constexpr (C == 1) {
-        col /= 2u;
-        px.t_col = clamp_u32(col);
-        px.t_desc = clamp_u32(desc);
+        px.t_col = col / 2u;
+        px.t_desc = desc;
         px.t_sc = px.t_tot_col = px.t_tot_desc = 0u;  // unused by the 1-channel test
     } else {
-        const uint64_t tot_col = col * 3u, tot_desc = desc * 3u;
-        px.t_sc = clamp_u32(tot_col / 2u);
-        px.t_tot_col = clamp_u32(tot_col);
-        px.t_tot_desc = clamp_u32(tot_desc);
+        px.t_tot_col = 3u * col;
+        px.t_tot_desc = 3u * desc;
+        px.t_sc = px.t_tot_col / 2u;
         px.t_col = px.t_desc = 0u;  // unused by the 3-channel test
     }
 }
@@ -458,6 +515,14 @@ LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col
 constexpr int kPredDX[12] = {-2, -1, 0, 1, 2, -2, -1, 0, 1, 2, -2, -1};
 constexpr int kPredDY[12] = {-2, -2, -2, -2, -2, -1, -1, -1, -1, -1, 0, 0};
 
+LV_D int pred_dx(uint32_t i) { return (int)(i % 5u) - 2; }
+LV_D int pred_dy(uint32_t i) { return (int)(i / 5u) - 2; }
+
+// free bits of a record that the tiles in LDS fold tests into
+constexpr uint32_t kRecBg = 1u << 11;   // decided background
+constexpr uint32_t kRecFwd = 1u << 12;  // fwd_gate
+constexpr uint32_t kRecAny = 1u << 13;  // gate a or gate b
+
 // static forward gate of a record whose target lies after the writer in raster order
 LV_D bool fwd_gate(uint32_t r) { return rec_gate_a(r) || (rec_gate_b(r) && rec_ghost_fwd(r)); }
 
@@ -482,10 +547,10 @@ LV_D ScanState scan_init() {
 // Overwritten slots of a pixel with their replacement values (the last applied writer's current
 // value), kept per thread in LDS so the sequential scan's loop carries only a slot bitmap: a sample
 // whose slot bit is set looks its slot up in the thread's entries. At most kRepl distinct slots;
-// pixels with more (very rare) go to the cooperative phase.
+// pixels with more (very rare) go to the fix point unmatched. w2 holds the record's last byte with the slot
+// above it.
 constexpr int kRepl = 4;
 struct ReplLds {
-    uint32_t slot[kRepl][TPB];
     uint32_t w0[kRepl][TPB], w1[kRepl][TPB], w2[kRepl][TPB];
 };
 
@@ -497,17 +562,15 @@ LV_D ReplLds& repl_lds() {
 
 template <int C>
 LV_D void raw_current(const View& v, const uint8_t* frame, uint32_t q, uint64_t& ra, uint32_t& rb) {
-    uint32_t col[C], desc[C];
-    current_value<C>(v, frame, q, col, desc);
-    encode_raw<C>(col, desc, ra, rb);
+    record_of<C>(load_colour<C>(frame, q), load_desc<C>(v.desc_cur, q), ra, rb);
 }
 
 // Fills the thread's entries from the applied writers, the latest in raster order first (it owns
 // its slot). Returns the slot bitmap (mod 64) and the entry count, or false beyond kRepl slots.
-// rec_of(i) is the update record of predecessor i.
-template <int C, typename RecOf>
-LV_D bool build_repl(const View& v, const uint8_t* frame, int x, int y, uint32_t applied, uint64_t& sbm, int& n,
-                     RecOf rec_of) {
+// rec_of(i) is the update record of predecessor i, colour_of(i, q) its packed colour.
+template <int C, typename RecOf, typename ColourOf>
+LV_D bool build_repl(const View& v, int x, int y, uint32_t applied, uint64_t& sbm, int& n, RecOf rec_of,
+                     ColourOf colour_of) {
     ReplLds& R = repl_lds();
     const int t = (int)threadIdx.x;
     sbm = 0;
@@ -515,20 +578,19 @@ LV_D bool build_repl(const View& v, const uint8_t* frame, int x, int y, uint32_t
     for (uint32_t m = applied; m;) {
         const int i = 31 - __builtin_clz(m);
         m &= ~(1u << i);
-        const uint32_t q = (uint32_t)((y + kPredDY[i]) * v.W + (x + kPredDX[i]));
+        const uint32_t q = (uint32_t)((y + pred_dy((uint32_t)i)) * v.W + (x + pred_dx((uint32_t)i)));
         const uint32_t sl = rec_slot_diff(rec_of(i));
         bool seen = false;
 #pragma unroll
-        for (int k = 0; k < kRepl; ++k) seen = seen || (k < n && R.slot[k][t] == sl);
+        for (int k = 0; k < kRepl; ++k) seen = seen || (k < n && R.w2[k][t] >> 8 == sl);
         if (seen) continue;
         if (n == kRepl) return false;
         uint64_t ra;
         uint32_t rb;
-        raw_current<C>(v, frame, q, ra, rb);
-        R.slot[n][t] = sl;
+        record_of<C>(colour_of(i, q), load_desc<C>(v.desc_cur, q), ra, rb);
         R.w0[n][t] = (uint32_t)ra;
         R.w1[n][t] = (uint32_t)(ra >> 32);
-        R.w2[n][t] = rb;
+        R.w2[n][t] = rb | sl << 8;
         sbm |= 1ull << (sl & 63u);
         ++n;
     }
@@ -548,7 +610,7 @@ LV_D void scan_batch(const uint8_t* lut, const PxCtx<C>& px, uint64_t sbm, int n
         uint32_t b = rb[j];
         if ((sbm >> (st.s & 63u)) & 1u) {
             for (int k = 0; k < nrep; ++k)
-                if (R.slot[k][t] == st.s) {
+                if (R.w2[k][t] >> 8 == st.s) {
                     a = (uint64_t)R.w0[k][t] | ((uint64_t)R.w1[k][t] << 32);
                     b = R.w2[k][t];
                     break;
@@ -724,14 +786,20 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
         } else {
             uint32_t pc = 0;
             uint32_t intra[C];
+            uint32_t taps[C][4];
+            tile_taps(tile, lx, ly, taps);
+            const uint32_t centre = tile_colour(tile, lx + 2, ly + 2);
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                uint32_t taps[4];
-                taps_from_tile<C>(tile, lx, ly, c, taps);
-                const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
-                intra[c] = lbsp_threshold_sad(taps, ref, lut[ref]);
-                *at(v.desc_cur, p * C + c) = (uint16_t)intra[c];
+                const uint32_t ref = (centre >> (8 * c)) & 255u;
+                intra[c] = lbsp_threshold_packed(taps[c], ref, lut[ref]);
                 pc += popc(intra[c]);
+            }
+            if constexpr (C == 3) {
+                poke<UnalignedU32>(v.desc_cur, 6u * p, intra[0] | intra[1 % C] << 16);
+                poke<UnalignedU16>(v.desc_cur, 6u * p + 4u, (uint16_t)intra[2 % C]);
+            } else {
+                *at(v.desc_cur, p) = (uint16_t)intra[0];
             }
             nz = pc >= (C == 1 ? 2u : 4u);
             const uint32_t frame_no = cur_frame(v);
@@ -790,53 +858,50 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     if constexpr (ALGO == kSuBSENSE) block_add<TPB>(nz ? 1u : 0u, v.sc->nz_part);
 }
 
-// a tile pixel's per-frame match inputs, loaded together with the tile and staged in LDS (the
-// regrouping of a tile's pixels moves them between threads after the tile barrier)
+// a pixel's per-frame match inputs, loaded together with the tile: intra descriptors of the current frame with
+// the ROI and the previous unstable flag above the last one, and R
 template <int C>
 struct PxIn {
-    uint16_t desc[C];  // intra descriptors of the current frame
-    uint8_t roi, unst;
+    uint32_t w[C == 3 ? 2 : 1];
     float R;
+    LV_D uint32_t desc(int c) const { return (w[c / 2] >> (16 * (c & 1))) & 0xFFFFu; }
+    LV_D bool roi() const { return (w[C == 3 ? 1 : 0] >> 16) & 1u; }
+    LV_D uint32_t unst() const { return w[C == 3 ? 1 : 0] >> 24; }
 };
 
 template <int C, int ALGO>
 LV_D PxIn<C> load_px_in(const View& v, uint32_t q, bool in) {
     PxIn<C> r;
-    r.roi = in ? *at(v.roi, q) : (uint8_t)0;
-#pragma unroll
-    for (int c = 0; c < C; ++c) r.desc[c] = *at(v.desc_cur, q * C + c);
+    const uint8_t roi = *at(v.roi, q);
+    const DescWords<C> d = load_desc<C>(v.desc_cur, q);
+    uint32_t unst = 0;
+    r.R = 0.f;
     if constexpr (ALGO == kSuBSENSE) {
         r.R = *at(v.R, q);
-        r.unst = *at(v.unstable, q);
+        unst = *at(v.unstable, q);
+    }
+    const uint32_t flags = (in && roi ? 1u << 16 : 0u) | unst << 24;
+    if constexpr (C == 3) {
+        r.w[0] = d.w0;
+        r.w[1 % (C == 3 ? 2 : 1)] = d.w1 | flags;
     } else {
-        r.R = 0.f;
-        r.unst = 0;
+        r.w[0] = d.w0 | flags;
     }
     return r;
 }
 
-// the match context from the LDS frame tile (5x5 window at win; the tile is complete behind a
-// workgroup barrier, so plain loads) and the staged inputs
-template <int C, int ALGO, int RS>
-LV_D void build_ctx_staged(const View& v, const uint8_t* win, const PxIn<C>& in, PxCtx<C>& px) {
+// the match context of tile-local pixel (lx, ly) from the LDS frame tile (complete behind a workgroup
+// barrier) and the inputs
+template <int C, int ALGO>
+LV_D void build_ctx_staged(const View& v, const FrameTile<C>& tile, int lx, int ly, const PxIn<C>& in, PxCtx<C>& px) {
+    const uint32_t centre = tile_colour(tile, lx + 2, ly + 2);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        px.cur[c] = win[2 * RS + 2 * C + c];
-        px.intra[c] = in.desc[c];
+        px.cur[c] = (centre >> (8 * c)) & 255u;
+        px.intra[c] = in.desc(c);
     }
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            uint32_t acc = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int n = 4 * w + k;
-                acc |= (uint32_t)win[(kLbspDY[n] + 2) * RS + (kLbspDX[n] + 2) * C + c] << (8 * k);
-            }
-            px.taps[c][w] = acc;
-        }
-    if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, in.R, in.unst, px);
+    tile_taps(tile, lx, ly, px.taps);
+    if constexpr (ALGO == kSuBSENSE) subsense_thresholds<C>(v, in.R, in.unst(), px);
     else lobster_thresholds<C>(v, px);
 }
 
@@ -845,57 +910,44 @@ LV_D void build_ctx_staged(const View& v, const uint8_t* win, const PxIn<C>& in,
 // to the continuation, which then reads it instead of rebuilding it from the frame.
 template <int C>
 LV_D void store_ctx(uint32_t* d, const PxCtx<C>& px) {
-    uint32_t w[kCtxWords] = {};
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[c * 4 + k] = px.taps[c][k];
-    uint32_t cur = 0;
-#pragma unroll
-    for (int c = 0; c < C; ++c) cur |= px.cur[c] << (8 * c);
-    w[12] = cur;
-    w[13] = px.intra[0] | (C == 3 ? px.intra[1 % C] << 16 : 0u);
-    w[14] = C == 3 ? px.intra[2 % C] : 0u;
-    w[15] = px.t_sc;
-    w[16] = px.t_tot_col;
-    w[17] = px.t_tot_desc;
-    w[18] = px.t_col;
-    w[19] = px.t_desc;
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const gptr<u32x4> q = (gptr<u32x4>)d;
 #pragma unroll
-    for (int k = 0; k < kCtxWords / 4; ++k) q[k] = u32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+    for (int c = 0; c < C; ++c) q[c] = u32x4{px.taps[c][0], px.taps[c][1], px.taps[c][2], px.taps[c][3]};
+    if constexpr (C == 3) {
+        q[3] = u32x4{px.cur[0] | px.cur[1] << 8 | px.cur[2] << 16, px.intra[0] | px.intra[1] << 16, px.intra[2], px.t_sc};
+        q[4] = u32x4{px.t_tot_col, px.t_tot_desc, px.t_col, px.t_desc};
+    } else {
+        q[3] = u32x4{px.cur[0], px.intra[0], 0u, px.t_sc};
+        q[4] = u32x4{px.t_tot_col, px.t_tot_desc, px.t_col, px.t_desc};
+    }
 }
 
 template <int C>
 LV_D void load_ctx(const uint32_t* d, PxCtx<C>& px) {
-    uint32_t w[kCtxWords];
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     const gptr<const u32x4> q = (gptr<const u32x4>)d;
 #pragma unroll
-    for (int k = 0; k < kCtxWords / 4; ++k) {
-        const u32x4 u = q[k];
-        w[4 * k] = u.x;
-        w[4 * k + 1] = u.y;
-        w[4 * k + 2] = u.z;
-        w[4 * k + 3] = u.w;
-    }
-#pragma unroll
     for (int c = 0; c < C; ++c) {
+        const u32x4 t = q[c];
+        px.taps[c][0] = t.x;
+        px.taps[c][1] = t.y;
+        px.taps[c][2] = t.z;
+        px.taps[c][3] = t.w;
+    }
+    const u32x4 a = q[3], b = q[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) px.taps[c][k] = w[c * 4 + k];
-        px.cur[c] = (w[12] >> (8 * c)) & 255u;
-    }
-    px.intra[0] = w[13] & 0xFFFFu;
+    for (int c = 0; c < C; ++c) px.cur[c] = (a.x >> (8 * c)) & 255u;
+    px.intra[0] = a.y & 0xFFFFu;
     if constexpr (C == 3) {
-        px.intra[1 % C] = w[13] >> 16;
-        px.intra[2 % C] = w[14];
+        px.intra[1 % C] = a.y >> 16;
+        px.intra[2 % C] = a.z;
     }
-    px.t_sc = w[15];
-    px.t_tot_col = w[16];
-    px.t_tot_desc = w[17];
-    px.t_col = w[18];
-    px.t_desc = w[19];
+    px.t_sc = a.w;
+    px.t_tot_col = b.x;
+    px.t_tot_desc = b.y;
+    px.t_col = b.z;
+    px.t_desc = b.w;
 }
 
 // the same context with the taps read from the frame in global memory
@@ -931,9 +983,6 @@ LV_D void build_ctx_global(const View& v, const uint8_t* frame, int x, int y, Px
 struct GroupLds {
     uint32_t taps[TPB / kGroup][12];
 };
-
-LV_D int pred_dx(uint32_t i) { return (int)(i % 5u) - 2; }
-LV_D int pred_dy(uint32_t i) { return (int)(i / 5u) - 2; }
 
 // Writers of p applied by the match: bit i of the result is set when predecessor i targets p with an
 // open forward gate and its decision is background (CURRENT: the decisions of the fix point, else those of
@@ -1063,22 +1112,30 @@ LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, c
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,
                       uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px, bool& push, uint32_t& target);
 
-// records and previous raw decisions of the raster-earlier part of a tile's 5x5 neighbourhood:
-// rows y0-2 .. y0+TH-1, columns x0-2 .. x0+TW+1
+// Records of the raster-earlier part of a tile's 5x5 neighbourhood (rows y0-2 .. y0+TH-1, columns x0-2 ..
+// x0+TW+1) with the guess (background in the previous frame) and the forward gate folded into free bits, so
+// that an applied writer is one masked compare.
 struct PredTile {
     static constexpr int LW = TW + 4, LH = TH + 2;
     uint32_t rec[LH][LW];
-    uint8_t guess[LH][LW];
 };
 
 LV_D void load_pred_tile(PredTile& t, const View& v, int x0, int y0) {
-    for (int i = threadIdx.x; i < PredTile::LW * PredTile::LH; i += TPB) {
-        const int ly = i / PredTile::LW, lx = i % PredTile::LW, gx = x0 + lx - 2, gy = y0 + ly - 2;
-        const bool in = gx >= 0 && gx < v.W && gy >= 0 && gy < v.H;
-        const size_t q = (size_t)gy * v.W + gx;
-        t.rec[ly][lx] = in ? *at(v.rec, q) : kRecNone;
-        t.guess[ly][lx] = in ? (*at(v.last_raw, q) ? 1 : 0) : 1;
-    }
+    auto put = [&](int r, int c) {
+        const int gx = x0 + c - 2, gy = y0 + r - 2;
+        uint32_t w = kRecNone;
+        if (gx >= 0 && gx < v.W && gy >= 0 && gy < v.H) {
+            const uint32_t q = (uint32_t)(gy * v.W + gx);
+            w = *at(v.rec, q);
+            w |= (*at(v.last_raw, q) == 0 ? kRecBg : 0u) | (fwd_gate(w) ? kRecFwd : 0u);
+        }
+        t.rec[r][c] = w;
+    };
+    const int lx = (int)threadIdx.x % TW, ly = (int)threadIdx.x / TW;
+    put(ly, lx);
+    if (ly < PredTile::LH - TH) put(ly + TH, lx);
+    else if (threadIdx.x >= TPB - 4u * PredTile::LH)  // the last columns, by the threads without a second row
+        put((TPB - 1 - (int)threadIdx.x) / 4, TW + (int)threadIdx.x % 4);
 }
 
 // candidate writers of tile-local pixel (lx,ly) whose guessed decision is background
@@ -1086,10 +1143,9 @@ LV_D uint32_t applied_writers_tile(const PredTile& t, int lx, int ly) {
     uint32_t m = 0;
 #pragma unroll
     for (int i = 0; i < 12; ++i) {
-        const int ty = ly + 2 + kPredDY[i], tx = lx + 2 + kPredDX[i];
-        const uint32_t r = t.rec[ty][tx];
+        const uint32_t r = t.rec[ly + 2 + kPredDY[i]][lx + 2 + kPredDX[i]];
         const uint32_t code = (uint32_t)((2 - kPredDY[i]) * 5 + (2 - kPredDX[i]));
-        if (rec_tgt(r) == code && fwd_gate(r) && t.guess[ty][tx] == 0) m |= 1u << i;
+        m |= (r & (31u | kRecBg | kRecFwd)) == (code | kRecBg | kRecFwd) ? 1u << i : 0u;
     }
     return m;
 }
@@ -1105,12 +1161,6 @@ struct MatchLds {
     } tile;
     PredTile pred;
     alignas(4) uint8_t lut[256];
-    uint16_t perm[TPB];
-    uint32_t nfg[TPB / 64];
-    union {
-        PxIn<CMAX> big[TPB];
-        PxIn<1> c1[TPB];
-    } in;
 };
 
 template <int CMAX>
@@ -1125,12 +1175,6 @@ LV_D FrameTile<C>& tile_of(MatchLds<CMAX>& m) {
     else return m.tile.c1;
 }
 
-template <int C, int CMAX>
-LV_D PxIn<C>* px_in_of(MatchLds<CMAX>& m) {
-    if constexpr (C == CMAX) return m.in.big;
-    else return m.in.c1;
-}
-
 template <int C, int ALGO, int KF, int CMAX = C>
 LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
     static_assert(C == CMAX || C == 1, "a match instantiation shares the LDS of CMAX channels");
@@ -1141,48 +1185,23 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
     PredTile& pred = L.pred;
     uint8_t* lut = L.lut;
     const int ntx = (v.W + TW - 1) / TW;
-    const int tid = (int)bid;
-    const int x0 = (tid % ntx) * TW, y0 = (tid / ntx) * TH;
-    uint16_t* s_perm = L.perm;
-    uint32_t* s_nfg = L.nfg;
-    PxIn<C>* s_in = px_in_of<C>(L);
-    // this thread's tile pixel before the regrouping: its inputs are loaded alongside the tile
-    const int ox = x0 + (int)threadIdx.x % TW, oy = y0 + (int)threadIdx.x / TW;
-    const bool oin = ox < v.W && oy < v.H;
-    const PxIn<C> pin = load_px_in<C, ALGO>(v, oin ? (uint32_t)(oy * v.W + ox) : 0u, oin);
+    const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
+    // The tile's pixels stay with their threads: the scan is cut after a few samples, so foreground pixels
+    // cost a wavefront little, and gathering them into shared wavefronts (two barriers, the inputs through LDS)
+    // no longer pays (1391 -> 1344 us for a batch of 64 without it, 250 -> 240 us at 3840x2160).
+    const int lx = (int)threadIdx.x % TW, ly = (int)threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
+    const bool inside = x < v.W && y < v.H;
+    const uint32_t p = (uint32_t)(y * v.W + x);
+    const PxIn<C> in = load_px_in<C, ALGO>(v, inside ? p : 0u, inside);
     load_frame_tile<C>(tile, frame, v.W, v.H, x0, y0);
     load_pred_tile(pred, v, x0, y0);
     load_lut(lut, v.sc);
-    s_in[threadIdx.x] = pin;
     __syncthreads();
-    // A wavefront scans as long as its slowest lane, and foreground pixels scan every sample: the
-    // tile's pixels are regrouped so those that were foreground in the previous frame share
-    // wavefronts (stable order within each group). Each pixel's match depends on the tile data only.
-    {
-        const int t = (int)threadIdx.x;
-        const bool likely_fg = oin && pred.guess[t / TW + 2][t % TW + 2] != 0 && pin.roi;
-        const unsigned long long bal = __ballot(likely_fg);
-        const int lane = t & 63, wave = t >> 6;
-        if (lane == 0) s_nfg[wave] = (uint32_t)__popcll(bal);
-        __syncthreads();
-        uint32_t fg_before = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull)), nfg = 0;
-        for (int w = 0; w < TPB / 64; ++w) {
-            fg_before += w < wave ? s_nfg[w] : 0u;
-            nfg += s_nfg[w];
-        }
-        const uint32_t pos = likely_fg ? (uint32_t)TPB - nfg + fg_before : (uint32_t)t - fg_before;
-        s_perm[pos] = (uint16_t)t;
-        __syncthreads();
-    }
-    const int src = s_perm[threadIdx.x];
-    const int lx = src % TW, ly = src / TW, x = x0 + lx, y = y0 + ly;
-    const uint32_t p = (uint32_t)(y * v.W + x);
     uint32_t examined = 0;
     bool cont = false, push = false;
     uint32_t target = 0;
-    const PxIn<C> in = s_in[src];
-    PxCtx<C> px;
-    if (x < v.W && y < v.H && in.roi)
+    PxCtx<C> px{};
+    if (in.roi())
         cont = !match_pixel<C, ALGO, KF>(v, frame, lut, tile, pred, in, lx, ly, x, y, p, seq_limit, examined, px, push,
                                          target);
     // unfinished pixels go to the continuation with their context: one atomic per wavefront, on
@@ -1220,18 +1239,20 @@ LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, c
     // more than kRepl overwritten slots (very rare): the pixel keeps its guess for now and goes to the first
     // fix-point worklist itself, where a group matches it against any number of writers.
     // The replacements are gathered before the context is built, so the two are not live together.
-    auto rec_of = [&](int i) { return pred.rec[ly + 2 + kPredDY[i]][lx + 2 + kPredDX[i]]; };
-    const uint8_t guess = pred.guess[ly + 2][lx + 2];
-    const bool fits = build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
+    auto rec_of = [&](int i) { return pred.rec[ly + 2 + pred_dy((uint32_t)i)][lx + 2 + pred_dx((uint32_t)i)]; };
+    auto colour_of = [&](int i, uint32_t) { return tile_colour(tile, lx + 2 + pred_dx((uint32_t)i), ly + 2 + pred_dy((uint32_t)i)); };
+    const uint32_t own = pred.rec[ly + 2][lx + 2];
+    const uint8_t guess = (own & kRecBg) ? 0 : 1;
+    const bool fits = build_repl<C>(v, x, y, applied, sbm, nrep, rec_of, colour_of);
     const uint32_t limit = !fits ? 0u : seq_limit < N ? seq_limit : N;
-    build_ctx_staged<C, ALGO, FrameTile<C>::PITCH>(v, &tile.px[FrameTile<C>::at(lx, ly, 0)], in, px);
-    scan_seq<C, ALGO, FrameTile<C>::PITCH, KF>(v, lut, px, x, y, sbm, nrep, st, limit);
+    build_ctx_staged<C, ALGO>(v, tile, lx, ly, in, px);
+    scan_seq<C, ALGO, 1, KF>(v, lut, px, x, y, sbm, nrep, st, limit);
     examined = st.s;
     *at(v.mres, p) = pack_state(st);
     if (fits && st.good < (uint32_t)v.REQ && st.s < N) return false;
     const uint8_t fg = !fits ? guess : st.good < (uint32_t)v.REQ ? 1 : 0;
     *at(v.dec, p) = fg;
-    push = fg != guess && forward_target(v, pred.rec[ly + 2][lx + 2], x, y, target);
+    push = fg != guess && forward_target(v, own, x, y, target);
     if (!fits) {
         push = true;
         target = p;
@@ -1304,9 +1325,10 @@ LV_D void match_seq_lanes(const View& v, const uint8_t* lut, const uint32_t* s_p
         const uint32_t applied = applied_writers_global(v, x, y);
         uint64_t sbm;
         int nrep;
-        auto rec_of = [&](int i) { return *at(v.rec, (y + kPredDY[i]) * v.W + (x + kPredDX[i])); };
+        auto rec_of = [&](int i) { return *at(v.rec, (y + pred_dy((uint32_t)i)) * v.W + (x + pred_dx((uint32_t)i))); };
+        auto colour_of = [&](int, uint32_t q) { return load_colour<C>(frame, q); };
         // at most kRepl slots: phase A keeps the others (same writers, same guesses)
-        (void)build_repl<C>(v, frame, x, y, applied, sbm, nrep, rec_of);
+        (void)build_repl<C>(v, x, y, applied, sbm, nrep, rec_of, colour_of);
         ScanState st = unpack_state(*at(v.mres, p));
         const uint32_t s0 = st.s;
         scan_seq<C, ALGO, 0, KF>(v, lut, px, x, y, sbm, nrep, st, (uint32_t)v.N);
@@ -1527,18 +1549,6 @@ struct PxState {
     uint32_t mres;
     uint8_t roi, last_fg, blinks, last_raw, last_raw_blink;
 };
-struct __attribute__((packed, aligned(1))) UnalignedU16 {
-    uint16_t v;
-};
-template <typename W, typename T>
-LV_D auto peek(T* base, uint32_t byte) {
-    return ((gptr<const W>)((gptr<const uint8_t>)base + byte))->v;
-}
-template <typename W, typename T, typename V>
-LV_D void poke(T* base, uint32_t byte, V value) {
-    ((gptr<W>)((gptr<uint8_t>)base + byte))->v = value;
-}
-
 template <int C>
 LV_D void load_px_state(const View& v, uint32_t p, PxState<C>& s) {
     s.roi = *at(v.roi, p);
@@ -1673,9 +1683,6 @@ LV_D uint32_t feedback_pixel(const View& v, uint32_t p, PxState<C>& s, const uin
 // The tile's 5x5 neighbourhood in LDS, a wavefront per row: records with the tests of a write folded into their
 // free bits (a writer is then one masked compare instead of two reads and four tests), and the writers' current
 // colours and intra descriptors (the values they write) as the rows' bytes.
-constexpr uint32_t kRecBg = 1u << 11;   // decided background
-constexpr uint32_t kRecFwd = 1u << 12;  // fwd_gate
-constexpr uint32_t kRecAny = 1u << 13;  // gate a or gate b
 template <int C>
 struct UpdateTile {
     static constexpr int LW = TW + 4, LH = TH + 4;
@@ -1728,7 +1735,7 @@ LV_D void update_body(const View& v, uint32_t bid, uint32_t nblk) {
     PxState<C> s;
     if constexpr (ALGO == kSuBSENSE) load_px_state<C>(v, p, s);
     __syncthreads();
-    auto colour = [&](int hx, int hy, int c) { return (uint32_t)t.px.px[FrameTile<C>::at(hx, hy, c)]; };
+    auto colour = [&](int hx, int hy, int c) { return (tile_colour(t.px, hx, hy) >> (8 * c)) & 255u; };
     auto descriptor = [&](int hx, int hy, int c) { return (uint32_t)((const uint16_t*)t.desc[hy])[hx * C + c]; };
     const uint32_t own = t.rec[ly + 2][lx + 2];
     const bool own_bg = (own & kRecBg) != 0;
@@ -2618,12 +2625,13 @@ LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
     if (x >= v.W || y >= v.H) return;
     const uint32_t p = (uint32_t)(y * v.W + x);
     const bool roi = *at(v.roi, p) != 0, in = roi && x > 2 && y > 2 && x < v.W - 2 && y < v.H - 2;
+    uint32_t taps[C][4];
+    tile_taps(tile, lx, ly, taps);
+    const uint32_t centre = tile_colour(tile, lx + 2, ly + 2);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        uint32_t taps[4];
-        taps_from_tile<C>(tile, lx, ly, c, taps);
-        const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
-        *at(v.last_desc, p * C + c) = (uint16_t)(in ? lbsp_threshold_sad(taps, ref, lut[ref]) : 0u);
+        const uint32_t ref = (centre >> (8 * c)) & 255u;
+        *at(v.last_desc, p * C + c) = (uint16_t)(in ? lbsp_threshold_packed(taps[c], ref, lut[ref]) : 0u);
         *at(v.last_color, p * C + c) = (uint8_t)(roi ? ref : 0u);
     }
 }
@@ -2674,15 +2682,14 @@ __global__ void __launch_bounds__(TPB) k_lbsp_abs(const uint8_t* __restrict__ im
     const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
     if (x >= W || y >= H) return;
     const bool in = x >= 2 && y >= 2 && x < W - 2 && y < H - 2;
+    uint32_t taps[C][4];
+    tile_taps(tile, lx, ly, taps);
+    const uint32_t centre = tile_colour(tile, lx + 2, ly + 2);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
+        const uint32_t ref = (centre >> (8 * c)) & 255u;
         uint16_t d = 0;
-        if (in) {
-            uint32_t taps[4];
-            taps_from_tile<C>(tile, lx, ly, c, taps);
-            const uint32_t ref = tile.px[FrameTile<C>::at(lx + 2, ly + 2, c)];
-            d = (uint16_t)(PACKED ? lbsp_threshold_packed(taps, ref, t) : lbsp_threshold_sad(taps, ref, t));
-        }
+        if (in) d = (uint16_t)(PACKED ? lbsp_threshold_packed(taps[c], ref, t) : lbsp_threshold_sad(taps[c], ref, t));
         out[((size_t)y * W + x) * C + c] = d;
     }
 }
@@ -2744,8 +2751,8 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
 
 template <int C, int ALGO>
 __global__ void __launch_bounds__(TPB) k_describe(View v) { describe_body<C, ALGO>(v, LV_SINGLE_BID); }
-// occupancy 6 (at most 80 VGPRs, 26 KB of LDS per 256-thread block) fits both fetch depths without spilling
-#define LV_MATCH_WAVES(KF) __attribute__((amdgpu_waves_per_eu(6)))
+// occupancy 7 (at most 72 VGPRs) fits both fetch depths without spilling
+#define LV_MATCH_WAVES(KF) __attribute__((amdgpu_waves_per_eu(7)))
 template <int C, int ALGO, int KF>
 __global__ void __launch_bounds__(TPB) LV_MATCH_WAVES(KF) k_match(View v) { match_body<C, ALGO, KF>(v, LV_SINGLE_BID); }
 // phase B holds 80 VGPRs at occupancy 6 as well
