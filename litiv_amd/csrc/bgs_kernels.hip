@@ -1812,6 +1812,10 @@ constexpr int PW = 64, PH = 16;  // post-processing tile; 256 threads x 4 pixels
 // zone, and components inside it, which are holes. The border components of all zones are joined
 // across zone edges by union-find; a border component is outside iff its root is the root of the
 // component holding pixel (0,0).
+// Each kernel is bound by one wavefront's chain of rounds, not by memory, so a round's lane shifts are DPP moves
+// and a zone row comes in four loads. Shifts through the LDS crossbar and byte loads with a ballot per row: the
+// update launch that holds the closing at 320x240 26.9 -> 9.2 us; linking 39.9 -> 26.1 us and holes 10.1 -> 6.5 us
+// at 3840x2160; the holes of 64 mixed streams 20.6 -> 12.9 us.
 constexpr int ZS = 64;                  // zone side
 constexpr int ZPB = TPB / 64;           // zones per block, one per wavefront
 constexpr uint32_t kZoneComps = 128;    // border components per zone (at most 126 of 252 pixels)
@@ -1823,13 +1827,38 @@ LV_D uint64_t lane_bcast(uint64_t x, int l) {
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
 }
-LV_D uint64_t from_lane_above(uint64_t x, int d, int lane) {  // lane - d, 0 for the first d lanes
-    const uint64_t r = __shfl_up(x, (unsigned)d, 64);
-    return lane >= d ? r : 0ull;
+// lane - N (SHR) or lane + N (SHL) within the rows of 16 lanes, `fill` past the row's end, as DPP moves: a shift
+// through the LDS crossbar takes an order of magnitude longer, and a flood is a chain of them
+template <int CTRL, int ROWS = 0xf>
+LV_D uint64_t dpp64(uint64_t x, uint32_t fill) {
+    const int lo = __builtin_amdgcn_update_dpp((int)fill, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)fill, (int)(uint32_t)(x >> 32), CTRL, ROWS, 0xf, false);
+    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
 }
-LV_D uint64_t from_lane_below(uint64_t x, int d, int lane) {  // lane + d, 0 for the last d lanes
-    const uint64_t r = __shfl_down(x, (unsigned)d, 64);
-    return lane + d < 64 ? r : 0ull;
+constexpr int kRowShr = 0x110, kRowShl = 0x100, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
+// What the column fills of a zone need of its pixels z (lane y holds row y), computed once per zone: products
+// of z over the window each scan step covers. Down the rows: in-row shifts of 1, 2, 4, 8 lanes, then from the
+// last lane of the row before (broadcast 15) and of the first half (broadcast 31). Up the rows: the same shifts
+// the other way, then from the first lane of the row after, row by row.
+struct ColumnWindows {
+    uint64_t z, d1, d2, d4, d15, d31, u1, u2, u4, u[3];
+};
+LV_D ColumnWindows column_windows(uint64_t z, int lane) {
+    ColumnWindows w;
+    w.z = z;
+    w.d1 = z & dpp64<kRowShr + 1>(z, ~0u);
+    w.d2 = w.d1 & dpp64<kRowShr + 2>(w.d1, ~0u);
+    w.d4 = w.d2 & dpp64<kRowShr + 4>(w.d2, ~0u);
+    w.d15 = w.d4 & dpp64<kRowShr + 8>(w.d4, ~0u);  // from the row's first lane to this one
+    w.d31 = w.d15 & dpp64<kRowBcast15, 0xa>(w.d15, ~0u);
+    w.u1 = z & dpp64<kRowShl + 1>(z, ~0u);
+    w.u2 = w.u1 & dpp64<kRowShl + 2>(w.u1, ~0u);
+    w.u4 = w.u2 & dpp64<kRowShl + 4>(w.u2, ~0u);
+    const uint64_t u15 = w.u4 & dpp64<kRowShl + 8>(w.u4, ~0u);  // from this lane to the row's last one
+#pragma unroll
+    for (int r = 0; r < 3; ++r) w.u[r] = (lane >> 4) == r ? u15 : 0ull;
+    return w;
 }
 
 // the runs of z along the row that hold a bit of s (s within z). Adding s to z carries through
@@ -1840,33 +1869,62 @@ LV_D uint64_t fill_row(uint64_t z, uint64_t zr, uint64_t s) {
     const uint64_t ur = brev64(up);
     return brev64((zr & ~(zr + ur)) | ur);
 }
-// the runs of z down and up the columns that hold a bit of s: segmented OR scans over the lanes,
-// g = reached at this row from the rows above within the window, p = window all in z
-LV_D uint64_t fill_cols(uint64_t z, uint64_t s, int lane) {
-    uint64_t g = s, p = z;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t gu = from_lane_above(g, d, lane), pu = from_lane_above(p, d, lane);
-        g |= p & gu;
-        p &= pu;
-    }
-    p = z;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t gd = from_lane_below(g, d, lane), pd = from_lane_below(p, d, lane);
-        g |= p & gd;
-        p &= pd;
-    }
+// the runs of z down and up the columns that hold a bit of s: segmented OR scans over the lanes
+LV_D uint64_t fill_cols(const ColumnWindows& w, uint64_t g) {
+    g |= w.z & dpp64<kRowShr + 1>(g, 0u);
+    g |= w.d1 & dpp64<kRowShr + 2>(g, 0u);
+    g |= w.d2 & dpp64<kRowShr + 4>(g, 0u);
+    g |= w.d4 & dpp64<kRowShr + 8>(g, 0u);
+    g |= w.d15 & dpp64<kRowBcast15, 0xa>(g, 0u);
+    g |= w.d31 & dpp64<kRowBcast31, 0xc>(g, 0u);
+    g |= w.z & dpp64<kRowShl + 1>(g, 0u);
+    g |= w.u1 & dpp64<kRowShl + 2>(g, 0u);
+    g |= w.u2 & dpp64<kRowShl + 4>(g, 0u);
+    g |= w.u4 & dpp64<kRowShl + 8>(g, 0u);
+    g |= w.u[2] & lane_bcast(g, 48);
+    g |= w.u[1] & lane_bcast(g, 32);
+    g |= w.u[0] & lane_bcast(g, 16);
     return g;
 }
 // the 4-connected components of z holding a bit of s; each round adds at least one bit or ends
-LV_D uint64_t flood(uint64_t z, uint64_t zr, uint64_t s, int lane) {
-    uint64_t f = s & z;
+LV_D uint64_t flood(const ColumnWindows& w, uint64_t zr, uint64_t s) {
+    uint64_t f = s & w.z;
     while (true) {
-        const uint64_t g = fill_cols(z, fill_row(z, zr, f), lane);
+        const uint64_t g = fill_cols(w, fill_row(w.z, zr, f));
         if (__ballot(g != f) == 0ull) return g;
         f = g;
     }
+}
+
+// The 64 bytes of a row from column x0 on as bits (set: not 0), zeros outside the image. Four 16-byte loads in
+// place of 64 ballots over single bytes; bit 7 of (b & 127) + 127 | b tells whether byte b is set, and one product
+// gathers the four bits of a word (bit 24 + i of the product is byte i's).
+LV_D uint64_t mask_row(const uint8_t* m, int W, int H, int x0, int gy) {
+    if (gy < 0 || gy >= H) return 0ull;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    struct __attribute__((packed, aligned(1))) Quad {
+        u32x4 v;
+    };
+    const int off = gy * W + x0, total = W * H;
+    uint32_t q[16];
+    if (off + 64 <= total) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32x4 t = peek<Quad>(m, (uint32_t)(off + 16 * k));
+            q[4 * k] = t.x, q[4 * k + 1] = t.y, q[4 * k + 2] = t.z, q[4 * k + 3] = t.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) q[k] = word_at(m, off + 4 * k, total);
+    }
+    uint32_t b[2] = {0u, 0u};
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const uint32_t nz = ((((q[k] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | q[k]) >> 7) & 0x01010101u;
+        b[k >> 3] |= ((nz * 0x01020408u) >> 24 & 15u) << (4 * (k & 7));
+    }
+    const uint64_t bits = ((uint64_t)b[1] << 32) | b[0];
+    return W - x0 >= ZS ? bits : bits & ((1ull << (W - x0)) - 1ull);
 }
 
 // raw bits of columns x0-2, x0-1, x0+64, x0+65 of row gy (bits 0..3)
@@ -1902,18 +1960,9 @@ LV_D void zone_close_body(const View& v, uint32_t bid, uint32_t nblk) {
     // the raw mask is the decisions (zero outside the ROI): they are final before the model update, so
     // this runs beside it
     const uint8_t* raw = v.dec;
-    // raw rows y0-2+r as 64-bit masks: lane = column for the loads, one ballot per row; lane y
-    // keeps row y, lanes 0..3 also rows 64..67
-    const int gx = x0 + lane;
-    uint64_t c0 = 0, c1 = 0;
-#pragma unroll 17
-    for (int r = 0; r < ZS + 4; ++r) {
-        const int gy = y0 - 2 + r;
-        const uint8_t b = (gx < W && gy >= 0 && gy < H) ? raw[(size_t)gy * (size_t)W + gx] : (uint8_t)0;
-        const uint64_t m = __ballot(b != 0);
-        if (r < ZS) c0 = lane == r ? m : c0;
-        else c1 = lane == r - ZS ? m : c1;
-    }
+    // raw rows y0-2 .. y0+65 as 64-bit masks: lane y has row y, lanes 0..3 also rows 64..67
+    const uint64_t c0 = mask_row(raw, W, H, x0, y0 - 2 + lane);
+    const uint64_t c1 = lane < 4 ? mask_row(raw, W, H, x0, y0 - 2 + ZS + lane) : 0ull;
     const uint32_t h0 = raw_halo(raw, W, H, x0, y0 - 2 + lane);
     const uint32_t h1 = lane < 4 ? raw_halo(raw, W, H, x0, y0 - 2 + ZS + lane) : 0u;
     {
@@ -1955,6 +2004,7 @@ LV_D void zone_close_body(const View& v, uint32_t bid, uint32_t nblk) {
     v.zbits[(size_t)z * ZS + lane] = zm;
     // border components in the order top row, left column, right column, bottom row
     const uint64_t zr = brev64(zm);
+    const ColumnWindows win = column_windows(zm, lane);
     uint64_t remT = lane_bcast(zm, 0), remB = lane_bcast(zm, 63);
     uint64_t remL = __ballot((zm & 1ull) != 0), remR = __ballot((zm >> 63) != 0);
     uint32_t cT = 255u, cB = 255u, cL = 255u, cR = 255u, k = 0;
@@ -1964,7 +2014,7 @@ LV_D void zone_close_body(const View& v, uint32_t bid, uint32_t nblk) {
         else if (remL) s = lane == __builtin_ctzll(remL) ? 1ull : 0ull;
         else if (remR) s = lane == __builtin_ctzll(remR) ? 1ull << 63 : 0ull;
         else s = lane == 63 ? 1ull << __builtin_ctzll(remB) : 0ull;
-        const uint64_t f = flood(zm, zr, s, lane);
+        const uint64_t f = flood(win, zr, s);
         const uint64_t fT = lane_bcast(f, 0), fB = lane_bcast(f, 63);
         const uint64_t fL = __ballot((f & 1ull) != 0), fR = __ballot((f >> 63) != 0);
         if ((fT >> lane) & 1ull) cT = k;
@@ -1988,16 +2038,10 @@ LV_D void zone_close_body(const View& v, uint32_t bid, uint32_t nblk) {
     if (lane == 0) v.zcount[z] = k;
 }
 
+// Root of a node, with path halving. Every store replaces a parent by one of its ancestors, so parents stay
+// below their nodes; a store that races with a union may drop the link that union made to the node, which the
+// union then makes again between the old and the new parent (it goes on with the value it replaced).
 LV_D uint32_t g_find(uint32_t* lab, uint32_t a) {
-    while (true) {
-        const uint32_t pa = __hip_atomic_load(&lab[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (pa == a) return a;
-        a = pa;
-    }
-}
-
-// the same without concurrent unions: path halving (every store is an ancestor of the node)
-LV_D uint32_t g_find_halving(uint32_t* lab, uint32_t a) {
     while (true) {
         const uint32_t pa = __hip_atomic_load(&lab[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (pa == a) return a;
@@ -2061,10 +2105,10 @@ LV_D void zone_holes_body(const View& v, uint32_t bid, uint32_t nblk) {
     const uint32_t cT = e[lane], cB = e[64 + lane], cL = e[128 + lane], cR = e[192 + lane];
     const uint32_t k = v.zcount[z];
     const uint32_t c00 = v.zedge[0];  // component of pixel (0,0) in zone 0, 255 if it is foreground
-    const uint32_t root = c00 == 255u ? 0xFFFFFFFFu : g_find_halving(v.zpar, c00);
+    const uint32_t root = c00 == 255u ? 0xFFFFFFFFu : g_find(v.zpar, c00);
     const uint32_t base = (uint32_t)z * kZoneComps;
-    const bool o0 = (uint32_t)lane < k && g_find_halving(v.zpar, base + lane) == root;
-    const bool o1 = (uint32_t)lane + 64u < k && g_find_halving(v.zpar, base + lane + 64) == root;
+    const bool o0 = (uint32_t)lane < k && g_find(v.zpar, base + lane) == root;
+    const bool o1 = (uint32_t)lane + 64u < k && g_find(v.zpar, base + lane + 64) == root;
     const uint64_t m0 = __ballot(o0), m1 = __ballot(o1);
     auto outside = [&](uint32_t c) {
         return c < 64u ? ((m0 >> c) & 1ull) != 0 : (c < 128u && ((m1 >> (c - 64u)) & 1ull) != 0);
@@ -2073,7 +2117,7 @@ LV_D void zone_holes_body(const View& v, uint32_t bid, uint32_t nblk) {
     uint64_t s = (outside(cL) ? 1ull : 0ull) | (outside(cR) ? 1ull << 63 : 0ull);
     if (lane == 0) s |= sT;
     if (lane == 63) s |= sB;
-    const uint64_t o = flood(zm, brev64(zm), s, lane);
+    const uint64_t o = flood(column_windows(zm, lane), brev64(zm), s);
     v.hbits[(size_t)z * ZS + lane] = zm & ~o;
 }
 
@@ -2743,7 +2787,7 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
 
 // Several kernels take two or three kinds of work in one launch: the small, latency-bound kinds in the
 // first blocks, so that they run beside the kind that fills the chip instead of before or after it with a
-// launch of their own (4 to 5 us each on an idle chip, and the zones 25 us).
+// launch of their own (4 to 5 us each on an idle chip).
 #define LV_SINGLE_BID ((uint32_t)xcd_tile((int)blockIdx.x, (int)gridDim.x)), gridDim.x
 // kernels over a list that may fill only the first blocks: in dispatch order, so every XCD gets a share
 // (remapped, 700 busy blocks of 4096 would all run on two XCDs)

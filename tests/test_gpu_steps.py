@@ -186,3 +186,17 @@ def test_learning_rates_around_the_divisibility_range(algo, lr):
 def test_sample_counts(n):
     # the slot draw's reciprocal (powers of two and their neighbours), slots past 64
     run_sequence(SUBSENSE, flashing(70, 30, 3, 5), bg_samples=n, required_bg_samples=min(n, 2), lr=1.0)
+
+
+@pytest.mark.parametrize("w,h", [(5, 5), (6, 63), (63, 6), (64, 65), (65, 64), (127, 130), (129, 9), (192, 67)])
+@pytest.mark.parametrize("density", [0.05, 0.4])
+def test_zone_rows_and_floods(w, h, density):
+    """rows of 64 that end inside, at or past the image, and hole fills that cross zone edges both ways"""
+    from litiv_amd import BackgroundSubtractorSuBSENSE
+    from test_gpu_kernels import _annuli, _oracle_post
+    rng = np.random.default_rng(w * 1000 + h)
+    raw = np.where(rng.random((h, w)) < density, 255, 0).astype(np.uint8) | _annuli(rng, h, w, 6, 45)
+    sub = BackgroundSubtractorSuBSENSE()
+    sub.initialize(np.zeros((h, w, 3), np.uint8))
+    exp, n_holes = _oracle_post(raw, int(sub.scalars()["median_k"]))
+    assert np.array_equal(sub.debug_postprocess(raw), exp), "%d hole px" % n_holes
