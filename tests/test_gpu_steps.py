@@ -200,3 +200,10 @@ def test_zone_rows_and_floods(w, h, density):
     sub.initialize(np.zeros((h, w, 3), np.uint8))
     exp, n_holes = _oracle_post(raw, int(sub.scalars()["median_k"]))
     assert np.array_equal(sub.debug_postprocess(raw), exp), "%d hole px" % n_holes
+
+
+@pytest.mark.parametrize("c", [3, 1])
+@pytest.mark.parametrize("w,h", [(15, 23), (23, 15), (71, 65), (95, 79), (64, 71), (71, 64), (17, 17)])
+def test_frame_level_cells_of_ragged_sizes(w, h, c):
+    """cells of 8 to 15 pixels a side: ten columns as words or the plain loop, up to the frame's last byte"""
+    run_sequence(SUBSENSE, flashing(w, h, c, 8, seed=w + h))
