@@ -309,13 +309,13 @@ typedef struct lvbgs_binclassif {
  * Device pointers, width x height 8-bit masks sharing one row stride in bytes (0 = width); d_gt NULL
  * counts every pixel as a don't-care (metrics.cpp:26-29), d_roi NULL means no ROI. Ordered on
  * `stream` (hipStream_t or NULL); synchronizes it before returning. Allocates a small device
- * buffer per call (about 8 bytes per 1024 pixels). */
+ * buffer per call (24 bytes per 4096 pixels, at most 24 KiB). */
 int lvbgs_binclassif_accumulate(const void* d_classif, const void* d_gt, const void* d_roi, int width, int height,
                                 size_t stride, lvbgs_binclassif* counts, void* stream);
 /* The same counts without any device allocation. No counterpart in the reference: it is for callers
  * that cannot allocate (code under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc). The partial counts live in a static 512 KiB device array of the library, one copy per
- * device that uses it, held until the process ends; so a frame may hold at most
+ * hipMalloc). The partial counts live in a static 24 KiB device array of the library, one copy per
+ * device that uses it, held until the process ends. A frame may hold at most
  * LVBGS_BINCLASSIF_NOALLOC_MAX_PIXELS pixels (LVBGS_ERR_TOO_LARGE beyond, before any launch). Every
  * call on one device shares that array: calls that overlap on one device (from several host threads)
  * race and must be serialized by the caller. Arguments and results as lvbgs_binclassif_accumulate. */

@@ -207,3 +207,21 @@ def test_zone_rows_and_floods(w, h, density):
 def test_frame_level_cells_of_ragged_sizes(w, h, c):
     """cells of 8 to 15 pixels a side: ten columns as words or the plain loop, up to the frame's last byte"""
     run_sequence(SUBSENSE, flashing(w, h, c, 8, seed=w + h))
+
+
+@pytest.mark.parametrize("w,h", [(16, 1), (17, 1), (4096, 1), (4097, 1), (4096, 1024), (4096, 1025), (4099, 1027)])
+def test_score_chunks_and_words(w, h):
+    """every pair of a result and a ground-truth value in words of four, and sizes around a chunk and a grid"""
+    import torch
+    from litiv_amd import BinClassif
+    from oracle_lib import binclassif
+    i = np.arange(h * w, dtype=np.uint32)
+    res = np.where(i % 3 == 0, 255, i & 255).astype(np.uint8).reshape(h, w)
+    gt = np.where(i % 5 == 0, np.array([50, 85, 170, 255])[i // 5 % 4], i >> 8 & 255).astype(np.uint8).reshape(h, w)
+    roi = (np.random.default_rng(w + h).integers(0, 9, (h, w)) * 16).astype(np.uint8)
+    d = [torch.from_numpy(x).cuda() for x in (res, gt, roi)]
+    torch.cuda.synchronize()
+    for k in (2, 3):
+        b = BinClassif().accumulate_device(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr() if k == 3 else None, w, h)
+        got = tuple(b.counts()[n] for n in ("tp", "tn", "fp", "fn", "se", "dc"))
+        assert got == binclassif(res, gt, roi if k == 3 else None)
