@@ -98,31 +98,38 @@ LV_D uint32_t lbsp_threshold_sad(const uint32_t taps[4], uint32_t ref, uint32_t 
 }
 
 // lbsp_threshold_packed, for the frame kernels, whose taps come packed from the tile in LDS and, in the
-// sample match, stay in registers across the whole scan (a quarter of the registers; describe 694 -> 669 us
-// for a batch of 64 against the other form). One v_mqsad_u32_u8 per word: window
-// k of the quad SAD starts at byte k of S0, so it sees tap 4w+k in its byte 0; S1 holds the
-// reference in byte 0 and zeros elsewhere, and the masked SAD skips the bytes where S1 is zero, so
-// result k = |tap - ref| + ~t, which wraps past 2^32 (bit 31 clears) exactly when |tap - ref| > t
-// (both at most 255). v_alignbit shifts those bits in, tap 15 first, so bit n ends up holding tap
-// n's "|v-ref| <= t"; the result is its complement. The mask would also skip byte 0 when ref == 0:
-// that case compares the complemented taps with 255 instead (255 - v against 255 - 0 has the same
-// absolute difference).
-LV_D uint32_t lbsp_threshold_packed(const uint32_t taps[4], uint32_t ref, uint32_t t) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const uint32_t acc = ~t;
-    const u32x4 a = {acc, acc, acc, acc};
-    const uint32_t flip = ref == 0u ? 0xFFFFFFFFu : 0u;
-    const uint32_t r = ref ^ (flip & 0xFFu);
-    uint32_t d = 0;
+// sample match, stay in registers across the whole scan. Four taps at once, without per-byte instructions:
+// |v - ref| > t as v > hi = min(ref + t, 255) or v < lo = max(ref - t, 0). v > hi is the carry out of
+// v + (255 - hi), v < lo the carry out of (255 - v) + lo; the carry out of a byte is the majority of its two
+// bits 7 and of the carry into them, which is bit 7 of the sum of the low 7 bits. The two limits come from a
+// table by ref, each in all four bytes. Two words' flags (bit 7 of each byte) are gathered by one product:
+// bits 3 and 7 of byte j times 2^(29 - 7j) reach bits 32 + j and 36 + j, nothing else reaches bits 32 to 39.
+// Measured issue times: plain logic, shifts and adds 2.6 cycles, three-operand forms, v_perm and products 4.5,
+// v_mqsad_u32_u8 17. Against one of these and four v_alignbit a word (which also needed the taps flipped for a
+// reference of 0): 64 mixed streams' match 1345 -> 1245 us, phase B 678 -> 635 us, describe 675 -> 645 us.
+struct LbspLimits {
+    uint32_t above, lo;  // 255 - hi and lo, in every byte
+};
+LV_HD LbspLimits lbsp_limits(uint32_t ref, uint32_t t) {
+    const uint32_t hi = ref + t < 255u ? ref + t : 255u, lo = ref > t ? ref - t : 0u;
+    return {(255u - hi) * 0x01010101u, lo * 0x01010101u};
+}
+LV_D uint32_t lbsp_threshold_packed(const uint32_t taps[4], LbspLimits l) {
+    constexpr uint32_t kLow = 0x7F7F7F7Fu;
+    const uint32_t above_low = l.above & kLow, lo_low = (l.lo & kLow) + kLow;
+    uint32_t m[4];
 #pragma unroll
-    for (int w = 3; w >= 0; --w) {
-        const u32x4 q = __builtin_amdgcn_mqsad_u32_u8((uint64_t)(taps[w] ^ flip), r, a);
-        d = __builtin_amdgcn_alignbit(d, q[3], 31u);
-        d = __builtin_amdgcn_alignbit(d, q[2], 31u);
-        d = __builtin_amdgcn_alignbit(d, q[1], 31u);
-        d = __builtin_amdgcn_alignbit(d, q[0], 31u);
+    for (int w = 0; w < 4; ++w) {
+        const uint32_t v = taps[w], v_low = v & kLow;
+        const uint32_t over = __builtin_amdgcn_bitop3_b32(v, l.above, v_low + above_low, 0xE8);  // majority
+        m[w] = over | __builtin_amdgcn_bitop3_b32(v, l.lo, lo_low - v_low, 0x8E);  // majority with ~v
     }
-    return ~d & 0xFFFFu;
+    // flags of words 2h and 2h + 1 in bits 3 and 7 of the bytes, then as 8 bits
+    uint32_t b[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        b[h] = __umulhi(__builtin_amdgcn_bitop3_b32(0x0F0F0F0Fu, m[2 * h] >> 4, m[2 * h + 1], 0xCA) & 0x88888888u, 0x20408100u);
+    return __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0400u);
 }
 
 // ------------------------------------------------------------------------------------------

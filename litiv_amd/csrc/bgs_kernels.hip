@@ -387,10 +387,11 @@ LV_D void taps_from_global(const uint8_t* frame, int W, int x, int y, int c, uin
     }
 }
 
-// lut_lds: 4-byte aligned
-LV_D void load_lut(uint8_t* lut_lds, const Scalars* sc) {
-    static_assert(offsetof(Scalars, lut) % 4 == 0, "the LUT is read in words");
-    if (threadIdx.x < 64u) ((uint32_t*)lut_lds)[threadIdx.x] = *at((const uint32_t*)sc->lut, threadIdx.x);
+// the threshold limits of every colour (a block of 256 threads)
+LV_D void load_lut(LbspLimits* lut, const Scalars* sc) {
+    static_assert(TPB == 256, "one entry per thread");
+    const uint32_t k = threadIdx.x;
+    lut[k] = lbsp_limits(k, *at(sc->lut, k));
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -443,7 +444,7 @@ LV_D void lobster_thresholds(const View& v, PxCtx<C>& px) {
 
 // one sample test; returns true on a match and accumulates the SuBSENSE distances
 template <int C, int ALGO, int RS>
-LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col[C], const uint32_t desc[C],
+LV_D bool test_sample(const PxCtx<C>& px, const LbspLimits* lut, const uint32_t col[C], const uint32_t desc[C],
                       uint32_t& tot_desc, uint32_t& tot_sum) {
     if constexpr (ALGO == kSuBSENSE && C == 3) {
         // all colour tests first: a sample failing any of them fails whatever the descriptors say
@@ -457,7 +458,7 @@ LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const uint32_t cd = cdv[c];
-            const uint32_t inter = lbsp_threshold_packed(px.taps[c], col[c], lut[col[c]]);
+            const uint32_t inter = lbsp_threshold_packed(px.taps[c], lut[col[c]]);
             const uint32_t dd = (popc(px.intra[c] ^ desc[c]) + popc(inter ^ desc[c])) >> 1;
             uint32_t sum = (dd >> 1) * 15u + cd;
             sum = sum > 255u ? 255u : sum;
@@ -472,7 +473,7 @@ LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col
     } else if constexpr (ALGO == kSuBSENSE && C == 1) {
         const uint32_t cd = absdiff(px.cur[0], col[0]);
         if (cd > px.t_col) return false;
-        const uint32_t inter = lbsp_threshold_packed(px.taps[0], col[0], lut[col[0]]);
+        const uint32_t inter = lbsp_threshold_packed(px.taps[0], lut[col[0]]);
         const uint32_t dd = (popc(px.intra[0] ^ desc[0]) + popc(inter ^ desc[0])) >> 1;
         if (dd > px.t_desc) return false;
         uint32_t sum = (dd >> 2) * 15u + cd;
@@ -492,7 +493,7 @@ LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const uint32_t cd = cdv[c];
-            const uint32_t inter = lbsp_threshold_packed(px.taps[c], col[c], lut[col[c]]);
+            const uint32_t inter = lbsp_threshold_packed(px.taps[c], lut[col[c]]);
             const uint32_t dd = popc(inter ^ desc[c]);
             if (dd > px.t_desc) return false;
             tc += cd;
@@ -504,7 +505,7 @@ LV_D bool test_sample(const PxCtx<C>& px, const uint8_t* lut, const uint32_t col
     } else {
         const uint32_t cd = absdiff(px.cur[0], col[0]);
         if (cd > px.t_col) return false;
-        const uint32_t inter = lbsp_threshold_packed(px.taps[0], col[0], lut[col[0]]);
+        const uint32_t inter = lbsp_threshold_packed(px.taps[0], lut[col[0]]);
         tot_desc = 0;
         tot_sum = 0;
         return popc(inter ^ desc[0]) <= px.t_desc;
@@ -599,7 +600,7 @@ LV_D bool build_repl(const View& v, int x, int y, uint32_t applied, uint64_t& sb
 
 // One batch of KF loaded samples of a sequential scan (stops at the limit or at REQ matches).
 template <int C, int ALGO, int RS, int KF>
-LV_D void scan_batch(const uint8_t* lut, const PxCtx<C>& px, uint64_t sbm, int nrep, ScanState& st, uint32_t limit,
+LV_D void scan_batch(const LbspLimits* lut, const PxCtx<C>& px, uint64_t sbm, int nrep, ScanState& st, uint32_t limit,
                      uint32_t REQ, const uint64_t (&ra)[KF], const uint32_t (&rb)[KF]) {
     const ReplLds& R = repl_lds();
     const int t = (int)threadIdx.x;
@@ -642,7 +643,7 @@ constexpr uint32_t kSampleStride = 64u * (C == 3 ? 3u : 1u);
 // kMaxFetch samples) at constant offsets from a running pointer keep all KF loads in flight together
 // without address arithmetic.
 template <int C, int ALGO, int RS, int KF>
-LV_D void scan_seq(const View& v, const uint8_t* lut, const PxCtx<C>& px, int x, int y, uint64_t sbm, int nrep,
+LV_D void scan_seq(const View& v, const LbspLimits* lut, const PxCtx<C>& px, int x, int y, uint64_t sbm, int nrep,
                    ScanState& st, uint32_t limit) {
     const uint32_t p = (uint32_t)(y * v.W + x);
     const uint32_t REQ = (uint32_t)v.REQ;
@@ -743,7 +744,7 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
     const uint8_t* frame = v.frame;
     const double lr = v.lr;
     __shared__ FrameTile<C> tile;
-    __shared__ alignas(4) uint8_t lut[256];
+    __shared__ alignas(8) LbspLimits lut[256];
     const int ntx = (v.W + TW - 1) / TW;
     const int tid = (int)bid;
     const int x0 = (tid % ntx) * TW, y0 = (tid / ntx) * TH;
@@ -792,7 +793,7 @@ LV_D void describe_body(const View& v, uint32_t bid, uint32_t nblk) {
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 const uint32_t ref = (centre >> (8 * c)) & 255u;
-                intra[c] = lbsp_threshold_packed(taps[c], ref, lut[ref]);
+                intra[c] = lbsp_threshold_packed(taps[c], lut[ref]);
                 pc += popc(intra[c]);
             }
             if constexpr (C == 3) {
@@ -1013,7 +1014,7 @@ LV_D uint32_t group_writers(const View& v, int x, int y, bool active, uint32_t& 
 // Scans on from st.s to REQ matches or N samples. Every lane of the wavefront calls; the lanes of a group
 // share px, x, y, applied and st.
 template <int C, int ALGO>
-LV_D void scan_group(const View& v, const uint8_t* frame, const uint8_t* lut, const PxCtx<C>& px, int x, int y,
+LV_D void scan_group(const View& v, const uint8_t* frame, const LbspLimits* lut, const PxCtx<C>& px, int x, int y,
                      uint32_t applied, uint32_t slot, ScanState& st, bool active) {
     const uint32_t N = (uint32_t)v.N, REQ = (uint32_t)v.REQ;
     const int lane = (int)(threadIdx.x & 63u), gbase = lane & ~(kGroup - 1);
@@ -1108,7 +1109,7 @@ LV_D void group_ctx(const View& v, const uint8_t* frame, int x, int y, bool acti
 // ----------------------------------------------------------------------------------------------
 struct PredTile;
 template <int C, int ALGO, int KF>
-LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, const FrameTile<C>& tile,
+LV_D bool match_pixel(const View& v, const uint8_t* frame, const LbspLimits* lut, const FrameTile<C>& tile,
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,
                       uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px, bool& push, uint32_t& target);
 
@@ -1160,7 +1161,7 @@ struct MatchLds {
         FrameTile<1> c1;
     } tile;
     PredTile pred;
-    alignas(4) uint8_t lut[256];
+    alignas(8) LbspLimits lut[256];
 };
 
 template <int CMAX>
@@ -1183,7 +1184,7 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
     MatchLds<CMAX>& L = match_lds<CMAX>();
     FrameTile<C>& tile = tile_of<C>(L);
     PredTile& pred = L.pred;
-    uint8_t* lut = L.lut;
+    LbspLimits* lut = L.lut;
     const int ntx = (v.W + TW - 1) / TW;
     const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
     // The tile's pixels stay with their threads: the scan is cut after a few samples, so foreground pixels
@@ -1227,7 +1228,7 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
 // Phase A: sequential scan of at most v_seq_limit samples. Returns true when the pixel is final;
 // otherwise its partial state is left in mres for the cooperative phase.
 template <int C, int ALGO, int KF>
-LV_D bool match_pixel(const View& v, const uint8_t* frame, const uint8_t* lut, const FrameTile<C>& tile,
+LV_D bool match_pixel(const View& v, const uint8_t* frame, const LbspLimits* lut, const FrameTile<C>& tile,
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,
                       uint32_t seq_limit, uint32_t& examined, PxCtx<C>& px, bool& push, uint32_t& target) {
     // guess: raster-earlier writers decide as in the previous frame
@@ -1310,7 +1311,7 @@ LV_D void push_first_mixed(const View& v, bool push, uint32_t t, uint32_t stripe
 // (1 K entries), 640x480 194 / 153 (20 K), 960x720 254 / 260 (50 K), 1920x1080 408 / 423 (170 K),
 // 3840x2160 1208 / 1282 (450 K).
 template <int C, int ALGO, int KF>
-LV_D void match_seq_lanes(const View& v, const uint8_t* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
+LV_D void match_seq_lanes(const View& v, const LbspLimits* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
                           uint32_t nblk) {
     const uint8_t* frame = v.frame;
     uint32_t examined = 0;
@@ -1341,7 +1342,7 @@ LV_D void match_seq_lanes(const View& v, const uint8_t* lut, const uint32_t* s_p
 }
 
 template <int C, int ALGO>
-LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
+LV_D void match_seq_groups(const View& v, const LbspLimits* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
                            uint32_t nblk) {
     const uint8_t* frame = v.frame;
     const uint32_t lane = threadIdx.x & 63u;
@@ -1382,7 +1383,7 @@ LV_D void match_seq_groups(const View& v, const uint8_t* lut, const uint32_t* s_
 
 template <int C, int ALGO, int KF>
 LV_D void match_seq_body(const View& v, uint32_t bid, uint32_t nblk) {
-    __shared__ alignas(4) uint8_t lut[256];
+    __shared__ alignas(8) LbspLimits lut[256];
     __shared__ uint32_t s_pre[kContStripes + 1];  // exclusive prefix of the stripe counts
     stripe_prefix(v.sc->cont_cnt, s_pre);
     load_lut(lut, v.sc);
@@ -1424,7 +1425,7 @@ LV_D bool rematch_done(const View& v, uint32_t p, int x, int y, const ScanState&
 // result (a background pixel examines 2 to 5 of 50 samples, so nine in ten do): only the records and decisions
 // around it are read. A writer that turns later pushes the pixel again, and later iterations match in full.
 template <int C, int ALGO>
-LV_D void rematch(const View& v, const uint8_t* lut, GroupLds& L, const uint32_t* pre, uint32_t n, uint32_t i0,
+LV_D void rematch(const View& v, const LbspLimits* lut, GroupLds& L, const uint32_t* pre, uint32_t n, uint32_t i0,
                   uint32_t k, uint32_t* wl_next) {
     const uint8_t* frame = v.frame;
     const uint32_t lane = threadIdx.x & 63u, i = i0 + lane / kGroup;
@@ -1450,7 +1451,7 @@ LV_D void rematch(const View& v, const uint8_t* lut, GroupLds& L, const uint32_t
 
 // fix-point iterations from k0 on in one workgroup (normally no work is left)
 template <int C, int ALGO>
-LV_D void fixpoint_tail(const View& v, const uint8_t* lut, GroupLds& L, uint32_t* s_pre, uint32_t k0, uint32_t cap) {
+LV_D void fixpoint_tail(const View& v, const LbspLimits* lut, GroupLds& L, uint32_t* s_pre, uint32_t k0, uint32_t cap) {
     __shared__ uint32_t s_n;
     for (uint32_t k = k0;; ++k) {
         __syncthreads();
@@ -1488,7 +1489,7 @@ LV_D void fixpoint_tail(const View& v, const uint8_t* lut, GroupLds& L, uint32_t
 enum FixKind : int { kFixMore, kFixLast, kFixTail };
 template <int C, int ALGO, int KIND>
 LV_D void fixpoint_body(const View& v, uint32_t bid, uint32_t nblk, uint32_t k, uint32_t cap) {
-    __shared__ alignas(4) uint8_t lut[256];
+    __shared__ alignas(8) LbspLimits lut[256];
     __shared__ GroupLds L;
     __shared__ uint32_t s_pre[kContStripes + 1];
     if constexpr (KIND == kFixTail) {
@@ -2689,7 +2690,7 @@ LV_D void refresh_pending(const View& v, uint32_t bid, uint32_t nblk) {
 template <int C>
 LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
     __shared__ FrameTile<C> tile;
-    __shared__ alignas(4) uint8_t lut[256];
+    __shared__ alignas(8) LbspLimits lut[256];
     const int ntx = (v.W + TW - 1) / TW;
     const int x0 = ((int)bid % ntx) * TW, y0 = ((int)bid / ntx) * TH;
     load_frame_tile<C>(tile, img, v.W, v.H, x0, y0);
@@ -2705,7 +2706,7 @@ LV_D void init_desc_body(const View& v, const uint8_t* img, uint32_t bid) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const uint32_t ref = (centre >> (8 * c)) & 255u;
-        *at(v.last_desc, p * C + c) = (uint16_t)(in ? lbsp_threshold_packed(taps[c], ref, lut[ref]) : 0u);
+        *at(v.last_desc, p * C + c) = (uint16_t)(in ? lbsp_threshold_packed(taps[c], lut[ref]) : 0u);
         *at(v.last_color, p * C + c) = (uint8_t)(roi ? ref : 0u);
     }
 }
@@ -2763,7 +2764,7 @@ __global__ void __launch_bounds__(TPB) k_lbsp_abs(const uint8_t* __restrict__ im
     for (int c = 0; c < C; ++c) {
         const uint32_t ref = (centre >> (8 * c)) & 255u;
         uint16_t d = 0;
-        if (in) d = (uint16_t)(PACKED ? lbsp_threshold_packed(taps[c], ref, t) : lbsp_threshold_sad(taps[c], ref, t));
+        if (in) d = (uint16_t)(PACKED ? lbsp_threshold_packed(taps[c], lbsp_limits(ref, min(t, 255u))) : lbsp_threshold_sad(taps[c], ref, t));
         out[((size_t)y * W + x) * C + c] = d;
     }
 }
@@ -2825,13 +2826,15 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
 
 template <int C, int ALGO>
 __global__ void __launch_bounds__(TPB) k_describe(View v) { describe_body<C, ALGO>(v, LV_SINGLE_BID); }
-// occupancy 7 (at most 72 VGPRs) fits both fetch depths without spilling
+// 72 VGPRs at occupancy 7 fit both fetch depths without spilling
 #define LV_MATCH_WAVES(KF) __attribute__((amdgpu_waves_per_eu(7)))
 template <int C, int ALGO, int KF>
 __global__ void __launch_bounds__(TPB) LV_MATCH_WAVES(KF) k_match(View v) { match_body<C, ALGO, KF>(v, LV_SINGLE_BID); }
-// phase B holds 80 VGPRs at occupancy 6 as well
+// Phase B needs 96 VGPRs. A single stream's grid does not fill the chip at occupancy 6, and the scratch of a kernel
+// that spills costs each launch more than the waves give (occupancy 6 against 5: 320x240 14.8 and 12.2 us,
+// 3840x2160 128 and 124 us). A batch's grid does (64 mixed streams: 635 and 654 us).
 template <int C, int ALGO, int KF>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(6))) k_match_seq(View v) {
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(5))) k_match_seq(View v) {
     match_seq_body<C, ALGO, KF>(v, LV_LIST_BID);
 }
 template <int C, int ALGO, int KIND>

@@ -225,3 +225,20 @@ def test_score_chunks_and_words(w, h):
         b = BinClassif().accumulate_device(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr() if k == 3 else None, w, h)
         got = tuple(b.counts()[n] for n in ("tp", "tn", "fp", "fn", "se", "dc"))
         assert got == binclassif(res, gt, roi if k == 3 else None)
+
+
+@pytest.mark.parametrize("c", [1, 3])
+@pytest.mark.parametrize("t", [0, 1, 2, 126, 127, 128, 129, 253, 254, 255])
+def test_lbsp_limits_of_every_byte(t, c):
+    """centres and taps of every value, with differences just at, below and above the threshold"""
+    from test_gpu_kernels import _lbsp_gpu, orc
+    h, w = 40, 130
+    r = np.random.default_rng(t)
+    img = r.integers(0, 256, (h, w, c), dtype=np.uint8)
+    near = r.random((h, w, c)) < 0.7  # values at distance t - 1, t, t + 1 of a common centre, and the extremes
+    centre = int(r.integers(0, 256))
+    d = centre + r.choice([-t - 1, -t, 1 - t, 0, t - 1, t, t + 1, -256, 256], (h, w, c))
+    img[near] = np.clip(d, 0, 255).astype(np.uint8)[near]
+    ref = np.zeros((h, w, c), np.uint16)
+    orc().orc_lbsp_compute_abs(img, w, h, c, t, ref)
+    assert np.array_equal(_lbsp_gpu(img, t, packed=True), ref)
