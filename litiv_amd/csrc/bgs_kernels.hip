@@ -1815,8 +1815,8 @@ constexpr int PW = 64, PH = 16;  // post-processing tile; 256 threads x 4 pixels
 // component holding pixel (0,0).
 // Each kernel is bound by one wavefront's chain of rounds, not by memory, so a round's lane shifts are DPP moves
 // and a zone row comes in four loads. Shifts through the LDS crossbar and byte loads with a ballot per row: the
-// update launch that holds the closing at 320x240 26.9 -> 9.2 us; linking 39.9 -> 26.1 us and holes 10.1 -> 6.5 us
-// at 3840x2160; the holes of 64 mixed streams 20.6 -> 12.9 us.
+// update launch that holds the closing at 320x240 26.9 -> 9.2 us; holes 10.1 -> 6.5 us at 3840x2160, and of 64
+// mixed streams 20.6 -> 12.9 us.
 constexpr int ZS = 64;                  // zone side
 constexpr int ZPB = TPB / 64;           // zones per block, one per wavefront
 constexpr uint32_t kZoneComps = 128;    // border components per zone (at most 126 of 252 pixels)
@@ -2052,8 +2052,11 @@ LV_D uint32_t g_find(uint32_t* lab, uint32_t a) {
     }
 }
 
+// joins a < b; most pairs meet as roots, which one atomic links
 LV_D void g_union(uint32_t* lab, uint32_t a, uint32_t b) {
-    bool done = false;
+    const uint32_t first = atomicMin(&lab[b], a);
+    bool done = first == b;
+    b = first;
     while (!done) {
         a = g_find(lab, a);
         b = g_find(lab, b);
@@ -2079,20 +2082,19 @@ LV_D void zone_link(uint32_t* par, uint32_t za, uint32_t zb, uint32_t a, uint32_
     if (a != 255u && b != 255u && !dup) g_union(par, za * kZoneComps + a, zb * kZoneComps + b);
 }
 
-// unions across the right and bottom edges of every zone
+// unions across the right and bottom edges of every zone. Bound by chains of atomics across XCDs, so each edge
+// has a wavefront: against one for both edges of a zone that first looked up both roots, 3840x2160 24.7 -> 19.9 us,
+// 1920x1080 12.7 -> 10.0, 320x240 6.6 -> 5.0, 64 mixed streams 45.6 -> 27.4 us.
 LV_D void zone_link_body(const View& v, uint32_t bid, uint32_t nblk) {
     const int lane = (int)(threadIdx.x & 63u), wv = (int)(threadIdx.x >> 6);
     const int nzx = (v.W + ZS - 1) / ZS, nzy = (v.H + ZS - 1) / ZS;
-    const int z = (int)bid * ZPB + wv;
-    if (z >= nzx * nzy) return;
-    const int zx = z % nzx, zy = z / nzx;
+    const int z = ((int)bid * ZPB + wv) >> 1;
+    const bool right = (wv & 1) == 0;
+    if (z >= nzx * nzy || (right ? z % nzx + 1 == nzx : z / nzx + 1 == nzy)) return;
+    const int z2 = right ? z + 1 : z + nzx;
     const uint8_t* e = v.zedge;
-    if (zx + 1 < nzx)
-        zone_link(v.zpar, (uint32_t)z, (uint32_t)z + 1u, e[(size_t)z * 256 + 192 + lane],
-                  e[(size_t)(z + 1) * 256 + 128 + lane], lane);
-    if (zy + 1 < nzy)
-        zone_link(v.zpar, (uint32_t)z, (uint32_t)(z + nzx), e[(size_t)z * 256 + 64 + lane],
-                  e[(size_t)(z + nzx) * 256 + lane], lane);
+    zone_link(v.zpar, (uint32_t)z, (uint32_t)z2, e[(size_t)z * 256 + (right ? 192 : 64) + lane],
+              e[(size_t)z2 * 256 + (right ? 128 : 0) + lane], lane);
 }
 
 // holes of a zone: its 0-pixels minus the flood from the border pixels of outside components
@@ -2956,6 +2958,7 @@ void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]) 
     g[kGridTile] = cdiv(v.W, TW) * cdiv(v.H, TH);
     g[kGridPost] = cdiv(v.W, PW) * cdiv(v.H, PH);
     g[kGridZone] = cdiv((size_t)cdiv(v.W, ZS) * cdiv(v.H, ZS), ZPB);
+    g[kGridLink] = cdiv((size_t)2 * cdiv(v.W, ZS) * cdiv(v.H, ZS), ZPB);
     g[kGridCell] = !v.lr_scaling ? 0u : cdiv((size_t)v.dsW * v.dsH, TPB);
     g[kGridOne] = 1u;
     // single stream: a block per 1024 pixels (16 groups each; the worklists hold a few per cent of them)
@@ -2995,7 +2998,7 @@ static void frame_step_t(const View& v, const StepOptions& opt, hipStream_t st) 
     hipLaunchKernelGGL((k_update<C, ALGO>), dim3(nzone + ncell + g[kGridTile]), dim3(TPB), 0, st, v, nzone, ncell);
     if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
     if constexpr (kSub) {
-        hipLaunchKernelGGL(k_zone_link, dim3(nzone), dim3(TPB), 0, st, v);
+        hipLaunchKernelGGL(k_zone_link, dim3(g[kGridLink]), dim3(TPB), 0, st, v);
         hipLaunchKernelGGL(k_zone_holes, dim3(1 + nzone), dim3(TPB), 0, st, v, 1u);
         hipLaunchKernelGGL((k_median<true>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
         hipLaunchKernelGGL((k_dilate_final<C>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
@@ -3037,7 +3040,7 @@ void batch_step(const View* d_views, int ns, const uint32_t* const prefix[kNumGr
     hipLaunchKernelGGL(kb_update, dim3(nzone + ncell + total[kGridTile]), dim3(TPB), 0, st, args(kGridZone), nzone,
                        args(kGridCell), ncell, args(kGridTile));
     if (opt.timed_stage == 3) (void)hipEventRecord(opt.ev_end, st);
-    hipLaunchKernelGGL(kb_zone_link, dim3(nzone), dim3(TPB), 0, st, args(kGridZone));
+    hipLaunchKernelGGL(kb_zone_link, dim3(total[kGridLink]), dim3(TPB), 0, st, args(kGridLink));
     hipLaunchKernelGGL(kb_zone_holes, dim3(none + nzone), dim3(TPB), 0, st, args(kGridOne), none, args(kGridZone));
     hipLaunchKernelGGL(kb_median, dim3(total[kGridPost]), dim3(TPB), 0, st, args(kGridPost));
     hipLaunchKernelGGL(kb_dilate_final, dim3(total[kGridPost]), dim3(TPB), 0, st, args(kGridPost));
@@ -3090,7 +3093,7 @@ void launch_postprocess_probe(const View& view, uint8_t* raw, hipStream_t st) {
     uint32_t g[kNumGrids];
     kernel_grids(v, StepOptions{}, g);
     hipLaunchKernelGGL(k_zone_close, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
-    hipLaunchKernelGGL(k_zone_link, dim3(g[kGridZone]), dim3(TPB), 0, st, v);
+    hipLaunchKernelGGL(k_zone_link, dim3(g[kGridLink]), dim3(TPB), 0, st, v);
     hipLaunchKernelGGL(k_zone_holes, dim3(g[kGridZone]), dim3(TPB), 0, st, v, 0u);
     hipLaunchKernelGGL((k_median<true>), dim3(g[kGridPost]), dim3(TPB), 0, st, v);
 }

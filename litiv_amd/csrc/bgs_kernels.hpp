@@ -35,6 +35,7 @@ enum GridKind : int {
     kGridTile = 0,   // 64x4 pixel tiles (describe, match, update)
     kGridPost,       // 64x16 tiles (median, dilate)
     kGridZone,       // 64x64 hole-filling zones, four per block
+    kGridLink,       // their right and bottom edges, four per block
     kGridCell,       // 256 frame-level cells per block (0 when learning-rate scaling is off)
     kGridOne,        // one block per stream
     kGridFix,        // fix-point iteration grid
