@@ -2127,16 +2127,6 @@ LV_D void zone_holes_body(const View& v, uint32_t bid, uint32_t nblk) {
 // Post-processing masks are 0/255 bytes; the median and dilation kernels below work on four pixels
 // per 32-bit word. Words start at columns that are multiples of 4 (tile origins are), so when the
 // row pitch W is too a word is one aligned load or store; other widths assemble bytes.
-// in_image: 0xFF for each byte of the word at (gx..gx+3, gy) that lies inside the image
-LV_D uint32_t in_image_bytes(int W, int H, int gx, int gy) {
-    if (gy < 0 || gy >= H || gx + 3 < 0 || gx >= W) return 0u;
-    if (gx >= 0 && gx + 3 < W) return 0xFFFFFFFFu;
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (gx + i >= 0 && gx + i < W) m |= 0xFFu << (8 * i);
-    return m;
-}
 
 // bytes (gx..gx+3, gy) of a W x H byte image, `pad` for those outside it; gx % 4 == 0
 LV_D uint32_t load_mask_word(const uint8_t* m, int W, int H, int gx, int gy, uint32_t pad) {
@@ -2173,11 +2163,11 @@ LV_D void store_out_word(uint8_t* m, int W, int H, int gx, int gy, uint32_t w) {
     for (int i = 0; i < 4 && gx + i < W; ++i) m[(size_t)gy * (size_t)W + gx + i] = (uint8_t)(w >> (8 * i));
 }
 
-// bits (gx..gx+3, gy) of a zone bitmap (gx % 4 == 0), zero outside the image
-LV_D uint32_t zone_bits4(const uint64_t* bits, int W, int H, int gx, int gy) {
+// bits (gx..gx+31, gy) of a zone bitmap (gx % 32 == 0), zero outside the image
+LV_D uint32_t zone_bits32(const uint64_t* bits, int W, int H, int gx, int gy) {
     if (gx < 0 || gy < 0 || gx >= W || gy >= H) return 0u;
     const size_t zi = (size_t)(gy / ZS) * (size_t)((W + ZS - 1) / ZS) + (size_t)(gx / ZS);
-    return (uint32_t)(bits[zi * ZS + (size_t)(gy % ZS)] >> (gx % ZS)) & 15u;
+    return ((const uint32_t*)bits)[(zi * ZS + (size_t)(gy % ZS)) * 2 + (size_t)(gx % ZS / 32)];
 }
 // four bits -> four bytes of 0/255 (the products of the bits with 1, 2^7, 2^14, 2^21 never
 // overlap, so bit i lands alone at bit 8i)
@@ -2186,12 +2176,8 @@ LV_D uint32_t expand4(uint32_t b) { return ((b * 0x00204081u) & 0x01010101u) * 2
 // byte window of two adjacent words: bytes s..s+3 of (lo, hi)
 LV_D uint32_t bytes_at(uint32_t hi, uint32_t lo, uint32_t s) { return __builtin_amdgcn_alignbyte(hi, lo, s); }
 
-// AND (OR) of the word whose bytes start 4 bytes into a, b, c and its shifts by up to 3 bytes either
-// way: the 7-wide erosion (dilation) of the 0/255 bytes of b along the row
-LV_D uint32_t erode7_word(uint32_t a, uint32_t b, uint32_t c) {
-    return b & bytes_at(b, a, 1) & bytes_at(b, a, 2) & bytes_at(b, a, 3) & bytes_at(c, b, 1) & bytes_at(c, b, 2) &
-           bytes_at(c, b, 3);
-}
+// OR of the word whose bytes start 4 bytes into a, b, c and its shifts by up to 3 bytes either way: the 7-wide
+// dilation of the 0/255 bytes of b along the row
 LV_D uint32_t dilate7_word(uint32_t a, uint32_t b, uint32_t c) {
     return b | bytes_at(b, a, 1) | bytes_at(b, a, 2) | bytes_at(b, a, 3) | bytes_at(c, b, 1) | bytes_at(c, b, 2) |
            bytes_at(c, b, 3);
@@ -2200,17 +2186,22 @@ LV_D uint32_t dilate7_word(uint32_t a, uint32_t b, uint32_t c) {
 // mask = raw | holes | erode7(PreFlood); last_fg = medianBlur(mask, k) (SUB:544-547; LOB:578 uses
 // the raw mask directly). Binary median with zero padding = majority count over the k x k window.
 // Counts are kept one per byte (at most 13 per column and 169 per window, so no byte carries into
-// the next) and the majority test adds 128 - need to every byte and keeps bit 7.
+// the next) and the majority test adds 128 - need to every byte and keeps bit 7. Holes and erosion stay bits (32
+// columns a word) until the counts, as the zones have them. Bound by its LDS passes: with bytes throughout, one row
+// of column counts an item and counts over 13 columns whatever k is, 3840x2160 29.2 -> 20.0 us, 1920x1080 9.3 -> 6.4,
+// 64 mixed streams 156 -> 106 us.
 template <bool SUBSENSE>
 LV_D void median_body(const View& v, uint32_t bid, uint32_t nblk) {
     constexpr int HM = 6, HE = 3;           // median halo (k <= 13), erosion halo
     constexpr int MWW = (PW + 16) / 4;      // mask words: columns x0-8 .. x0+PW+7
     constexpr int MH = PH + 2 * HM;         // mask rows: y0-6 .. y0+PH+5
-    constexpr int EWW = (PW + 24) / 4;      // PreFlood words: columns x0-12 .. x0+PW+11
     constexpr int EH = MH + 2 * HE;         // PreFlood rows: y0-9 .. y0+PH+8
+    constexpr int BW = PW / 32 + 2;         // words of a row's bits: columns x0-32 .. x0+PW+31
     constexpr int OWW = PW / 4;             // output words per row
-    __shared__ uint32_t s_pre[EH][EWW];
-    __shared__ uint32_t s_eh[EH][MWW];
+    static_assert(EH * BW <= TPB, "an item per thread");
+    __shared__ uint32_t s_pre[EH][BW];
+    __shared__ uint32_t s_eh[EH][BW];
+    __shared__ uint32_t s_bits[MH][BW];
     __shared__ uint32_t s_mask[MH][MWW];
     __shared__ uint32_t s_col[PH][MWW];
     const int W = v.W, H = v.H;
@@ -2219,42 +2210,48 @@ LV_D void median_body(const View& v, uint32_t bid, uint32_t nblk) {
     const int x0 = (tid % ntx) * PW, y0 = (tid / ntx) * PH;
     const int k = v.median_k, r = k / 2, need = (k * k + 1) / 2;
     if constexpr (SUBSENSE) {
-        // erosion treats the outside of the image as 255
-        for (int i = threadIdx.x; i < EH * EWW; i += TPB) {
-            const int ly = i / EWW, wx = i % EWW;
-            // PreFlood = 255 except at its 0-pixels, 255 outside the image
-            s_pre[ly][wx] = expand4(~zone_bits4(v.zbits, W, H, x0 - 12 + 4 * wx, y0 - HM - HE + ly) & 15u);
+        const int ly = (int)threadIdx.x / BW, j = (int)threadIdx.x % BW, gx = x0 + 32 * (j - 1);
+        // PreFlood is set except at its 0-pixels, and set outside the image
+        if (ly < EH) s_pre[ly][j] = ~zone_bits32(v.zbits, W, H, gx, y0 - HM - HE + ly);
+        __syncthreads();
+        // horizontal 7-erosion (the outer three columns of a row's bits are not used)
+        if (ly < EH) {
+            const uint32_t w = s_pre[ly][j], l = s_pre[ly][max(j - 1, 0)], r = s_pre[ly][min(j + 1, BW - 1)];
+            uint32_t e = w;
+#pragma unroll
+            for (uint32_t a = 1; a <= (uint32_t)HE; ++a)
+                e &= __builtin_amdgcn_alignbit(w, l, 32u - a) & __builtin_amdgcn_alignbit(r, w, a);
+            s_eh[ly][j] = e;
         }
         __syncthreads();
-        // horizontal 7-erosion; mask word j (columns x0-8+4j..) is PreFlood word j+1
-        for (int i = threadIdx.x; i < EH * MWW; i += TPB) {
-            const int ly = i / MWW, j = i % MWW;
-            s_eh[ly][j] = erode7_word(s_pre[ly][j], s_pre[ly][j + 1], s_pre[ly][j + 2]);
-        }
-        __syncthreads();
-    }
-    // the mask as 0/1 bytes, zero outside the image; mask row ly is PreFlood row ly+3
-    for (int i = threadIdx.x; i < MH * MWW; i += TPB) {
-        const int ly = i / MWW, j = i % MWW, gx = x0 - 8 + 4 * j, gy = y0 - HM + ly;
-        uint32_t m;
-        if constexpr (SUBSENSE) {
+        // holes | erosion inside the image; mask row ly is PreFlood row ly+3
+        if (ly < MH) {
+            const int gy = y0 - HM + ly, left = W - gx;
             uint32_t e = s_eh[ly][j];
 #pragma unroll
             for (int a = 1; a <= 2 * HE; ++a) e &= s_eh[ly + a][j];
-            m = (load_mask_word(v.last_raw, W, H, gx, gy, 0u) | expand4(zone_bits4(v.hbits, W, H, gx, gy)) | e) &
-                in_image_bytes(W, H, gx, gy);
-        } else {
-            m = load_mask_word(v.last_raw, W, H, gx, gy, 0u);
+            const bool in = gx >= 0 && left > 0 && gy >= 0 && gy < H;
+            const uint32_t image = !in ? 0u : left >= 32 ? ~0u : (1u << left) - 1u;
+            s_bits[ly][j] = (zone_bits32(v.hbits, W, H, gx, gy) | e) & image;
         }
+        __syncthreads();
+    }
+    // the mask as 0/1 bytes, zero outside the image
+    for (int i = threadIdx.x; i < MH * MWW; i += TPB) {
+        const int ly = i / MWW, j = i % MWW, b = 24 + 4 * j;
+        uint32_t m = load_mask_word(v.last_raw, W, H, x0 - 8 + 4 * j, y0 - HM + ly, 0u);
+        if constexpr (SUBSENSE) m |= expand4(s_bits[ly][b >> 5] >> (b & 31) & 15u);
         s_mask[ly][j] = m & 0x01010101u;
     }
     __syncthreads();
-    // column counts over k rows
-    for (int i = threadIdx.x; i < PH * MWW; i += TPB) {
-        const int ly = i / MWW, j = i % MWW;
+    // column counts over k rows, two rows an item: the second drops a row and takes in the next
+    static_assert(PH % 2 == 0 && PH / 2 * MWW <= TPB, "an item per thread");
+    if (threadIdx.x < PH / 2 * MWW) {
+        const int ly = (int)threadIdx.x / MWW * 2, j = (int)threadIdx.x % MWW, a0 = HM + ly - r;
         uint32_t c = 0;
-        for (int a = HM + ly - r; a <= HM + ly + r; ++a) c += s_mask[a][j];
+        for (int a = a0; a <= a0 + 2 * r; ++a) c += s_mask[a][j];
         s_col[ly][j] = c;
+        s_col[ly + 1][j] = c - s_mask[a0][j] + s_mask[a0 + 2 * r + 1][j];
     }
     __syncthreads();
     // row counts over k columns: output word q (columns x0+4q..) starts at byte 4q+8 of the counts
@@ -2264,13 +2261,11 @@ LV_D void median_body(const View& v, uint32_t bid, uint32_t nblk) {
         uint32_t w[5];
 #pragma unroll
         for (int u = 0; u < 5; ++u) w[u] = s_col[ly][q + u];
-        uint32_t s = 0;
+        auto from = [&](int b) { return b & 3 ? bytes_at(w[(b >> 2) + 1], w[b >> 2], (uint32_t)(b & 3)) : w[b >> 2]; };
+        uint32_t s = w[2];
 #pragma unroll
-        for (int o = -HM; o <= HM; ++o) {
-            const int b = 8 + o, wi = b >> 2, sh = b & 3;
-            const uint32_t t = sh ? bytes_at(w[wi + 1], w[wi], (uint32_t)sh) : w[wi];
-            s += (o >= -r && o <= r) ? t : 0u;
-        }
+        for (int o = 1; o <= HM; ++o)
+            if (o <= r) s += from(8 - o) + from(8 + o);  // uniform
         const uint32_t bits = ((s + bias) >> 7) & 0x01010101u;
         store_mask_word(v.last_fg, W, H, x0 + 4 * q, y0 + ly, bits * 255u);
         if constexpr (!SUBSENSE)

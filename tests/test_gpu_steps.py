@@ -242,3 +242,19 @@ def test_lbsp_limits_of_every_byte(t, c):
     ref = np.zeros((h, w, c), np.uint16)
     orc().orc_lbsp_compute_abs(img, w, h, c, t, ref)
     assert np.array_equal(_lbsp_gpu(img, t, packed=True), ref)
+
+
+@pytest.mark.parametrize("k", [1, 3, 11, 13])
+@pytest.mark.parametrize("w,h", [(64, 16), (65, 17), (127, 33), (200, 47)])
+def test_median_windows_and_mask_bits(w, h, k):
+    """the smallest and largest windows at tile edges, and erosions whose words end inside or past the image"""
+    from litiv_amd import BackgroundSubtractorSuBSENSE
+    from test_gpu_kernels import _oracle_post
+    rng = np.random.default_rng(w + k)
+    coarse = np.kron(rng.random((h // 9 + 1, w // 11 + 1)) < 0.55, np.ones((9, 11), bool))[:h, :w]
+    raw = np.where(coarse ^ (rng.random((h, w)) < 0.04), 255, 0).astype(np.uint8)
+    sub = BackgroundSubtractorSuBSENSE(median_blur_kernel=k)
+    sub.initialize(np.zeros((h, w, 3), np.uint8))
+    assert int(sub.scalars()["median_k"]) == k
+    exp, n_holes = _oracle_post(raw, k)
+    assert np.array_equal(sub.debug_postprocess(raw), exp), "%d hole px" % n_holes
