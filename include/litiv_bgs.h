@@ -125,9 +125,9 @@ typedef struct lvbgs_stats {
     uint32_t max_fixpoint_iter;
     uint32_t width, height, channels, n_roi;
     uint64_t examined_speculative; /* samples examined by the speculative match kernel alone */
-    uint32_t fixpoint_work[8];     /* [0]: pixels finished by the cooperative match phase;
+    uint32_t fixpoint_work[8];     /* [0]: pixels finished by the match continuation (phase B);
                                       [k]: worklist size of fix-point iteration k (1..7) */
-    uint64_t examined_cooperative; /* samples examined by the cooperative match phase */
+    uint64_t examined_cooperative; /* samples examined by the match continuation */
 } lvbgs_stats;
 int lvbgs_get_stats(lvbgs_ctx* ctx, lvbgs_stats* out);
 
@@ -188,7 +188,7 @@ void* lvbgs_batch_stream(lvbgs_batch* b);
 typedef struct lvbgs_batch_options {
     int use_graph;          /* capture the step once as a hipGraph and replay it */
     int seq_limit;          /* samples scanned by the sequential match phase (1..255) */
-    int cont_blocks;        /* cooperative match phase: grid of a stream, at most */
+    int cont_blocks;        /* match continuation: grid of a stream, at most */
     int cont_px_per_block;  /*   ... and ceil(pixels / this) when > 0 */
     int fixpoint_launches;  /* full-grid fix-point iterations before the one-workgroup tail */
     int fixpoint_blocks;    /* fix-point grid of a stream, at most */

@@ -6,18 +6,20 @@
 // step below reproduces that order exactly without a sequential sweep:
 //   describe : per pixel, everything that does not depend on other pixels' decisions
 //              (LBSP, thresholds, RNG draws, diffusion target/slot/gates)       -> rec, desc_cur
-//   match    : speculative ordered sample scan; samples diffused in by raster-earlier
-//              neighbours are applied under a guess of their decision (previous raw mask)
+//   match    : speculative ordered scan of the first samples (phase A); samples diffused in by
+//              raster-earlier neighbours are applied under a guess of their decision (previous raw
+//              mask)
+//   match_seq: the scans that phase A cut (phase B), one lane per pixel or, for short lists, 16
 //   fixpoint : pixels whose writers' decisions differ from the guess are re-matched, and the
-//              change propagates through a de-duplicated worklist until nothing changes. The
-//              writer graph is acyclic (raster order), so the fix point is unique and equals the
-//              sequential result.
-//   feedback : FP32 maps (D_last, D_min, raw segm, T, v, R), raw mask, blink bookkeeping
-//   update   : each pixel gathers, in raster order, the writes aimed at its samples from the 5x5
-//              window (self-update included); the last writer of a slot wins. No atomics.
-//   post     : close 3x3, hole fill (union-find CCL of the background), erode 7x7, binary
-//              median k x k, dilate 7x7, blink masks, final-segmentation averages
-//   control  : frame-level downsampled analysis, LBSP LUT adaptation, model reset, caps
+//              change propagates through worklists until nothing changes. The writer graph is
+//              acyclic (raster order), so the fix point is unique and equals the sequential result.
+//   update   : FP32 maps (D_last, D_min, raw segm, T, v, R), raw mask, blink bookkeeping; each pixel
+//              gathers, in raster order, the writes aimed at its samples from the 5x5 window
+//              (self-update included); the last writer of a slot wins. No atomics. The launch also
+//              holds the 3x3 closing with the zones' border components and the down-sampled cells.
+//   post     : hole fill (union-find over the zones), erode 7x7, binary median k x k, dilate 7x7,
+//              blink masks, final-segmentation averages, pending model reset
+//   control  : LBSP LUT adaptation, model reset, caps (beside the zones' holes)
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -1226,7 +1228,7 @@ LV_D void match_body(const View& v, uint32_t bid, uint32_t nblk) {
 }
 
 // Phase A: sequential scan of at most v_seq_limit samples. Returns true when the pixel is final;
-// otherwise its partial state is left in mres for the cooperative phase.
+// otherwise its partial state is left in mres for phase B.
 template <int C, int ALGO, int KF>
 LV_D bool match_pixel(const View& v, const uint8_t* frame, const LbspLimits* lut, const FrameTile<C>& tile,
                       const PredTile& pred, const PxIn<C>& in, int lx, int ly, int x, int y, uint32_t p,

@@ -25,7 +25,7 @@ struct StepOptions {
     int fetch_depth = 4;         // sample loads in flight per lane in the sequential phase (2 or 4)
     int cont_blocks = 0;         // grid of phase B (grid-stride over unfinished pixels; 0: by frame size)
     int fix_px_per_block = 0;    // > 0: fix-point grid of a stream = ceil(npx / this), at most fixpoint_blocks
-    int cont_px_per_block = 0;   // > 0: cooperative grid of a stream = ceil(npx / this), at most cont_blocks
+    int cont_px_per_block = 0;   // > 0: phase B grid of a stream = ceil(npx / this), at most cont_blocks
     int timed_stage = 0;         // 0: none, 1: the match kernel (phase A), 2: the whole step, 3: the update kernel
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
 };
@@ -39,7 +39,7 @@ enum GridKind : int {
     kGridCell,       // 256 frame-level cells per block (0 when learning-rate scaling is off)
     kGridOne,        // one block per stream
     kGridFix,        // fix-point iteration grid
-    kGridCont,       // cooperative match grid
+    kGridCont,       // phase B grid
     kNumGrids
 };
 void kernel_grids(const View& v, const StepOptions& opt, uint32_t g[kNumGrids]);
