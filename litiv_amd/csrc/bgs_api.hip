@@ -487,9 +487,9 @@ static int check_lr(lvbgs_ctx* c, double lr) {
 }
 
 // Samples scanned per pixel before phase B takes over in the single-stream path: one batch of four
-// loads. Measured per frame on MI355X at 4 / 8 / 12 / 255 samples: 320x240 RGB 127 / 129 / 131 / 157 us,
-// 1280x720 286 / 288 / 291 / 357, 3840x2160 grey 998 / 1002 / 1006 / 1025, LOBSTER 640x512 grey 79 / 80 /
-// 82 / 88, 3840x2160 RGB 779 / 780 / 787 / 817.
+// loads. Measured per frame on MI355X at 4 / 8 / 12 / 255 samples: 320x240 RGB 82 / 82 / 84 / 108 us,
+// 1280x720 188 / 190 / 194 / 208, 3840x2160 grey 723 / 724 / 727 / 743, LOBSTER 640x512 grey 55 / 56 / 57 / 64,
+// 3840x2160 RGB 914 / 916 / 923 / 943.
 constexpr uint32_t kSeqLimit = 4;
 
 static int step(lvbgs_ctx* c, const uint8_t* d_img, uint8_t* d_mask, double lr) {

@@ -2981,9 +2981,11 @@ static void frame_step_t(const View& v, const StepOptions& opt, hipStream_t st) 
     // phase B finishes the scans phase A cut; it exits at once when there are none
     if (opt.fetch_depth == 4) hipLaunchKernelGGL((k_match_seq<C, ALGO, 4>), dim3(g[kGridCont]), dim3(TPB), 0, st, v);
     else hipLaunchKernelGGL((k_match_seq<C, ALGO, 2>), dim3(g[kGridCont]), dim3(TPB), 0, st, v);
-    // the second iteration's worklist is about a hundredth of the first's: on small frames (a dozen entries)
-    // the tail takes it (320x240 126.8 -> 124.8 us; 1920x1080 408 -> 420)
-    const uint32_t launches = opt.fixpoint_launches >= 0 ? (uint32_t)opt.fixpoint_launches : v.npx < 600000u ? 1u : 2u;
+    // the second iteration's worklist is about a hundredth of the first's to a tenth: on small frames the tail, one
+    // workgroup, takes it. Step with one / two launches, us: 320x240 81.2 / 82.1, 480x360 85.1 / 86.0, 640x480
+    // 97.1 / 97.1, 800x600 116.2 / 116.7; but 960x540 grey 159.9 / 124.8, 880x660 232 / 165, 1280x720 305 / 190
+    // with more change in the frame, so the line lies where one launch still gains.
+    const uint32_t launches = opt.fixpoint_launches >= 0 ? (uint32_t)opt.fixpoint_launches : v.npx < 200000u ? 1u : 2u;
     const uint32_t cap = (uint32_t)opt.tail_cap;
     for (uint32_t k = 1; k < launches; ++k)
         hipLaunchKernelGGL((k_fixpoint<C, ALGO, kFixMore>), dim3(g[kGridFix]), dim3(TPB), 0, st, v, k, cap);

@@ -11,7 +11,8 @@ namespace lvbgs {
 constexpr int kMaxFetch = 4;
 constexpr int kCtxWords = 20;  // words of a cached match context
 // entries of a continuation list up to which phase B of the match gives each a lane group; the streams of
-// a batch share it
+// a batch share it. Step with lanes / by this rule / with groups, us: 320x240 111 / 82 / 83, LOBSTER 640x512 grey
+// 65 / 56 / 56, 1280x720 195 / 193 / 211, 3840x2160 902 / 901 / 985
 constexpr uint32_t kGroupLimit = 32768;
 
 struct StepOptions {
