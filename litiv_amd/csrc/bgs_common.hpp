@@ -71,6 +71,29 @@ LV_HD bool divides31(uint32_t d, uint32_t m) {
     return __builtin_fmaf(-rintf(rem * r), mf, rem) == 0.0f;
 }
 
+// Word loads from byte buffers: the 32-bit word at byte `off` of a buffer of `total` bytes (4 at least) is read from
+// byte `at`, with all four bytes inside the buffer, and then gives the bytes from the beyond-th on; nothing for
+// beyond < 0 (left of the buffer) or > 3 (past it). I holds every offset of the buffer's rows.
+template <typename I>
+struct WordPlace {
+    I at, beyond;
+};
+template <typename I>
+LV_HD WordPlace<I> word_place(I off, I total) {
+    const I at = off < 0 ? 0 : off > total - 4 ? total - 4 : off;
+    return {at, off - at};
+}
+
+// How the tiles of a stand-alone LBSP image are read. Below 5 pixels a side no pixel has a whole patch, and an
+// image may be smaller than a word: nothing is read. A tile reaches at most 66 columns past the last row's end, so
+// 32-bit offsets serve images that stay 256 bytes below 2^31; larger ones take 64-bit offsets. (The frame kernels
+// need no rule: a frame with an ROI has 5 pixels a side, and at most 2^28 pixels.)
+enum LbspForm : int { kLbspEmpty, kLbsp32, kLbsp64 };
+LV_HD LbspForm lbsp_form(int W, int H, int C) {
+    if (W < 5 || H < 5) return kLbspEmpty;
+    return (uint64_t)W * (uint64_t)H * (uint64_t)C <= 0x7FFFFFFFull - 256u ? kLbsp32 : kLbsp64;
+}
+
 // ------------------------------------------------------------------------------------------
 // LBSP 16-bit double cross (LBSP.hpp:275-298): bit n compares the centre with (x+DX[n], y+DY[n]).
 // ------------------------------------------------------------------------------------------

@@ -310,23 +310,23 @@ struct FrameTile<1> {
 
 // a 32-bit word at any byte offset of a buffer of `total` bytes (4 at least), zeros outside it; the last bytes
 // of a buffer come from its last whole word
-LV_D uint32_t word_at(const uint8_t* base, int off, int total) {
-    const int o = off < 0 ? 0 : off > total - 4 ? total - 4 : off;
-    const uint32_t w = peek<UnalignedU32>(base, (uint32_t)o);
-    const int beyond = off - o;  // < 0: left of the buffer, > 0: bytes to drop
-    return beyond < 0 || beyond > 3 ? 0u : w >> (8 * beyond);
+template <typename I>
+LV_D uint32_t word_at(const uint8_t* base, I off, I total) {
+    const WordPlace<I> p = word_place(off, total);
+    const uint32_t w = sizeof(I) == 4 ? peek<UnalignedU32>(base, (uint32_t)p.at) : peek<UnalignedU32>(base + p.at, 0u);
+    return p.beyond < 0 || p.beyond > 3 ? 0u : w >> (8 * (int)p.beyond);
 }
 
 // Pixels left and right of the image come out as whatever lies beside them in the frame: no pixel of the ROI
-// reaches them.
-template <int C>
+// reaches them. I: the type of byte offsets.
+template <int C, typename I = int>
 LV_D void load_frame_tile(FrameTile<C>& t, const uint8_t* frame, int W, int H, int x0, int y0) {
     using T = FrameTile<C>;
-    const int total = W * H * C;
+    const I total = (I)W * H * C;
     if constexpr (C == 3) {
         auto put = [&](int r, int c) {
             const int gy = y0 + r - 2;
-            t.px[r][c] = gy >= 0 && gy < H ? word_at(frame, (gy * W + x0 + c - 2) * 3, total) & 0xFFFFFFu : 0u;
+            t.px[r][c] = gy >= 0 && gy < H ? word_at(frame, ((I)gy * W + x0 + c - 2) * 3, total) & 0xFFFFFFu : 0u;
         };
         const int lx = (int)threadIdx.x % TW, ly = (int)threadIdx.x / TW;
 #pragma unroll
@@ -335,7 +335,7 @@ LV_D void load_frame_tile(FrameTile<C>& t, const uint8_t* frame, int W, int H, i
     } else {
         const int r = (int)threadIdx.x / T::WORDS, l = (int)threadIdx.x % T::WORDS, gy = y0 + r - 2;
         if (r < T::LH) {
-            const uint32_t w = gy >= 0 && gy < H ? word_at(frame, gy * W + x0 - 4 + 4 * l, total) : 0u;
+            const uint32_t w = gy >= 0 && gy < H ? word_at(frame, (I)gy * W + x0 - 4 + 4 * l, total) : 0u;
             *(uint32_t*)&t.px[r][4 * l] = w;
         }
     }
@@ -2742,18 +2742,23 @@ LV_D void background_body(const View& v, void* out, uint32_t bid) {
     }
 }
 
-// stand-alone LBSP map (LBSP::compute2, LBSP.cpp:102-123): absolute threshold t
-// LBSP with an absolute threshold over a whole image, through either form of the threshold test
-template <int C, bool PACKED>
+// stand-alone LBSP map (LBSP::compute2, LBSP.cpp:102-123) with the absolute threshold t, through either form of
+// the threshold test
+template <int C, bool PACKED, int FORM>
 __global__ void __launch_bounds__(TPB) k_lbsp_abs(const uint8_t* __restrict__ img, int W, int H, uint32_t t,
                                                 uint16_t* __restrict__ out) {
     __shared__ FrameTile<C> tile;
     const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH;
     const int tid = xcd_tile((int)blockIdx.x, ntx * nty);
     const int x0 = (tid % ntx) * TW, y0 = (tid / ntx) * TH;
-    load_frame_tile<C>(tile, img, W, H, x0, y0);
-    __syncthreads();
     const int lx = threadIdx.x % TW, ly = threadIdx.x / TW, x = x0 + lx, y = y0 + ly;
+    if constexpr (FORM == kLbspEmpty) {
+        if (x < W && y < H)
+            for (int c = 0; c < C; ++c) out[((size_t)y * W + x) * C + c] = 0;
+        return;
+    }
+    load_frame_tile<C, std::conditional_t<FORM == kLbsp64, int64_t, int>>(tile, img, W, H, x0, y0);
+    __syncthreads();
     if (x >= W || y >= H) return;
     const bool in = x >= 2 && y >= 2 && x < W - 2 && y < H - 2;
     uint32_t taps[C][4];
@@ -3074,15 +3079,18 @@ void launch_background_desc(const View& v, uint16_t* out_desc, hipStream_t st) {
     else hipLaunchKernelGGL((k_background<1, true>), dim3(b), dim3(TPB), 0, st, v, (void*)out_desc);
 }
 
-void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st) {
-    const unsigned tiles = cdiv(W, TW) * cdiv(H, TH);
-    if (packed) {
-        if (C == 3) hipLaunchKernelGGL((k_lbsp_abs<3, true>), dim3(tiles), dim3(TPB), 0, st, img, W, H, t, out);
-        else hipLaunchKernelGGL((k_lbsp_abs<1, true>), dim3(tiles), dim3(TPB), 0, st, img, W, H, t, out);
-    } else {
-        if (C == 3) hipLaunchKernelGGL((k_lbsp_abs<3, false>), dim3(tiles), dim3(TPB), 0, st, img, W, H, t, out);
-        else hipLaunchKernelGGL((k_lbsp_abs<1, false>), dim3(tiles), dim3(TPB), 0, st, img, W, H, t, out);
+template <int C, bool PACKED>
+static void lbsp_abs_t(const uint8_t* img, int W, int H, uint32_t t, uint16_t* out, hipStream_t st) {
+    const dim3 g(cdiv(W, TW) * cdiv(H, TH)), b(TPB);
+    switch (lbsp_form(W, H, C)) {
+    case kLbspEmpty: hipLaunchKernelGGL((k_lbsp_abs<C, PACKED, kLbspEmpty>), g, b, 0, st, img, W, H, t, out); break;
+    case kLbsp32: hipLaunchKernelGGL((k_lbsp_abs<C, PACKED, kLbsp32>), g, b, 0, st, img, W, H, t, out); break;
+    case kLbsp64: hipLaunchKernelGGL((k_lbsp_abs<C, PACKED, kLbsp64>), g, b, 0, st, img, W, H, t, out); break;
     }
+}
+void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st) {
+    if (C == 3) (packed ? lbsp_abs_t<3, true> : lbsp_abs_t<3, false>)(img, W, H, t, out, st);
+    else (packed ? lbsp_abs_t<1, true> : lbsp_abs_t<1, false>)(img, W, H, t, out, st);
 }
 
 // the SuBSENSE hole-filling and median kernels alone, on a raw mask
