@@ -158,9 +158,9 @@ int lvbgs_set_fixpoint_schedule(lvbgs_ctx* ctx, int launches, int blocks);
  * depend on it. */
 int lvbgs_set_match_schedule(lvbgs_ctx* ctx, int seq_limit, int cont_blocks);
 
-/* LBSP self-check: lvbgs_lbsp_compute_abs through the form of the threshold test the frame kernels
- * use (taps packed four per register, masked quad SADs) instead of the per-tap form; the two must give
- * the same bits. */
+/* LBSP self-check: lvbgs_lbsp_compute_abs through the form of the threshold test the frame kernels use (taps
+ * packed four per register, compared with the threshold's two limits as byte carries) instead of the per-tap
+ * form; the two must give the same bits. RGB images take the packed form from either entry point. */
 int lvbgs_debug_lbsp_packed(const void* d_img, int width, int height, int channels, int threshold, void* d_out,
                             void* stream);
 

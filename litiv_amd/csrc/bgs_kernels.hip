@@ -3089,7 +3089,9 @@ static void lbsp_abs_t(const uint8_t* img, int W, int H, uint32_t t, uint16_t* o
     }
 }
 void launch_lbsp_abs(const uint8_t* img, int W, int H, int C, uint32_t t, uint16_t* out, bool packed, hipStream_t st) {
-    if (C == 3) (packed ? lbsp_abs_t<3, true> : lbsp_abs_t<3, false>)(img, W, H, t, out, st);
+    // RGB tiles give their taps packed, so the per-tap form would take them apart again. A call, per-tap / packed,
+    // us: RGB 1920x1080 29.2 / 27.9, 3840x2160 72.6 / 67.5; grey 1920x1080 18.7 / 20.3
+    if (C == 3) lbsp_abs_t<3, true>(img, W, H, t, out, st);
     else (packed ? lbsp_abs_t<1, true> : lbsp_abs_t<1, false>)(img, W, H, t, out, st);
 }
 
