@@ -150,12 +150,13 @@ void* lvbgs_stream(lvbgs_ctx* ctx);
 int lvbgs_set_timing(lvbgs_ctx* ctx, const char* stage);
 int lvbgs_take_timing(lvbgs_ctx* ctx, double* total_ms, int* count);
 
-/* Fix-point schedule: full-grid iterations before the single-workgroup tail, and their grid size. */
+/* Fix-point schedule: full-grid iterations before the single-workgroup tail (0..64) and their grid size
+ * (1..65535). -1 launches and 0 blocks, the defaults, choose them by the frame size. Results do not depend on it. */
 int lvbgs_set_fixpoint_schedule(lvbgs_ctx* ctx, int launches, int blocks);
 
 /* Match schedule: samples scanned per pixel by the sequential phase (1..255; 0, the default: 4)
- * before unfinished pixels move to the continuation, and the grid of the continuation. Results do not
- * depend on it. */
+ * before unfinished pixels move to the continuation, and the grid of the continuation (1..65535; 0, the
+ * default: by the frame size). Results do not depend on it. */
 int lvbgs_set_match_schedule(lvbgs_ctx* ctx, int seq_limit, int cont_blocks);
 
 /* LBSP self-check: lvbgs_lbsp_compute_abs through the form of the threshold test the frame kernels use (taps

@@ -435,11 +435,13 @@ class BackgroundSubtractor:
         return ms.value, n.value
 
     def set_fixpoint_schedule(self, launches, blocks):
+        """Full-grid fix-point iterations (0..64; -1 = by the frame size) and their grid (1..65535; 0 = by the
+        frame size); results do not depend on it."""
         self._check(lib().lvbgs_set_fixpoint_schedule(self._h, int(launches), int(blocks)))
 
-    def set_match_schedule(self, seq_limit, cont_blocks=1024):
+    def set_match_schedule(self, seq_limit, cont_blocks=0):
         """Samples scanned per pixel by the sequential match phase (1..255; 0 = automatic: 4) and the
-        continuation grid; results do not depend on it."""
+        continuation grid (1..65535; 0 = by the frame size); results do not depend on it."""
         self._check(lib().lvbgs_set_match_schedule(self._h, int(seq_limit), int(cont_blocks)))
 
     def debug_rng(self, frame, phase, event, n):

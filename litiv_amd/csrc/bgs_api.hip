@@ -906,14 +906,14 @@ extern "C" int lvbgs_take_timing(lvbgs_ctx* c, double* total_ms, int* count) {
 }
 
 extern "C" int lvbgs_set_fixpoint_schedule(lvbgs_ctx* c, int launches, int blocks) {
-    if (!c || launches < 0 || launches > 64 || blocks < 1 || blocks > 65535) return LVBGS_ERR_ARG;
+    if (!c || launches < -1 || launches > 64 || blocks < 0 || blocks > 65535) return LVBGS_ERR_ARG;
     c->opt.fixpoint_launches = launches;
     c->opt.fixpoint_blocks = blocks;
     return LVBGS_OK;
 }
 
 extern "C" int lvbgs_set_match_schedule(lvbgs_ctx* c, int seq_limit, int cont_blocks) {
-    if (!c || seq_limit < 0 || seq_limit > 255 || cont_blocks < 1 || cont_blocks > 65535) return LVBGS_ERR_ARG;
+    if (!c || seq_limit < 0 || seq_limit > 255 || cont_blocks < 0 || cont_blocks > 65535) return LVBGS_ERR_ARG;
     c->opt.seq_limit = seq_limit;
     c->opt.cont_blocks = cont_blocks;
     return LVBGS_OK;

@@ -258,3 +258,35 @@ def test_median_windows_and_mask_bits(w, h, k):
     assert int(sub.scalars()["median_k"]) == k
     exp, n_holes = _oracle_post(raw, k)
     assert np.array_equal(sub.debug_postprocess(raw), exp), "%d hole px" % n_holes
+
+
+def test_schedules_return_to_automatic():
+    """after any override the calls that name the automatic values leave a context as it was created"""
+    import inspect
+
+    from litiv_amd import BackgroundSubtractorSuBSENSE
+    from litiv_amd.bgs import LvbgsError
+    from test_gpu_parity import SUB_STATE
+    assert inspect.signature(BackgroundSubtractorSuBSENSE.set_match_schedule).parameters["cont_blocks"].default == 0
+    frames = flashing(150, 90, 3, 8)
+    a, b = BackgroundSubtractorSuBSENSE(), BackgroundSubtractorSuBSENSE()
+    for m in (a, b):
+        m.initialize(frames[0])
+    a.set_match_schedule(7, 3)
+    a.set_fixpoint_schedule(0, 1)
+    for t, f in enumerate(frames):
+        if t == 4:
+            a.set_match_schedule(0)
+            a.set_fixpoint_schedule(-1, 0)
+        assert np.array_equal(a.apply(f), b.apply(f)), t
+        if t >= 4:  # what phase A examined and handed on follows from its limit
+            sa, sb = a.stats(), b.stats()
+            assert (sa["examined_speculative"], sa["fixpoint_work"][0]) == (sb["examined_speculative"], sb["fixpoint_work"][0])
+    for name in SUB_STATE:
+        assert np.array_equal(a.state(name), b.state(name)), name
+    for bad in ((-1, 1), (256, 1), (1, -1), (1, 65536)):
+        with pytest.raises(LvbgsError):
+            a.set_match_schedule(*bad)
+    for bad in ((-2, 1), (65, 1), (1, -1), (1, 65536)):
+        with pytest.raises(LvbgsError):
+            a.set_fixpoint_schedule(*bad)
