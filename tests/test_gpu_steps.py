@@ -290,3 +290,38 @@ def test_schedules_return_to_automatic():
     for bad in ((-2, 1), (65, 1), (1, -1), (1, 65536)):
         with pytest.raises(LvbgsError):
             a.set_fixpoint_schedule(*bad)
+
+
+def _distinct_slots(rec, raw):
+    """per pixel, how many sample slots its raster-earlier neighbours overwrite if those that were background in
+    the mask `raw` write: the record's target is the pixel and its forward gate is open"""
+    h, w = rec.shape
+    gate = ((rec >> 5) & 1 | (rec >> 6) & (rec >> 7) & 1).astype(bool) & (raw == 0)
+    slots = np.full((12, h, w), -1, np.int64)
+    for i in range(12):
+        dx, dy = i % 5 - 2, i // 5 - 2  # the writer stands at (x + dx, y + dy)
+        hit = np.where(gate & ((rec & 31) == (2 - dy) * 5 + 2 - dx), rec >> 24, -1)
+        slots[i, 2:, 2:-2] = hit[2 + dy:h + dy, 2 + dx:w - 2 + dx]
+    slots.sort(axis=0)
+    return (slots[0] >= 0).astype(int) + ((slots[1:] != slots[:-1]) & (slots[1:] >= 0)).sum(axis=0)
+
+
+@pytest.mark.parametrize("limit", [4, 255])
+def test_pixels_past_the_entries_of_a_thread_occur(limit):
+    # five or more overwritten slots: such pixels keep their guess and list themselves. They must occur in the
+    # frames, and the masks must be the oracle's
+    from test_gpu_parity import _pair
+    frames = flashing(484, 325, 3, 5)
+    gpu, orc = _pair(SUBSENSE)
+    gpu.set_match_schedule(limit)
+    gpu.initialize(frames[0])
+    orc.initialize(frames[0])
+    unmatched = 0
+    for f in frames:
+        raw = gpu.state("last_raw")
+        assert np.array_equal(gpu.apply(f, learningRate=1.0), orc.apply(f, 1.0))
+        n = _distinct_slots(gpu.state("rec"), raw)
+        past = (n > 4) & (gpu.state("roi") != 0)
+        unmatched += int(past.sum())
+        assert (gpu.state("mres")[past] >> 24).all()  # the fix point matched them
+    assert unmatched >= 5, unmatched
