@@ -325,3 +325,44 @@ def test_pixels_past_the_entries_of_a_thread_occur(limit):
         unmatched += int(past.sum())
         assert (gpu.state("mres")[past] >> 24).all()  # the fix point matched them
     assert unmatched >= 5, unmatched
+
+
+def test_iteration_cap_is_reported_by_synchronize():
+    """the steps' error bits reach lvbgs_synchronize and lvbgs_batch_synchronize through the context's pinned word,
+    stay until the next initialize, and stay with the context that they belong to"""
+    import torch
+
+    from litiv_amd import BackgroundSubtractorSuBSENSE, Batch, Server
+    from litiv_amd.bgs import ERR_DEVICE, LvbgsError
+    frames = flashing(96, 72, 3, 8)
+    d = [torch.from_numpy(f).cuda() for f in frames]
+    mask = torch.empty((72, 96), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    srv = Server(hbm_budget=1 << 30, fixpoint_launches=0)
+    srv.debug_fixpoint_cap(0)
+    sid = srv.open(d[0].data_ptr(), 96, 72, 3)
+    member = srv.member(sid)
+    member.synchronize()
+    failed = False
+    for t in range(8):
+        srv.submit(sid, d[t].data_ptr(), mask.data_ptr(), tag=t)
+        srv.drain()
+        failed = any(int(s) == ERR_DEVICE for _, _, s in srv.poll())
+        if failed:
+            break
+    assert failed, "no frame needed the fix point"
+    # the server has closed the stream; its context waits in the server's pool
+    other = BackgroundSubtractorSuBSENSE()
+    other.initialize(frames[0])
+    other.apply(frames[1])
+    batch = Batch([other, member])
+    for call in (member.synchronize, batch.synchronize, member.synchronize):
+        with pytest.raises(LvbgsError) as e:
+            call()
+        assert e.value.code == ERR_DEVICE
+    other.synchronize()
+    member.initialize(frames[0])
+    member.synchronize()
+    batch.synchronize()
+    batch.close()
+    srv.close_server()
