@@ -317,9 +317,10 @@ int lvbgs_binclassif_accumulate(const void* d_classif, const void* d_gt, const v
  * that cannot allocate (code under HIP graph capture, serving loops and harnesses that forbid
  * hipMalloc). The partial counts live in a static 24 KiB device array of the library, one copy per
  * device that uses it, held until the process ends. A frame may hold at most
- * LVBGS_BINCLASSIF_NOALLOC_MAX_PIXELS pixels (LVBGS_ERR_TOO_LARGE beyond, before any launch). Every
- * call on one device shares that array: calls that overlap on one device (from several host threads)
- * race and must be serialized by the caller. Arguments and results as lvbgs_binclassif_accumulate. */
+ * LVBGS_BINCLASSIF_NOALLOC_MAX_PIXELS pixels (LVBGS_ERR_TOO_LARGE beyond, before any launch): a limit of
+ * the interface, kept for its callers; the array would serve any size. Every call on one device shares
+ * that array: calls that overlap on one device (from several host threads) race and must be serialized
+ * by the caller. Arguments and results as lvbgs_binclassif_accumulate. */
 #define LVBGS_BINCLASSIF_NOALLOC_MAX_PIXELS 67100672ull
 int lvbgs_binclassif_accumulate_noalloc(const void* d_classif, const void* d_gt, const void* d_roi, int width,
                                         int height, size_t stride, lvbgs_binclassif* counts, void* stream);

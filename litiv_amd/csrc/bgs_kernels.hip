@@ -213,14 +213,6 @@ LV_D void encode_raw(const uint32_t col[C], const uint32_t desc[C], uint64_t& ra
 }
 
 template <int C>
-LV_D void load_sample(const View& v, uint32_t s, uint32_t p, uint32_t col[C], uint32_t desc[C]) {
-    uint64_t ra;
-    uint32_t rb;
-    fetch_raw<C>(v, s, p, ra, rb);
-    decode_raw<C>(ra, rb, col, desc);
-}
-
-template <int C>
 LV_D void store_raw(const View& v, uint32_t s, uint32_t p, uint64_t ra, uint32_t rb) {
     const size_t idx = sample_index(v, s, p);
     // non-temporal: scattered single-record writes gain nothing from being kept in L2
@@ -1306,12 +1298,10 @@ LV_D void push_first_mixed(const View& v, bool push, uint32_t t, uint32_t stripe
 
 // Phase B continues the scans phase A cut, over the dense list of unfinished pixels (its stripes walked in
 // order), with the context phase A cached (rebuilt from global memory past a stripe's cache).
-// Two forms, chosen by the length of the list: a group per pixel up to View::group_limit entries,
-// which is what the chip holds at once (256 CUs x 24 wavefronts x 4 groups = 24 K, taken as 32 K): there a lane
-// per pixel leaves most of it idle behind chains of 13 dependent loads. Past it a lane per pixel does the
-// same work with fewer instructions. Measured per frame, lanes / groups: 320x240 RGB 160 / 127 us
-// (1 K entries), 640x480 194 / 153 (20 K), 960x720 254 / 260 (50 K), 1920x1080 408 / 423 (170 K),
-// 3840x2160 1208 / 1282 (450 K).
+// Two forms, chosen by the length of the list: a group per pixel up to View::group_limit entries, where a
+// lane per pixel leaves most of the chip idle behind chains of 13 dependent loads (it holds 20 K groups at once at
+// this kernel's occupancy of 5: 256 CUs x 20 wavefronts x 4). Past it a lane per pixel does the same work with fewer
+// instructions. Both sides are measured at kGroupLimit.
 template <int C, int ALGO, int KF>
 LV_D void match_seq_lanes(const View& v, const LbspLimits* lut, const uint32_t* s_pre, uint32_t n, uint32_t bid,
                           uint32_t nblk) {
@@ -2300,8 +2290,8 @@ struct DilateTile {
     uint32_t fg[LH][FWW], h[LH][OWW];
 };
 
-// one allocation for the two kinds of block of the dilation launch, whichever channel counts it instantiates
-// (separate arrays took 16.6 KB and the dilation of a batch 220 us instead of 189)
+// one allocation for the two kinds of work of the dilation launch, whichever channel counts it instantiates
+// (a sum instead of a union takes as long: the dilation of 64 mixed streams 200 us either way)
 union SweepLds {
     RefreshTile refresh;
     DilateTile dilate;
@@ -2831,9 +2821,9 @@ LV_D void for_batch_block(const BatchArgs& b, F&& f) {
 template <int C, int ALGO>
 __global__ void __launch_bounds__(TPB) k_describe(View v) { describe_body<C, ALGO>(v, LV_SINGLE_BID); }
 // 72 VGPRs at occupancy 7 fit both fetch depths without spilling
-#define LV_MATCH_WAVES(KF) __attribute__((amdgpu_waves_per_eu(7)))
+#define LV_MATCH_WAVES __attribute__((amdgpu_waves_per_eu(7)))
 template <int C, int ALGO, int KF>
-__global__ void __launch_bounds__(TPB) LV_MATCH_WAVES(KF) k_match(View v) { match_body<C, ALGO, KF>(v, LV_SINGLE_BID); }
+__global__ void __launch_bounds__(TPB) LV_MATCH_WAVES k_match(View v) { match_body<C, ALGO, KF>(v, LV_SINGLE_BID); }
 // Phase B needs 96 VGPRs. A single stream's grid does not fill the chip at occupancy 6, and the scratch of a kernel
 // that spills costs each launch more than the waves give (occupancy 6 against 5: 320x240 14.8 and 12.2 us,
 // 3840x2160 128 and 124 us). A batch's grid does (64 mixed streams: 635 and 654 us).
@@ -2898,7 +2888,7 @@ __global__ void __launch_bounds__(TPB) k_background(View v, void* out) { backgro
     })
 __global__ void __launch_bounds__(TPB) kb_describe(BatchArgs b) { LV_BATCH_C(describe_body, kSuBSENSE); }
 template <int KF>
-__global__ void __launch_bounds__(TPB) LV_MATCH_WAVES(KF) kb_match(BatchArgs b) {
+__global__ void __launch_bounds__(TPB) LV_MATCH_WAVES kb_match(BatchArgs b) {
     LV_BATCH_C(match_body, kSuBSENSE, KF, 3);
 }
 template <int KF>
@@ -2912,6 +2902,8 @@ __global__ void __launch_bounds__(TPB) kb_fixpoint(BatchArgs b, uint32_t k, uint
         else fixpoint_body<1, kSuBSENSE, KIND>(v, bid, nblk, k, cap);
     });
 }
+// The general path of the cells (ten column weights in doubles) for two channel counts makes this kernel spill 11
+// VGPRs, 48 bytes of scratch a lane; without the cells it takes 72 VGPRs and none.
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(7))) kb_update(BatchArgs zone, uint32_t nzone, BatchArgs cell, uint32_t ncell,
                                                  BatchArgs tile) {
     const uint32_t b = blockIdx.x;

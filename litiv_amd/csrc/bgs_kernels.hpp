@@ -11,8 +11,9 @@ namespace lvbgs {
 constexpr int kMaxFetch = 4;
 constexpr int kCtxWords = 20;  // words of a cached match context
 // entries of a continuation list up to which phase B of the match gives each a lane group; the streams of
-// a batch share it. Step with lanes / by this rule / with groups, us: 320x240 111 / 82 / 83, LOBSTER 640x512 grey
-// 65 / 56 / 56, 1280x720 195 / 193 / 211, 3840x2160 902 / 901 / 985
+// a batch share it. Step with lanes / with groups, us: 320x240 (7 K entries) 115 / 90, 640x480 (9 K) 137 / 103,
+// LOBSTER 640x512 grey (20 K) 66 / 59; past the line 960x720 (109 K) 182 / 184, 1120x840 (130 K) 217 / 228,
+// 1920x1080 (168 K) 331 / 356, 3840x2160 (460 K) 991 / 1073
 constexpr uint32_t kGroupLimit = 32768;
 
 struct StepOptions {
