@@ -72,16 +72,10 @@ LV_HD bool divides31(uint32_t d, uint32_t m) {
 }
 
 // Word loads from byte buffers: the 32-bit word at byte `off` of a buffer of `total` bytes (4 at least) is read from
-// byte `at`, with all four bytes inside the buffer, and then gives the bytes from the beyond-th on; nothing for
-// beyond < 0 (left of the buffer) or > 3 (past it). I holds every offset of the buffer's rows.
+// the returned byte, with all four bytes inside the buffer. I holds every offset of the buffer's rows.
 template <typename I>
-struct WordPlace {
-    I at, beyond;
-};
-template <typename I>
-LV_HD WordPlace<I> word_place(I off, I total) {
-    const I at = off < 0 ? 0 : off > total - 4 ? total - 4 : off;
-    return {at, off - at};
+LV_HD I word_place(I off, I total) {
+    return off < 0 ? 0 : off > total - 4 ? total - 4 : off;
 }
 
 // How the tiles of a stand-alone LBSP image are read. Below 5 pixels a side no pixel has a whole patch, and an

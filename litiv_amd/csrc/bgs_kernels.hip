@@ -304,9 +304,10 @@ struct FrameTile<1> {
 // of a buffer come from its last whole word
 template <typename I>
 LV_D uint32_t word_at(const uint8_t* base, I off, I total) {
-    const WordPlace<I> p = word_place(off, total);
-    const uint32_t w = sizeof(I) == 4 ? peek<UnalignedU32>(base, (uint32_t)p.at) : peek<UnalignedU32>(base + p.at, 0u);
-    return p.beyond < 0 || p.beyond > 3 ? 0u : w >> (8 * (int)p.beyond);
+    const I o = word_place(off, total);
+    const uint32_t w = sizeof(I) == 4 ? peek<UnalignedU32>(base, (uint32_t)o) : peek<UnalignedU32>(base + o, 0u);
+    const I beyond = off - o;  // < 0: left of the buffer, > 0: bytes to drop
+    return beyond < 0 || beyond > 3 ? 0u : w >> (8 * (int)beyond);
 }
 
 // Pixels left and right of the image come out as whatever lies beside them in the frame: no pixel of the ROI

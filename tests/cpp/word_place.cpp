@@ -23,11 +23,11 @@ static long reads = 0;
 template <typename I>
 static void read_word(const std::vector<unsigned char>& buf, I off) {
     const I total = (I)buf.size();
-    const WordPlace<I> p = word_place(off, total);
-    CHECK(p.at >= 0 && p.at + 4 <= total, "total %ld off %ld reads from %ld", (long)total, (long)off, (long)p.at);
+    const I at = word_place(off, total), beyond = off - at;
+    CHECK(at >= 0 && at + 4 <= total, "total %ld off %ld reads from %ld", (long)total, (long)off, (long)at);
     uint32_t w = 0, want = 0;
-    for (int k = 0; k < 4; ++k) w |= (uint32_t)buf[(size_t)(p.at + k)] << (8 * k);
-    w = p.beyond < 0 || p.beyond > 3 ? 0u : w >> (8 * (int)p.beyond);
+    for (int k = 0; k < 4; ++k) w |= (uint32_t)buf[(size_t)(at + k)] << (8 * k);
+    w = beyond < 0 || beyond > 3 ? 0u : w >> (8 * (int)beyond);
     for (int k = 0; k < 4; ++k)
         if (off >= 0 && off + k < total) want |= (uint32_t)buf[(size_t)(off + k)] << (8 * k);
     CHECK(w == want, "total %ld off %ld: %08x, not %08x", (long)total, (long)off, w, want);
@@ -63,8 +63,8 @@ int main() {
         CHECK(form == kLbsp64 || far <= 0x7FFFFFFFll, "%dx%dx%d", s[0], s[1], s[2]);
         CHECK(form == kLbsp32 || total > 0x7FFFFFFFll - 256, "%dx%dx%d", s[0], s[1], s[2]);
         for (int64_t d = -300; d <= 300; ++d) {
-            const WordPlace<int64_t> p = word_place<int64_t>(total + d, total);
-            CHECK(p.at >= 0 && p.at + 4 <= total, "%dx%dx%d", s[0], s[1], s[2]);
+            const int64_t at = word_place<int64_t>(total + d, total);
+            CHECK(at >= 0 && at + 4 <= total, "%dx%dx%d", s[0], s[1], s[2]);
         }
     }
     std::printf("ok %ld\n", reads);
